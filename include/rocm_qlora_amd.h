@@ -181,6 +181,25 @@ int rq_nf4_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                   void* y, int64_t ldy, void* workspace, int64_t workspace_bytes,
                   hipStream_t stream);
 
+/* rq_nf4_linear with optional scratch memory (256-byte aligned device memory,
+ * contents ignored, free again once the call's kernels are done).  A 16-bit
+ * call given the bytes it needs decodes the weight into it once and multiplies
+ * by the dense MFMA GEMM (same operand roundings, another order of fp32 sums);
+ * any other call is rq_nf4_linear.  rq_nf4_linear_scratch_size reports those
+ * bytes where that is the faster route (many rows, and the calls that
+ * otherwise run on the generic kernels), 0 elsewhere. */
+int rq_nf4_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int64_t rank,
+                               int64_t* bytes);
+int rq_nf4_linear_scratch(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
+                          const uint8_t* w_packed, int64_t N, int64_t block_size,
+                          const void* absmax, int absmax_dtype,
+                          const uint8_t* c2, int c2_format, int64_t block2,
+                          const void* bias, int bias_dtype,
+                          const void* lora_x, int64_t ld_lora_x, const void* lora_a, const void* lora_b,
+                          int64_t ld_lora_b, int lora_dtype, int64_t rank, float scaling,
+                          void* y, int64_t ldy, void* workspace, int64_t workspace_bytes,
+                          void* scratch, int64_t scratch_bytes, hipStream_t stream);
+
 /* Bytes of the device scratch array behind rq_nf4_linear_noalloc (per GPU,
  * held until the process ends). */
 #define RQ_NOALLOC_SCRATCH_BYTES (32u << 20)
@@ -252,6 +271,19 @@ int rq_nf4_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t
                      float mask_scale, void* dx, int64_t lddx,
                      void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
+/* rq_nf4_linear_dx with optional scratch memory, as rq_nf4_linear_scratch. */
+int rq_nf4_linear_dx_scratch_size(int dy_dtype, int64_t M, int64_t N, int64_t K, int64_t block_size, int64_t rank,
+                                  int64_t* bytes);
+int rq_nf4_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy,
+                             const uint8_t* w_packed, int64_t K, int64_t block_size,
+                             const void* absmax, int absmax_dtype,
+                             const uint8_t* c2, int c2_format, int64_t block2,
+                             const void* lora_a, const void* lora_b, int64_t ld_lora_b, int lora_dtype,
+                             int64_t rank, float scaling, const uint8_t* lora_mask, int64_t ld_lora_mask,
+                             float mask_scale, void* dx, int64_t lddx,
+                             void* workspace, int64_t workspace_bytes, void* scratch, int64_t scratch_bytes,
+                             hipStream_t stream);
+
 /* ------------------------------------------------------------------------
  * INT8 and FP8 linears
  * ------------------------------------------------------------------------ */
@@ -284,6 +316,18 @@ int rq_int8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx
 int rq_int8_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy, const int8_t* q,
                       int64_t K, int64_t block_size, const void* scales, int scales_dtype, void* dx,
                       int64_t lddx, hipStream_t stream);
+
+/* rq_int8_linear and rq_int8_linear_dx with optional scratch memory, as
+ * rq_nf4_linear_scratch (dx: 0 the forward, 1 dX). */
+int rq_int8_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int dx,
+                                int64_t* bytes);
+int rq_int8_linear_scratch(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* q,
+                           int64_t N, int64_t block_size, const void* scales, int scales_dtype, const void* bias,
+                           int bias_dtype, void* y, int64_t ldy, void* scratch, int64_t scratch_bytes,
+                           hipStream_t stream);
+int rq_int8_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy, const int8_t* q,
+                              int64_t K, int64_t block_size, const void* scales, int scales_dtype, void* dx,
+                              int64_t lddx, void* scratch, int64_t scratch_bytes, hipStream_t stream);
 
 /* Bytes of workspace rq_fp8_quantize needs. */
 int rq_fp8_quantize_workspace_size(int64_t* bytes);

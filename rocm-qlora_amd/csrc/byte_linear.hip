@@ -16,6 +16,7 @@
 #include "rq_gemm_core.h"
 #include "rq_gemm8.h"
 #include "rq_fp8.h"
+#include "rq_dense.h"
 #include "rq_generic.h"
 
 namespace rq {
@@ -338,10 +339,16 @@ static int run_byte(const ByteLinearArgs& A, hipStream_t stream) {
   }
 }
 
-static int byte_linear(const ByteLinearArgs& A, hipStream_t stream) {
+static int byte_linear(const ByteLinearArgs& A, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
   int st = validate_byte(A);
   if (st != RQ_OK) return st;
   if (A.M == 0) return RQ_OK;
+  if (scratch && scratch_bytes > 0) {
+    const size_t need = dense_scratch_bytes(A.x_dtype, A.M, A.N, A.K, 0);
+    const GenericInt8 g = generic_args(A);
+    if (need > 0 && size_t(scratch_bytes) >= need && dense_int8_ok(g, false))
+      return run_dense_int8(g, false, scratch, size_t(scratch_bytes), stream);
+  }
   if (!byte_fast_ok(A)) return run_generic_int8_linear(generic_args(A), stream);
   if (A.x_dtype == RQ_DTYPE_BF16) return run_byte<RQ_DTYPE_BF16>(A, stream);
   return run_byte<RQ_DTYPE_F16>(A, stream);
@@ -373,20 +380,42 @@ int fp8_quantize(int dt, const void* t, int64_t rows, int64_t cols, int64_t ld, 
 // ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
-extern "C" int rq_int8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* q,
-                              int64_t N, int64_t block_size, const void* scales, int scales_dtype, const void* bias,
-                              int bias_dtype, void* y, int64_t ldy, hipStream_t stream) {
+extern "C" int rq_int8_linear_scratch(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* q,
+                                      int64_t N, int64_t block_size, const void* scales, int scales_dtype,
+                                      const void* bias, int bias_dtype, void* y, int64_t ldy, void* scratch,
+                                      int64_t scratch_bytes, hipStream_t stream) {
   rq::ByteLinearArgs A{};
   A.x = x; A.x_dtype = x_dtype; A.M = M; A.K = K; A.ldx = ldx;
   A.w = reinterpret_cast<const uint8_t*>(q); A.N = N;
   A.block_size = block_size; A.scales = scales; A.scales_dtype = scales_dtype;
   A.bias = bias; A.bias_dtype = bias_dtype; A.y = y; A.ldy = ldy;
-  return rq::byte_linear(A, stream);
+  return rq::byte_linear(A, scratch, scratch_bytes, stream);
 }
 
-extern "C" int rq_int8_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy, const int8_t* q,
-                                 int64_t K, int64_t block_size, const void* scales, int scales_dtype, void* dx,
-                                 int64_t lddx, hipStream_t stream) {
+extern "C" int rq_int8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* q,
+                              int64_t N, int64_t block_size, const void* scales, int scales_dtype, const void* bias,
+                              int bias_dtype, void* y, int64_t ldy, hipStream_t stream) {
+  return rq_int8_linear_scratch(x, x_dtype, M, K, ldx, q, N, block_size, scales, scales_dtype, bias, bias_dtype, y,
+                                ldy, nullptr, 0, stream);
+}
+
+extern "C" int rq_int8_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int dx,
+                                           int64_t* bytes) {
+  if (!bytes) return RQ_ERR_NULL_POINTER;
+  if (!rq::valid_float_dtype(x_dtype)) return RQ_ERR_BAD_DTYPE;
+  if (M < 0 || N < 1 || K < 1 || block_size < 0) return RQ_ERR_BAD_SHAPE;
+  const bool fast = !dx && K % 64 == 0 &&
+                    (block_size == 0 ||
+                     (block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0));
+  const int64_t C = dx ? K : N, R = dx ? N : K;
+  *bytes = fast && !rq::dense_beats_fused(M, C, R, false) ? 0 : int64_t(rq::dense_scratch_bytes(x_dtype, M, C, R, 0));
+  return RQ_OK;
+}
+
+extern "C" int rq_int8_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy,
+                                         const int8_t* q, int64_t K, int64_t block_size, const void* scales,
+                                         int scales_dtype, void* dx, int64_t lddx, void* scratch,
+                                         int64_t scratch_bytes, hipStream_t stream) {
   if (!dy || !q || !scales || !dx) return RQ_ERR_NULL_POINTER;
   if (!rq::valid_float_dtype(dy_dtype) || !rq::valid_float_dtype(scales_dtype)) return RQ_ERR_BAD_DTYPE;
   if (M < 0 || N <= 0 || K <= 0 || block_size < 0 || lddy < N || lddx < K) return RQ_ERR_BAD_SHAPE;
@@ -397,7 +426,19 @@ extern "C" int rq_int8_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_
   g.x = dy; g.x_dtype = dy_dtype; g.M = M; g.K = K; g.N = N; g.ldx = lddy;
   g.q = q; g.block_size = block_size; g.scales = scales; g.scales_dtype = scales_dtype;
   g.y = dx; g.ldy = lddx;
+  if (scratch && scratch_bytes > 0) {
+    const size_t need = rq::dense_scratch_bytes(dy_dtype, M, K, N, 0);
+    if (need > 0 && size_t(scratch_bytes) >= need && rq::dense_int8_ok(g, true))
+      return rq::run_dense_int8(g, true, scratch, size_t(scratch_bytes), stream);
+  }
   return rq::run_generic_int8_dx(g, stream);
+}
+
+extern "C" int rq_int8_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy, const int8_t* q,
+                                 int64_t K, int64_t block_size, const void* scales, int scales_dtype, void* dx,
+                                 int64_t lddx, hipStream_t stream) {
+  return rq_int8_linear_dx_scratch(dy, dy_dtype, M, N, lddy, q, K, block_size, scales, scales_dtype, dx, lddx, nullptr,
+                                   0, stream);
 }
 
 extern "C" int rq_fp8_quantize_workspace_size(int64_t* bytes) {

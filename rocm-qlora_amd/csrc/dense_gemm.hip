@@ -1,0 +1,561 @@
+// Linears over a weight decoded once per call, for many activation rows: one
+// launch writes RND(W_deq) in the activation dtype into scratch memory -- as
+// W rows [N][R] for the forward, as W^T rows [K][R] for dX, the reduction
+// length padded with zeros to a multiple of 64 -- and the dense MFMA GEMM
+// (rq_dense_gemm.h) multiplies by it.  The decoded weight is the reference's
+// own intermediate, dequantize_int4 / dequantize_int8 (...).to(x.dtype)
+// (quant_ops.py:55-78, :128-150, quant_linear.py:189-195), so only the order
+// of fp32 sums can differ from the fused kernels.
+//
+// Decoding costs one pass of N K / 2 (NF4) bytes in and 2 N K out, whatever
+// the row count; the fused GEMM decodes every weight tile again for each 256
+// activation rows, in the same issue slots and LDS as its MFMAs.
+#include "rq_dense_gemm.h"
+#include "rq_dense.h"
+#include "rq_launch.h"
+
+#include <algorithm>
+
+namespace rq {
+namespace {
+
+// ---------------------------------------------------------------------------
+// Weight sources: the codes as stored.  load(f, n): raw words of n codes at
+// flat index f; value(raw, i, lut): code i's fp32 value before its scale.
+// ---------------------------------------------------------------------------
+struct SrcNF4 {
+  static constexpr int kBytesPer8 = 4;  // bytes of 8 codes
+  const uint8_t* p;
+  __device__ __forceinline__ float at(int64_t f, const float* lut) const {
+    const uint32_t b = p[f >> 1];
+    return lut[(f & 1) ? b >> 4 : b & 15u];
+  }
+  // the values of the 8 codes in `w` (low word) in k order
+  __device__ static __forceinline__ void expand8(u32x2 w, const float* lut, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = lut[(w.x >> (4 * i)) & 15u];
+  }
+  __device__ static __forceinline__ u32x2 piece(const u32x4 (&r)[1], int i) { return u32x2{r[0][i], 0u}; }
+};
+struct SrcInt8 {
+  static constexpr int kBytesPer8 = 8;
+  const uint8_t* p;
+  __device__ __forceinline__ float at(int64_t f, const float*) const { return float(int8_t(p[f])); }
+  __device__ static __forceinline__ void expand8(u32x2 w, const float*, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = float(int8_t(uint8_t((i < 4 ? w.x : w.y) >> (8 * (i & 3)))));
+  }
+  __device__ static __forceinline__ u32x2 piece(const u32x4 (&r)[2], int i) {
+    return u32x2{r[i >> 1][2 * (i & 1)], r[i >> 1][2 * (i & 1) + 1]};
+  }
+};
+
+// The scale of flat element f of row n: blockwise over the flat weight
+// (log2 >= 0: power-of-two block), or one per row (bs 0).
+struct BlockOf {
+  int64_t bs;
+  int log2;
+  __device__ __forceinline__ int64_t operator()(int64_t f, int64_t n) const {
+    return bs == 0 ? n : (log2 >= 0 ? f >> log2 : f / bs);
+  }
+};
+
+constexpr int kDecThreads = 256;
+
+// W rows, K % 64 == 0 and blocks of at least 8 inside a row: the output is
+// the flat weight.  A lane takes 8 codes (one 16-byte store, consecutive
+// lanes consecutive bytes), four such per thread, all loads first.  HBM and
+// MALL writes bound it (measured at 4096 x 14336: see launch_decode).
+template <int XT, class Src, class Scale>
+__global__ __launch_bounds__(kDecThreads) void decode_rows_kernel(Src src, Scale scale, BlockOf blk, uint32_t n_chunks,
+                                                                  uint32_t row_chunks, u32x4* __restrict__ out) {
+  __shared__ float lut[16];
+  if (threadIdx.x < 16) lut[threadIdx.x] = u2f(kNF4Bits[threadIdx.x]);
+  __syncthreads();
+  const uint32_t c0 = blockIdx.x * (4 * kDecThreads) + threadIdx.x;
+  u32x2 w[4];
+  float s[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    uint32_t c = c0 + kDecThreads * j;
+    c = c < n_chunks ? c : n_chunks - 1;
+    if constexpr (Src::kBytesPer8 == 4)
+      w[j] = u32x2{__builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(src.p) + c), 0u};
+    else
+      w[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(src.p) + c);
+    s[j] = scale(blk(int64_t(c) * 8, c / row_chunks));
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t c = c0 + kDecThreads * j;
+    if (c >= n_chunks) break;
+    float v[8];
+    Src::expand8(w[j], lut, v);
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = cvt_pk<XT>(__fmul_rn(v[2 * k], s[j]), __fmul_rn(v[2 * k + 1], s[j]));
+    out[c] = u32x4{o[0], o[1], o[2], o[3]};
+  }
+}
+
+// W^T rows, N % 64 == 0, K % 64 == 0, blocks of at least 32 inside a row: a
+// workgroup takes 64 weight rows x 256 columns, a thread rows 2p, 2p + 1 (p
+// = thread % 32) and columns 32 (thread / 32) .. + 31.  It stores the pairs
+// {n, n + 1} as one word at [k][2p] of an LDS tile (32 lanes fill one 128-byte
+// row), which leaves as 128-byte runs of the output's rows.
+template <int XT, class Src, class Scale>
+__global__ __launch_bounds__(kDecThreads) void decode_cols_kernel(Src src, Scale scale, BlockOf blk, int64_t K,
+                                                                  int64_t ldo, uint16_t* __restrict__ out) {
+  __shared__ float lut[16];
+  __shared__ __attribute__((aligned(16))) uint8_t tile[256 * 128];
+  const int t = threadIdx.x, p = t & 31;
+  if (t < 16) lut[t] = u2f(kNF4Bits[t]);
+  __syncthreads();
+  const int64_t n0 = int64_t(blockIdx.y) * 64, k0 = int64_t(blockIdx.x) * 256, kc = k0 + 32 * (t >> 5);
+  constexpr int kPieces = Src::kBytesPer8 / 4;  // 16-byte loads of 32 codes
+  if (kc < K) {  // K is a multiple of 32: the thread's columns are all live
+    u32x4 w[2][kPieces];
+    float s[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int64_t f = (n0 + 2 * p + i) * K + kc;
+      const u32x4* src4 = reinterpret_cast<const u32x4*>(src.p + (f >> 3) * Src::kBytesPer8);
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j) w[i][j] = src4[j];
+      s[i] = scale(blk(f, n0 + 2 * p + i));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float v[2][8];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) Src::expand8(Src::piece(w[i], j), lut, v[i]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        *reinterpret_cast<uint32_t*>(tile + (32 * (t >> 5) + 8 * j + e) * 128 + 4 * p) =
+            cvt_pk<XT>(__fmul_rn(v[0][e], s[0]), __fmul_rn(v[1][e], s[1]));
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < 8; ++it) {
+    const int r = 32 * it + (t >> 3);
+    if (k0 + r < K)
+      *reinterpret_cast<u32x4*>(out + (k0 + r) * ldo + n0 + 8 * (t & 7)) =
+          *reinterpret_cast<const u32x4*>(tile + r * 128 + 16 * (t & 7));
+  }
+}
+
+// Every other layout: 64 x 64 tiles decoded element by element (coalesced
+// along k), written along either index; zeros past N and K up to the padded
+// reduction length.  out has `rows` rows of ldo.
+template <int XT, class Src, class Scale, bool TRANS>
+__global__ __launch_bounds__(kDecThreads) void decode_any_kernel(Src src, Scale scale, BlockOf blk, int64_t N,
+                                                                 int64_t K, int64_t rows, int64_t ldo,
+                                                                 uint16_t* __restrict__ out) {
+  __shared__ float lut[16];
+  __shared__ uint16_t tile[64][66];
+  const int t = threadIdx.x, c = t & 63;
+  if (t < 16) lut[t] = u2f(kNF4Bits[t]);
+  __syncthreads();
+  const int64_t k0 = int64_t(blockIdx.x) * 64, n0 = int64_t(blockIdx.y) * 64;
+#pragma unroll 4
+  for (int i = 0; i < 16; ++i) {
+    const int r = 4 * i + (t >> 6);
+    const int64_t n = n0 + r, k = k0 + c;
+    float v = 0.0f;
+    if (n < N && k < K) {
+      const int64_t f = n * K + k;
+      v = __fmul_rn(src.at(f, lut), scale(blk(f, n)));
+    }
+    tile[r][c] = uint16_t(to_x16<XT>(v));
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (int i = 0; i < 16; ++i) {
+    const int r = 4 * i + (t >> 6);
+    const int64_t row = (TRANS ? k0 : n0) + r, col = (TRANS ? n0 : k0) + c;
+    if (row < rows && col < ldo) out[row * ldo + col] = TRANS ? tile[c][r] : tile[r][c];
+  }
+}
+
+// The small operands, one launch: `cnt` words zeroed, and up to four 16-bit
+// copies out[r][c] = RND(in[r * sr + c * sc]) with zeros past the source's
+// rows and columns -- the GEMM's second LoRA operand, and for reduction lengths
+// that are not multiples of 64 the activations, the LoRA input and the first
+// LoRA factor.
+struct PadCopy {
+  const void* in;
+  int dt;
+  int64_t sr, sc;
+  int64_t rows, cols;          // live part
+  int64_t out_rows, out_cols;  // out_cols a multiple of 8
+  uint16_t* out;
+  int64_t first;               // first workgroup
+};
+struct PadCopies {
+  PadCopy c[4];
+  int n;
+  uint32_t* cnt;
+  int n_cnt;
+};
+
+template <int XT>
+__global__ __launch_bounds__(kDecThreads) void pad_copy_kernel(PadCopies P) {
+  const int64_t g = blockIdx.x;
+  if (g == 0)
+    for (int i = threadIdx.x; i < P.n_cnt; i += kDecThreads) P.cnt[i] = 0u;
+  for (int i = 0; i < P.n; ++i) {
+    const PadCopy& c = P.c[i];
+    const int64_t per = c.out_cols / 8, groups = c.out_rows * per;
+    const int64_t idx = (g - c.first) * kDecThreads + threadIdx.x;
+    if (g < c.first || idx >= groups) continue;
+    // lanes run along the source's contiguous index
+    int64_t r, c8;
+    if (c.sc == 1) {
+      r = idx / per;
+      c8 = (idx - r * per) * 8;
+    } else {
+      const int64_t q = idx / c.out_rows;
+      r = idx - q * c.out_rows;
+      c8 = q * 8;
+    }
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = r < c.rows && c8 + e < c.cols ? load_as_f32(c.in, r * c.sr + (c8 + e) * c.sc, c.dt) : 0.0f;
+    *reinterpret_cast<u32x4*>(c.out + r * c.out_cols + c8) =
+        u32x4{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3]), cvt_pk<XT>(v[4], v[5]), cvt_pk<XT>(v[6], v[7])};
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Plan
+// ---------------------------------------------------------------------------
+constexpr int kDnMaxSplits = 4;
+constexpr size_t kPad = 256;
+size_t up(size_t b) { return (b + kPad - 1) / kPad * kPad; }
+
+struct DensePlan {
+  int halves, tiles_m, tiles_n, whole, splits;
+  int64_t Rp, r16;
+  bool pad;  // the reduction length is padded: activations and factors copied
+  LoraRowsPlan lr;
+  size_t w, cnt, b16, u16, lpart, x, xl, s16, part, bytes;
+};
+
+// Microseconds of a tiling, from measurements with all 256 compute units busy:
+// 1.5 us per 64-k step of a 256 x 256 tile and 0.55 us of a 128 x 128 one
+// (N(0, 1) operands; power bound), K splits adding 20 and 8 us for their
+// partial tiles (2048 x 4096 x 4096: 128 tiles of 256 in two splits 77 us,
+// 512 tiles of 128 unsplit 69 us; 1024 x 4096 x 4096: 55.6 and 35.5 us;
+// 4096 x 4096 x 14336: 347 and 429 us).
+double pick_tiles(DensePlan& p, int64_t M, int64_t C, int nk, int cus) {
+  double best = 1e300;
+  for (int h = 2; h >= 1; --h) {
+    const int64_t B = 128 * h, tm = ceil_div(M, B), tn = ceil_div(C, B), T = tm * tn;
+    const double step = h == 2 ? 1.5 : 0.55, extra = h == 2 ? 20.0 : 8.0;
+    const int64_t lt = T % cus, lf = T - lt;
+    for (int s = 1; s <= kDnMaxSplits; s *= 2) {
+      if (s > 1 && (lt == 0 || lt * s > cus || nk / s < 4)) break;
+      const double t = step * (double(lf / cus) * nk + (lt ? double(ceil_div(nk, s)) : 0.0)) + (s > 1 ? extra : 0.0);
+      if (t < best) {
+        best = t;
+        p.halves = h;
+        p.tiles_m = int(tm);
+        p.tiles_n = int(tn);
+        p.splits = s;
+        p.whole = int(s > 1 ? lf : T);
+      }
+    }
+  }
+  return best;
+}
+
+DensePlan plan_dense(int64_t M, int64_t C, int64_t R, int64_t rank, int cus) {
+  DensePlan p{};
+  p.Rp = (R + 63) / 64 * 64;
+  p.pad = p.Rp != R;
+  p.r16 = rank > 0 ? (rank + 15) / 16 * 16 : 0;
+  pick_tiles(p, M, C, int(p.Rp / 64), cus);
+  size_t off = 0;
+  auto take = [&](size_t b) {
+    const size_t o = off;
+    off += up(b);
+    return o;
+  };
+  p.w = take(size_t(C) * p.Rp * 2);
+  p.cnt = take(size_t(p.tiles_m) * p.tiles_n - p.whole ? (size_t(p.tiles_m) * p.tiles_n - p.whole) * 4 : 4);
+  if (rank > 0) {
+    p.lr = plan_lora_rows(M, p.Rp, rank, cus);
+    p.b16 = take(size_t(C) * p.r16 * 2);
+    p.u16 = take(size_t(M) * p.r16 * 2);
+    p.lpart = take(p.lr.part_bytes);
+  }
+  if (p.pad) {
+    p.x = take(size_t(M) * p.Rp * 2);
+    if (rank > 0) {
+      p.xl = take(size_t(M) * p.Rp * 2);
+      p.s16 = take(size_t(rank) * p.Rp * 2);
+    }
+  }
+  if (p.splits > 1) {
+    const size_t B = 128 * p.halves, lt = size_t(p.tiles_m) * p.tiles_n - p.whole;
+    p.part = take(size_t(p.splits) * lt * B * B * 4);
+  }
+  p.bytes = off;
+  return p;
+}
+
+// A product: activations x [M][R], the weight's columns C.
+struct Product {
+  int xt;
+  const void* x;
+  int64_t ldx, M, C, R;
+  // LoRA: u = RND(RND(xl * pre) . RND(S)^T), S[j][r] at s[j s_j + r s_r];
+  // second factor F[c][j] at f[c f_c + j f_j]
+  int64_t rank;
+  const void* xl;
+  int64_t ldxl;
+  const void* s;
+  int64_t s_j, s_r;
+  bool prescale;
+  float pre;
+  const void* f;
+  int64_t f_c, f_j;
+  int lora_dt;
+  DenseEpi e;
+};
+
+template <int XT, class Src, class Scale>
+int launch_decode(Src src, Scale scale, int64_t N, int64_t K, int64_t bs, bool trans, int64_t Rp, uint16_t* out,
+                  hipStream_t stream) {
+  const BlockOf blk{bs, bs > 0 ? pow2_shift(bs) : -1};
+  const bool blocks_ok = bs == 0 || (blk.log2 >= 5 && K % bs == 0);
+  const int64_t chunks = N * (K / 8);
+  if (!trans && K % 64 == 0 && blocks_ok && aligned(src.p, 8) && chunks < int64_t(UINT32_MAX) - 4096) {
+    decode_rows_kernel<XT, Src, Scale><<<unsigned(ceil_div(chunks, 4 * kDecThreads)), kDecThreads, 0, stream>>>(
+        src, scale, blk, uint32_t(chunks), uint32_t(K / 8), reinterpret_cast<u32x4*>(out));
+  } else if (trans && K % 64 == 0 && N % 64 == 0 && blocks_ok && aligned(src.p, 16) && N / 64 <= 65535) {
+    decode_cols_kernel<XT, Src, Scale>
+        <<<dim3(unsigned(ceil_div(K, 256)), unsigned(N / 64)), kDecThreads, 0, stream>>>(src, scale, blk, K, Rp, out);
+  } else {
+    // tiles over the output: its padded reduction index and its rows
+    const int64_t tk = trans ? ceil_div(K, 64) : Rp / 64, tn = trans ? Rp / 64 : ceil_div(N, 64);
+    if (tn > 65535) return RQ_ERR_UNSUPPORTED;
+    const dim3 grid{unsigned(tk), unsigned(tn)};
+    if (trans)
+      decode_any_kernel<XT, Src, Scale, true><<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, K, Rp, out);
+    else
+      decode_any_kernel<XT, Src, Scale, false><<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, N, Rp, out);
+  }
+  return rq_check_launch();
+}
+
+// The launches of a product whose weight `decode` writes into w16.
+template <int XT, class Decode>
+int run_product(const Product& P, const Decode& decode, void* scratch, size_t bytes, hipStream_t stream) {
+  const DensePlan p = plan_dense(P.M, P.C, P.R, P.rank, device_cus());
+  if (!scratch || bytes < p.bytes) return RQ_ERR_WORKSPACE;
+  if (!aligned(scratch, 256)) return RQ_ERR_BAD_ALIGNMENT;
+  char* ws = static_cast<char*>(scratch);
+  uint16_t* w16 = reinterpret_cast<uint16_t*>(ws + p.w);
+  uint32_t* cnt = reinterpret_cast<uint32_t*>(ws + p.cnt);
+  int st = decode(w16, p.Rp);
+  if (st != RQ_OK) return st;
+
+  DenseEpi e = P.e;
+  DenseGemmArgs a{};
+  a.x = static_cast<const uint16_t*>(P.x);
+  a.ldx = P.ldx;
+  const uint16_t* xl = static_cast<const uint16_t*>(P.xl);
+  int64_t ldxl = P.ldxl;
+  const void* s = P.s;
+  int64_t s_j = P.s_j, s_r = P.s_r;
+  int s_dt = P.lora_dt;
+
+  PadCopies pc{};
+  int64_t groups = 0;
+  auto copy = [&](const void* in, int dt, int64_t sr, int64_t sc, int64_t rows, int64_t cols, int64_t out_rows,
+                  int64_t out_cols, size_t off) {
+    PadCopy& c = pc.c[pc.n++];
+    c = PadCopy{in, dt, sr, sc, rows, cols, out_rows, out_cols, reinterpret_cast<uint16_t*>(ws + off), groups};
+    groups += ceil_div(out_rows * (out_cols / 8), kDecThreads);
+    return reinterpret_cast<uint16_t*>(ws + off);
+  };
+  if (P.rank > 0) {
+    e.rank16 = int(p.r16);
+    e.u = reinterpret_cast<uint16_t*>(ws + p.u16);
+    e.b = copy(P.f, P.lora_dt, P.f_c, P.f_j, P.C, P.rank, P.C, p.r16, p.b16);
+  }
+  if (p.pad) {
+    const bool same = P.xl == P.x && P.ldxl == P.ldx;
+    a.x = copy(P.x, XT, P.ldx, 1, P.M, P.R, P.M, p.Rp, p.x);
+    a.ldx = p.Rp;
+    if (P.rank > 0) {
+      xl = same ? a.x : copy(P.xl, XT, P.ldxl, 1, P.M, P.R, P.M, p.Rp, p.xl);
+      ldxl = p.Rp;
+      s = copy(P.s, P.lora_dt, P.s_j, P.s_r, P.rank, P.R, P.rank, p.Rp, p.s16);
+      s_j = p.Rp;
+      s_r = 1;
+      s_dt = XT;
+    }
+  }
+  if (p.splits > 1) {
+    pc.cnt = cnt;
+    pc.n_cnt = p.tiles_m * p.tiles_n - p.whole;
+  }
+  if (pc.n > 0 || pc.n_cnt > 0) {
+    if (groups > int64_t(INT32_MAX)) return RQ_ERR_UNSUPPORTED;
+    pad_copy_kernel<XT><<<unsigned(std::max<int64_t>(groups, 1)), kDecThreads, 0, stream>>>(pc);
+    if ((st = rq_check_launch()) != RQ_OK) return st;
+  }
+  if (P.rank > 0) {
+    st = run_lora_rows(XT, xl, ldxl, P.M, p.Rp, s, s_dt, s_j, s_r, int(P.rank), P.prescale, P.pre, p.lr,
+                       reinterpret_cast<float*>(ws + p.lpart), reinterpret_cast<uint16_t*>(ws + p.u16), int(p.r16),
+                       stream);
+    if (st != RQ_OK) return st;
+  }
+  a.w = w16;
+  a.ldw = p.Rp;
+  a.M = P.M;
+  a.N = P.C;
+  a.nk = int(p.Rp / 64);
+  a.tiles_m = p.tiles_m;
+  a.tiles_n = p.tiles_n;
+  a.whole = p.whole;
+  a.splits = p.splits;
+  a.part = reinterpret_cast<float*>(ws + p.part);
+  a.tile_cnt = cnt;
+  const int64_t T = int64_t(p.tiles_m) * p.tiles_n;
+  const unsigned grid = unsigned(p.whole + (T - p.whole) * p.splits);
+  if (p.halves == 2) dense_gemm_kernel<XT, 2><<<grid, kDnThreads, 0, stream>>>(a, e);
+  else dense_gemm_kernel<XT, 1><<<grid, kDnThreads, 0, stream>>>(a, e);
+  return rq_check_launch();
+}
+
+// `fn(scale)` with the scale provider of an NF4 weight.
+template <class Fn>
+int with_nf4_scale(const void* absmax, int dt, const uint8_t* c2, int c2_format, int64_t block2, const Fn& fn) {
+  if (c2) {
+    const int sh = pow2_shift(block2);
+    switch (dt) {
+      case RQ_DTYPE_F32: return fn(ScaleDQ<RQ_DTYPE_F32>{c2, absmax, c2_format, sh, block2});
+      case RQ_DTYPE_BF16: return fn(ScaleDQ<RQ_DTYPE_BF16>{c2, absmax, c2_format, sh, block2});
+      default: return fn(ScaleDQ<RQ_DTYPE_F16>{c2, absmax, c2_format, sh, block2});
+    }
+  }
+  switch (dt) {
+    case RQ_DTYPE_F32: return fn(ScaleAbsmax<RQ_DTYPE_F32>{absmax});
+    case RQ_DTYPE_BF16: return fn(ScaleAbsmax<RQ_DTYPE_BF16>{absmax});
+    default: return fn(ScaleAbsmax<RQ_DTYPE_F16>{absmax});
+  }
+}
+
+template <int XT, class Src, class WithScale>
+int run_weight(const Product& P, const Src& src, const WithScale& with_scale, int64_t N, int64_t K, int64_t bs,
+               bool trans, void* scratch, size_t bytes, hipStream_t stream) {
+  return run_product<XT>(
+      P,
+      [&](uint16_t* w16, int64_t Rp) {
+        return with_scale([&](auto sc) { return launch_decode<XT>(src, sc, N, K, bs, trans, Rp, w16, stream); });
+      },
+      scratch, bytes, stream);
+}
+
+bool x16(int dt) { return dt == RQ_DTYPE_BF16 || dt == RQ_DTYPE_F16; }
+
+// 16-byte activation loads when the reduction is not copied into padded rows
+bool act_ok(const void* x, int64_t ldx, int64_t M, int64_t R) {
+  return R % 64 != 0 || (aligned(x, 16) && ldx % 8 == 0 && double(M) * double(ldx) * 2.0 < 4294967296.0);
+}
+
+}  // namespace
+
+size_t dense_scratch_bytes(int x_dtype, int64_t M, int64_t C, int64_t R, int64_t rank) {
+  const int64_t Rp = (R + 63) / 64 * 64;
+  if (!x16(x_dtype) || M < 1 || rank < 0 || rank > 256) return 0;
+  // 32-bit byte offsets into both operands, tile counts in an int
+  if (double(C) * double(Rp) * 2.0 >= 4294967296.0 || double(M) * double(Rp) * 2.0 >= 4294967296.0) return 0;
+  if (ceil_div(M, 128) * ceil_div(C, 128) > int64_t(1) << 28) return 0;
+  return plan_dense(M, C, R, rank > 0 ? rank : 0, device_cus()).bytes;
+}
+
+// Estimates in microseconds from measurements on the Llama-3-8B shapes (M = 64
+// .. 2048): the fused GEMM takes 1.15 us per 64-k step of a full wave of
+// 256 x 128 tiles (0.9 us while fewer than half the compute units have one)
+// and 12 us for its K splits; decoding takes 0.5 us per million weights and its
+// launches 6 us.  Both sides near the line, fused against dense: q forward M =
+// 2048 93 / 105 us, gate forward M = 512 86 / 111 us and M = 1024 165 / 142 us,
+// q dX M = 1024 90 / 62 us, down dX M = 512 98 / 116 us, M = 1024 183 / 145 us.
+bool dense_beats_fused(int64_t M, int64_t C, int64_t R, bool splits) {
+  if (M <= kGemvMaxM) return false;
+  const int cus = device_cus();
+  const GemmPlan f = plan_gemm(M, C, R, 0, cus, splits);
+  const int64_t T = int64_t(f.tiles_m) * f.tiles_n;
+  const double nk = double(R) / 64.0, step = T * f.splits >= cus / 2 ? 1.15 : 0.9;
+  const double waves = f.splits > 1 ? double(f.lf * 8 / cus) + 1.0 / f.splits : double(ceil_div(T, cus));
+  const double fused = nk * step * waves + (f.splits > 1 ? 12.0 : 0.0);
+  DensePlan p{};
+  const double dense = pick_tiles(p, M, C, int((R + 63) / 64), cus);
+  return dense + 6.0 + 0.5e-6 * double(C) * double(R) < fused;
+}
+
+bool dense_nf4_linear_ok(const LinearArgs& L) {
+  return act_ok(L.x, L.ldx, L.M, L.K) && (L.rank == 0 || act_ok(L.lora_x, L.ld_lora_x, L.M, L.K));
+}
+bool dense_nf4_dx_ok(const DxArgs& D) { return act_ok(D.dy, D.lddy, D.M, D.N); }
+bool dense_int8_ok(const GenericInt8& A, bool dx) { return act_ok(A.x, A.ldx, A.M, dx ? A.N : A.K); }
+
+int run_dense_nf4_linear(const LinearArgs& L, void* scratch, size_t bytes, hipStream_t stream) {
+  Product P{};
+  P.xt = L.x_dtype; P.x = L.x; P.ldx = L.ldx; P.M = L.M; P.C = L.N; P.R = L.K;
+  if (L.rank > 0) {
+    P.rank = L.rank; P.xl = L.lora_x; P.ldxl = L.ld_lora_x;
+    P.s = L.lora_a; P.s_j = L.K; P.s_r = 1; P.pre = 1.0f;
+    P.f = L.lora_b; P.f_c = L.ld_lora_b; P.f_j = 1;
+    P.lora_dt = L.lora_dtype;
+  }
+  P.e.bias = L.bias; P.e.bias_dt = L.bias_dtype; P.e.scaling = L.scaling;
+  P.e.y = static_cast<uint16_t*>(L.y); P.e.ldy = L.ldy;
+  auto ws = [&](auto fn) { return with_nf4_scale(L.absmax, L.absmax_dtype, L.c2, L.c2_format, L.block2, fn); };
+  const SrcNF4 src{L.w_packed};
+  return L.x_dtype == RQ_DTYPE_BF16
+             ? run_weight<RQ_DTYPE_BF16>(P, src, ws, L.N, L.K, L.block_size, false, scratch, bytes, stream)
+             : run_weight<RQ_DTYPE_F16>(P, src, ws, L.N, L.K, L.block_size, false, scratch, bytes, stream);
+}
+
+int run_dense_nf4_dx(const DxArgs& D, void* scratch, size_t bytes, hipStream_t stream) {
+  Product P{};
+  P.xt = D.dy_dtype; P.x = D.dy; P.ldx = D.lddy; P.M = D.M; P.C = D.K; P.R = D.N;
+  if (D.rank > 0) {
+    // g = RND(RND(dY * s) . RND(B)), then g . RND(A): S[j][n] = B[n][j], F[k][j] = A[j][k]
+    P.rank = D.rank; P.xl = D.dy; P.ldxl = D.lddy;
+    P.s = D.lora_b; P.s_j = 1; P.s_r = D.ld_lora_b; P.prescale = true; P.pre = D.scaling;
+    P.f = D.lora_a; P.f_c = 1; P.f_j = D.K;
+    P.lora_dt = D.lora_dtype;
+    P.e.mask = D.lora_mask; P.e.ldm = D.ld_lora_mask; P.e.mask_scale = D.mask_scale;
+  }
+  P.e.scaling = 1.0f;
+  P.e.y = static_cast<uint16_t*>(D.dx); P.e.ldy = D.lddx;
+  auto ws = [&](auto fn) { return with_nf4_scale(D.absmax, D.absmax_dtype, D.c2, D.c2_format, D.block2, fn); };
+  const SrcNF4 src{D.w_packed};
+  return D.dy_dtype == RQ_DTYPE_BF16
+             ? run_weight<RQ_DTYPE_BF16>(P, src, ws, D.N, D.K, D.block_size, true, scratch, bytes, stream)
+             : run_weight<RQ_DTYPE_F16>(P, src, ws, D.N, D.K, D.block_size, true, scratch, bytes, stream);
+}
+
+int run_dense_int8(const GenericInt8& A, bool dx, void* scratch, size_t bytes, hipStream_t stream) {
+  Product P{};
+  P.xt = A.x_dtype; P.x = A.x; P.ldx = A.ldx; P.M = A.M; P.C = dx ? A.K : A.N; P.R = dx ? A.N : A.K;
+  P.e.bias = dx ? nullptr : A.bias; P.e.bias_dt = A.bias_dtype; P.e.scaling = 1.0f;
+  P.e.y = static_cast<uint16_t*>(A.y); P.e.ldy = A.ldy;
+  auto ws = [&](auto fn) {
+    return with_nf4_scale(A.scales, A.scales_dtype, nullptr, 0, 1, fn);
+  };
+  const SrcInt8 src{reinterpret_cast<const uint8_t*>(A.q)};
+  return A.x_dtype == RQ_DTYPE_BF16
+             ? run_weight<RQ_DTYPE_BF16>(P, src, ws, A.N, A.K, A.block_size, dx, scratch, bytes, stream)
+             : run_weight<RQ_DTYPE_F16>(P, src, ws, A.N, A.K, A.block_size, dx, scratch, bytes, stream);
+}
+
+}  // namespace rq

@@ -45,6 +45,7 @@
 // k loops start staggered so that only one of them misses on each slice.
 #include "rq_gemm_core.h"
 #include "rq_gemm8.h"
+#include "rq_dense.h"
 #include "rq_generic.h"
 
 namespace rq {
@@ -527,6 +528,39 @@ extern "C" int rq_nf4_linear_dx_workspace_size(int dy_dtype, int64_t M, int64_t 
   const int st = rq::dx_workspace(D, &b);
   *bytes = int64_t(b);
   return st;
+}
+
+extern "C" int rq_nf4_linear_dx_scratch_size(int dy_dtype, int64_t M, int64_t N, int64_t K, int64_t block_size,
+                                             int64_t rank, int64_t* bytes) {
+  if (!bytes) return RQ_ERR_NULL_POINTER;
+  if (!rq::valid_float_dtype(dy_dtype)) return RQ_ERR_BAD_DTYPE;
+  if (M < 0 || N <= 0 || K <= 0 || block_size < 1 || rank < 0 || rank > 256) return RQ_ERR_BAD_SHAPE;
+  const bool fast = N % 64 == 0 && K % 64 == 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0 &&
+                    K % block_size == 0;
+  *bytes = fast && !rq::dense_beats_fused(M, K, N, false) ? 0
+                                                          : int64_t(rq::dense_scratch_bytes(dy_dtype, M, K, N, rank));
+  return RQ_OK;
+}
+
+extern "C" int rq_nf4_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy,
+                                        const uint8_t* w_packed, int64_t K, int64_t block_size, const void* absmax,
+                                        int absmax_dtype, const uint8_t* c2, int c2_format, int64_t block2,
+                                        const void* lora_a, const void* lora_b, int64_t ld_lora_b, int lora_dtype,
+                                        int64_t rank, float scaling, const uint8_t* lora_mask, int64_t ld_lora_mask,
+                                        float mask_scale, void* dx, int64_t lddx, void* workspace,
+                                        int64_t workspace_bytes, void* scratch, int64_t scratch_bytes,
+                                        hipStream_t stream) {
+  const rq::DxArgs D = pack_dx_args(dy, dy_dtype, M, N, lddy, w_packed, K, block_size, absmax, absmax_dtype, c2,
+                                    c2_format, block2, lora_a, lora_b, ld_lora_b, lora_dtype, rank, scaling,
+                                    lora_mask, ld_lora_mask, mask_scale, dx, lddx);
+  const int st = rq::validate_dx(D);
+  if (st != RQ_OK) return st;
+  if (scratch && scratch_bytes > 0 && M > 0) {
+    const size_t need = rq::dense_scratch_bytes(dy_dtype, M, K, N, D.rank > 0 ? D.rank : 0);
+    if (need > 0 && size_t(scratch_bytes) >= need && rq::dense_nf4_dx_ok(D))
+      return rq::run_dense_nf4_dx(D, scratch, size_t(scratch_bytes), stream);
+  }
+  return rq::run_nf4_dx(D, workspace, workspace_bytes < 0 ? 0 : size_t(workspace_bytes), stream);
 }
 
 extern "C" int rq_nf4_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy,

@@ -20,6 +20,7 @@
 #include "rq_launch.h"
 #include "rq_linear.h"
 #include "rq_linear_dev.h"
+#include "rq_dense.h"
 #include "rq_generic.h"
 
 namespace rq {
@@ -1604,6 +1605,31 @@ extern "C" int rq_nf4_linear_workspace_size(int x_dtype, int64_t M, int64_t K, i
   return st;
 }
 
+// rq_nf4_linear's routes; scratch: optional memory for the decoded weight
+static int run_linear(const LinearArgs& L, void* workspace, int64_t workspace_bytes, void* scratch,
+                      int64_t scratch_bytes, hipStream_t stream) {
+  int st = validate_linear(L);
+  if (st != RQ_OK || L.M == 0) return st;
+  if (workspace_bytes < 0 || scratch_bytes < 0) return RQ_ERR_BAD_SHAPE;
+  if (scratch && scratch_bytes > 0) {
+    const size_t need = dense_scratch_bytes(L.x_dtype, L.M, L.N, L.K, L.rank);
+    if (need > 0 && size_t(scratch_bytes) >= need && dense_nf4_linear_ok(L))
+      return run_dense_nf4_linear(L, scratch, size_t(scratch_bytes), stream);
+  }
+  if (!linear_fast_ok(L)) return run_generic_nf4_linear(L, workspace, size_t(workspace_bytes), stream);
+  if (L.x_dtype == RQ_DTYPE_F32) return run_nf4_linear_f32(L, workspace, size_t(workspace_bytes), stream);
+  if (L.M <= kGemvMaxM) return run_nf4_gemv(L, workspace, size_t(workspace_bytes), stream);
+  // the GEMM's workspace follows the synchronization area, whose last
+  // kGemmCountBytes serve as its K splits' tile counters
+  const bool area = workspace && size_t(workspace_bytes) >= kLinearSyncBytes;
+  return run_nf4_gemm(L, area ? static_cast<char*>(workspace) + kLinearSyncBytes : nullptr,
+                      area ? size_t(workspace_bytes) - kLinearSyncBytes : 0,
+                      area ? reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kLinearSyncBytes -
+                                                         kGemmCountBytes)
+                           : nullptr,
+                      kGemmCountBytes / 4, stream);
+}
+
 extern "C" int rq_nf4_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                              const uint8_t* w_packed, int64_t N, int64_t block_size, const void* absmax,
                              int absmax_dtype, const uint8_t* c2, int c2_format, int64_t block2,
@@ -1614,21 +1640,31 @@ extern "C" int rq_nf4_linear(const void* x, int x_dtype, int64_t M, int64_t K, i
   const LinearArgs L = pack_linear_args(x, x_dtype, M, K, ldx, w_packed, N, block_size, absmax, absmax_dtype,
                                         c2, c2_format, block2, bias, bias_dtype, lora_x, ld_lora_x, lora_a,
                                         lora_b, ld_lora_b, lora_dtype, rank, scaling, y, ldy);
-  int st = validate_linear(L);
-  if (st != RQ_OK || M == 0) return st;
-  if (workspace_bytes < 0) return RQ_ERR_BAD_SHAPE;
-  if (!linear_fast_ok(L)) return run_generic_nf4_linear(L, workspace, size_t(workspace_bytes), stream);
-  if (x_dtype == RQ_DTYPE_F32) return run_nf4_linear_f32(L, workspace, size_t(workspace_bytes), stream);
-  if (M <= kGemvMaxM) return run_nf4_gemv(L, workspace, size_t(workspace_bytes), stream);
-  // the GEMM's workspace follows the synchronization area, whose last
-  // kGemmCountBytes serve as its K splits' tile counters
-  const bool area = workspace && size_t(workspace_bytes) >= kLinearSyncBytes;
-  return run_nf4_gemm(L, area ? static_cast<char*>(workspace) + kLinearSyncBytes : nullptr,
-                      area ? size_t(workspace_bytes) - kLinearSyncBytes : 0,
-                      area ? reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kLinearSyncBytes -
-                                                         kGemmCountBytes)
-                           : nullptr,
-                      kGemmCountBytes / 4, stream);
+  return run_linear(L, workspace, workspace_bytes, nullptr, 0, stream);
+}
+
+extern "C" int rq_nf4_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size,
+                                          int64_t rank, int64_t* bytes) {
+  if (!bytes) return RQ_ERR_NULL_POINTER;
+  if (!valid_float_dtype(x_dtype)) return RQ_ERR_BAD_DTYPE;
+  if (M < 0 || N < 1 || K < 1 || block_size < 1 || rank < 0 || rank > 256) return RQ_ERR_BAD_SHAPE;
+  const bool fast = K % 64 == 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0;
+  *bytes = fast && !dense_beats_fused(M, N, K, true) ? 0 : int64_t(dense_scratch_bytes(x_dtype, M, N, K, rank));
+  return RQ_OK;
+}
+
+extern "C" int rq_nf4_linear_scratch(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
+                                     const uint8_t* w_packed, int64_t N, int64_t block_size, const void* absmax,
+                                     int absmax_dtype, const uint8_t* c2, int c2_format, int64_t block2,
+                                     const void* bias, int bias_dtype, const void* lora_x, int64_t ld_lora_x,
+                                     const void* lora_a, const void* lora_b, int64_t ld_lora_b, int lora_dtype,
+                                     int64_t rank, float scaling, void* y, int64_t ldy, void* workspace,
+                                     int64_t workspace_bytes, void* scratch, int64_t scratch_bytes,
+                                     hipStream_t stream) {
+  const LinearArgs L = pack_linear_args(x, x_dtype, M, K, ldx, w_packed, N, block_size, absmax, absmax_dtype,
+                                        c2, c2_format, block2, bias, bias_dtype, lora_x, ld_lora_x, lora_a,
+                                        lora_b, ld_lora_b, lora_dtype, rank, scaling, y, ldy);
+  return run_linear(L, workspace, workspace_bytes, scratch, scratch_bytes, stream);
 }
 
 // ===========================================================================

@@ -42,6 +42,14 @@ SIGNATURES = {
                       _P, _I32,                              # bias, dtype
                       _P, _I64, _P, _P, _I64, _I32, _I64, _F32,  # lora x, ld, A, B, ldB, dtype, rank, scaling
                       _P, _I64, _P, _I64, _P],               # y, ldy, workspace, bytes, stream
+    "rq_nf4_linear_scratch_size": [_I32, _I64, _I64, _I64, _I64, _I64, _P],
+    "rq_nf4_linear_scratch": [_P, _I32, _I64, _I64, _I64,    # x, dtype, M, K, ldx
+                              _P, _I64, _I64, _P, _I32,      # packed, N, block, absmax, dtype
+                              _P, _I32, _I64,                # c2, c2 format, block2
+                              _P, _I32,                      # bias, dtype
+                              _P, _I64, _P, _P, _I64, _I32, _I64, _F32,  # lora x, ld, A, B, ldB, dtype, rank, scaling
+                              _P, _I64, _P, _I64,            # y, ldy, workspace, bytes
+                              _P, _I64, _P],                 # scratch, bytes, stream
     "rq_nf4_linear_noalloc": [_P, _I32, _I64, _I64, _I64,    # x, dtype, M, K, ldx
                               _P, _I64, _I64, _P, _I32,      # packed, N, block, absmax, dtype
                               _P, _I32, _I64,                # c2, c2 format, block2
@@ -52,18 +60,33 @@ SIGNATURES = {
     "rq_gemm_tile_config": [_P],
     "rq_stream_capture_id": [_P, _P],
     "rq_nf4_linear_dx_workspace_size": [_I32, _I64, _I64, _I64, _I64, _P],
+    "rq_nf4_linear_dx_scratch_size": [_I32, _I64, _I64, _I64, _I64, _I64, _P],
     "rq_nf4_linear_dx": [_P, _I32, _I64, _I64, _I64,         # dy, dtype, M, N, lddy
                          _P, _I64, _I64, _P, _I32,           # packed, K, block, absmax, dtype
                          _P, _I32, _I64,                     # c2, c2 format, block2
                          _P, _P, _I64, _I32, _I64, _F32,     # A, B, ldB, dtype, rank, scaling
                          _P, _I64, _F32,                     # dropout mask, ld, mask scale
                          _P, _I64, _P, _I64, _P],            # dx, lddx, workspace, bytes, stream
+    "rq_nf4_linear_dx_scratch": [_P, _I32, _I64, _I64, _I64,         # dy, dtype, M, N, lddy
+                                 _P, _I64, _I64, _P, _I32,           # packed, K, block, absmax, dtype
+                                 _P, _I32, _I64,                     # c2, c2 format, block2
+                                 _P, _P, _I64, _I32, _I64, _F32,     # A, B, ldB, dtype, rank, scaling
+                                 _P, _I64, _F32,                     # dropout mask, ld, mask scale
+                                 _P, _I64, _P, _I64, _P, _I64, _P],  # dx, lddx, workspace, bytes, scratch, bytes, stream
     "rq_int8_linear": [_P, _I32, _I64, _I64, _I64,           # x, dtype, M, K, ldx
                        _P, _I64, _I64, _P, _I32,             # q, N, block, scales, dtype
                        _P, _I32, _P, _I64, _P],              # bias, dtype, y, ldy, stream
     "rq_int8_linear_dx": [_P, _I32, _I64, _I64, _I64,        # dy, dtype, M, N, lddy
                           _P, _I64, _I64, _P, _I32,          # q, K, block, scales, dtype
                           _P, _I64, _P],                     # dx, lddx, stream
+    "rq_int8_linear_scratch_size": [_I32, _I64, _I64, _I64, _I64, _I32, _P],
+    "rq_int8_linear_scratch": [_P, _I32, _I64, _I64, _I64,   # x, dtype, M, K, ldx
+                               _P, _I64, _I64, _P, _I32,     # q, N, block, scales, dtype
+                               _P, _I32, _P, _I64,           # bias, dtype, y, ldy
+                               _P, _I64, _P],                # scratch, bytes, stream
+    "rq_int8_linear_dx_scratch": [_P, _I32, _I64, _I64, _I64,  # dy, dtype, M, N, lddy
+                                  _P, _I64, _I64, _P, _I32,    # q, K, block, scales, dtype
+                                  _P, _I64, _P, _I64, _P],     # dx, lddx, scratch, bytes, stream
     "rq_merge_lora": [_P, _I32, _I64, _I64, _I64,           # w, format, N, K, block
                       _P, _I32, _P, _I32, _I64,             # scales, dtype, c2, c2 format, block2
                       _P, _P, _I64, _I32, _I64, _F32,       # A, B, ldB, dtype, rank, scaling

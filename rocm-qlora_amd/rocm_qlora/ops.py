@@ -139,6 +139,16 @@ def _workspace(x_dtype: torch.dtype, M: int, K: int, N: int, rank: int, dev) -> 
     return ws
 
 
+def _scratch(size_fn: str, dev, *args) -> Optional[torch.Tensor]:
+    """Scratch memory for one call, of the size `size_fn` reports (None when
+    none is used): from torch's caching allocator, which hands it out again in
+    stream order once the tensor is dropped."""
+    import ctypes
+    nbytes = ctypes.c_int64(0)
+    nat.call(size_fn, *args, ctypes.byref(nbytes))
+    return torch.empty(nbytes.value, dtype=torch.uint8, device=dev) if nbytes.value else None
+
+
 def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optional[torch.Tensor],
                out_features: int, block_size: int = 64, bias: Optional[torch.Tensor] = None, *,
                c2: Optional[torch.Tensor] = None, c2_scales: Optional[torch.Tensor] = None,
@@ -177,7 +187,11 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
     with on(dev):
         x2, ldx = _rows(x, K)
         M = x2.shape[0]
-        if (M > GEMV_MAX_M or x.dtype == torch.float32) and K % 64 == 0:  # 16-byte activation loads
+        # the decode GEMV reads any alignment; every other kernel whose rows are
+        # whole 64-element steps reads activations 16 bytes at a time
+        fast_shape = K % 64 == 0 and block_size >= 64 and not block_size & (block_size - 1) and K % block_size == 0
+        wide = K % 64 == 0 and (M > GEMV_MAX_M or x.dtype == torch.float32 or not fast_shape)
+        if wide:
             x2, ldx = _aligned_rows(x2, K)
         y = torch.empty((M, N), dtype=x.dtype, device=dev)
         if M == 0:
@@ -204,21 +218,22 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
                 lb, ldb = lb.contiguous(), rank
             lcode = nat.dtype_code(la.dtype)
             if lora_x is not None:
-                # the GEMM's and the fp32 path's LoRA operand kernels load 16
-                # bytes at a time
-                wide = (M > GEMV_MAX_M or x.dtype == torch.float32) and K % 64 == 0
                 xl, ldxl = (_aligned_rows if wide else _rows)(lora_x.to(x.dtype), K)
         b = bias.contiguous() if bias is not None else None
-        ws = _workspace(x.dtype, M, K, N, rank, dev)
+        scratch = None
+        if (M > GEMV_MAX_M or not fast_shape) and max(ldx, ldxl) * M < 1 << 31:
+            scratch = _scratch("rq_nf4_linear_scratch_size", dev, xcode, M, K, N, block_size, rank)
+        # a call with scratch memory needs no workspace of its own
+        ws = _workspace(x.dtype, M, K, N, rank, dev) if scratch is None else None
         codes = c2.reshape(-1).view(torch.uint8).contiguous() if dq else None
-        nat.call("rq_nf4_linear",
+        nat.call("rq_nf4_linear_scratch",
                  x2.data_ptr(), xcode, M, K, ldx,
                  packed.data_ptr(), N, block_size, scales.data_ptr(), nat.dtype_code(scales.dtype),
                  nat.ptr(codes), nat.C2_FP8_E4M3FNUZ if use_fp8_c2 else nat.C2_INT8, blocksize_2,
                  nat.ptr(b), nat.dtype_code(b.dtype) if b is not None else 0,
                  nat.ptr(xl), ldxl, nat.ptr(la), nat.ptr(lb), ldb, lcode, rank, float(scaling),
                  y.data_ptr(), N, nat.ptr(ws), ws.numel() if ws is not None else 0,
-                 nat.stream_handle(dev))
+                 nat.ptr(scratch), scratch.numel() if scratch is not None else 0, nat.stream_handle(dev))
     return y.reshape(*lead, N)
 
 
@@ -278,19 +293,21 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
             mk, ldm = _rows(lora_mask.reshape(-1, K).view(torch.uint8), K)
             if mk.shape[0] != M:
                 raise RuntimeError(f"lora_mask has {mk.shape[0]} rows, dY {M}")
-        import ctypes
-        nbytes = ctypes.c_int64(0)
-        nat.call("rq_nf4_linear_dx_workspace_size", nat.dtype_code(dy.dtype), M, N, K, rank, ctypes.byref(nbytes))
-        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dev) if nbytes.value else None
+        code = nat.dtype_code(dy.dtype)
+        scratch = ws = None
+        if lddy * M < 1 << 31:
+            scratch = _scratch("rq_nf4_linear_dx_scratch_size", dev, code, M, N, K, block_size, rank)
+        if scratch is None:
+            ws = _scratch("rq_nf4_linear_dx_workspace_size", dev, code, M, N, K, rank)
         codes = c2.reshape(-1).view(torch.uint8).contiguous() if dq else None
-        nat.call("rq_nf4_linear_dx",
+        nat.call("rq_nf4_linear_dx_scratch",
                  dy2.data_ptr(), nat.dtype_code(dy.dtype), M, N, lddy,
                  packed.data_ptr(), K, block_size, scales.data_ptr(), nat.dtype_code(scales.dtype),
                  nat.ptr(codes), nat.C2_FP8_E4M3FNUZ if use_fp8_c2 else nat.C2_INT8, blocksize_2,
                  nat.ptr(la), nat.ptr(lb), ldb, lcode, rank, float(scaling),
                  nat.ptr(mk), ldm, float(mask_scale),
                  dx.data_ptr(), K, nat.ptr(ws), ws.numel() if ws is not None else 0,
-                 nat.stream_handle(dev))
+                 nat.ptr(scratch), scratch.numel() if scratch is not None else 0, nat.stream_handle(dev))
     return dx.reshape(*lead, K)
 
 
@@ -332,10 +349,12 @@ def int8_linear(x: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, out_feat
         if M == 0:
             return y.reshape(*lead, N)
         b = bias.contiguous() if bias is not None else None
-        nat.call("rq_int8_linear", x2.data_ptr(), nat.dtype_code(x.dtype), M, K, ldx,
+        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(x.dtype), M, K, N, block_size, 0)
+        nat.call("rq_int8_linear_scratch", x2.data_ptr(), nat.dtype_code(x.dtype), M, K, ldx,
                  qf.data_ptr(), N, block_size, sc.data_ptr(), nat.dtype_code(sc.dtype),
                  nat.ptr(b), nat.dtype_code(b.dtype) if b is not None else 0,
-                 y.data_ptr(), N, nat.stream_handle(dev))
+                 y.data_ptr(), N, nat.ptr(scratch), scratch.numel() if scratch is not None else 0,
+                 nat.stream_handle(dev))
     return y.reshape(*lead, N)
 
 
@@ -360,14 +379,16 @@ def int8_linear_dx(dy: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, in_f
         raise RuntimeError(f"scales hold {sc.numel()} values, need {need}")
     lead = dy.shape[:-1]
     with on(dev):
-        dy2, lddy = _rows(dy, N)
+        dy2, lddy = _aligned_rows(dy, N) if N % 64 == 0 and dy.dtype != torch.float32 else _rows(dy, N)
         M = dy2.shape[0]
         dx = torch.empty((M, K), dtype=dy.dtype, device=dev)
         if M == 0:
             return dx.reshape(*lead, K)
-        nat.call("rq_int8_linear_dx", dy2.data_ptr(), nat.dtype_code(dy.dtype), M, N, lddy,
+        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(dy.dtype), M, K, N, block_size, 1)
+        nat.call("rq_int8_linear_dx_scratch", dy2.data_ptr(), nat.dtype_code(dy.dtype), M, N, lddy,
                  qf.data_ptr(), K, block_size, sc.data_ptr(), nat.dtype_code(sc.dtype),
-                 dx.data_ptr(), K, nat.stream_handle(dev))
+                 dx.data_ptr(), K, nat.ptr(scratch), scratch.numel() if scratch is not None else 0,
+                 nat.stream_handle(dev))
     return dx.reshape(*lead, K)
 
 

@@ -1,0 +1,175 @@
+"""Linears that decode the weight once into scratch memory and multiply by the
+dense MFMA GEMM (csrc/dense_gemm.hip): tile edges of both tile sizes, K
+splits, reduction lengths that are padded, every decode kernel, the LoRA and
+dropout epilogues, against the oracle at the tolerance of the other linears
+(16-bit results: rtol = atol = 1e-2, gradients relative to the largest).
+
+The entry points are called with scratch memory of the size the library
+reports for the dense path, whatever the row count, through the C ABI."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import qlora_ref as R
+from rocm_qlora import _native as nat
+from rocm_qlora import ops
+from rocm_qlora.quantization import double_quantize, quantize_int4, quantize_int8
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-2
+
+
+def _randn(g, *shape, scale=1.0):
+    return torch.randn(*shape, generator=g) * scale
+
+
+def _check(got, ref, relative=False):
+    got, ref = got.detach().cpu().float(), ref.detach().float()
+    assert got.shape == ref.shape
+    atol = TOL * (float(ref.abs().max()) if relative else 1.0)
+    err = (got - ref).abs()
+    bad = err > atol + TOL * ref.abs()
+    assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside tol; max err {float(err.max()):.4g}"
+
+
+# (M, K, N, block, rank, dtype, storage): rows and columns around the 128- and
+# 256-wide tiles, one to many 64-k steps (prefetches past the end; odd step
+# counts), splits (few tiles, long K), lengths padded to 64, blocks of 32 and
+# blocks that straddle rows, ranks of one and two epilogue steps and past 64
+FORWARD = [
+    (17, 64, 64, 64, 0, "bf16", "f32"),
+    (129, 128, 130, 64, 8, "bf16", "f32"),
+    (256, 192, 256, 64, 16, "fp16", "f32"),
+    (257, 320, 255, 64, 12, "bf16", "dq"),
+    (300, 2048, 96, 128, 80, "bf16", "bf16"),
+    (40, 320, 200, 32, 16, "bf16", "f32"),
+    (33, 37, 73, 64, 4, "fp16", "f32"),
+    (5, 1000, 301, 64, 12, "bf16", "dq"),
+    (1, 130, 1, 64, 1, "bf16", "f32"),
+    (1100, 4096, 512, 64, 64, "bf16", "f32"),
+]
+
+
+def _weight(g, N, K, block, storage, dev):
+    w = _randn(g, N, K, scale=0.02)
+    if storage == "dq":
+        st = double_quantize(w.to(dev), block, 256)
+        kw = dict(c2=st.c2, c2_scales=st.c2_scales, blocksize_2=256, use_fp8_c2=st.use_fp8_c2)
+        wf = R.double_dequantize(st.W_quant.cpu(), st.c2.cpu(), st.c2_scales.cpu().reshape(-1), (N, K), block, 256,
+                                 st.use_fp8_c2)
+        return st.W_quant, None, kw, wf
+    packed, s = quantize_int4(w.to(dev).to(torch.bfloat16 if storage == "bf16" else torch.float32), block)
+    s = s.reshape(-1)
+    return packed, s, {}, R.dequantize_int4(packed.cpu(), s.cpu(), block)[:N * K].reshape(N, K)
+
+
+@pytest.fixture
+def always_dense(monkeypatch):
+    """The wrappers with the rule set aside: scratch memory for every call and
+    the C entry point it belongs to (a block size no fused kernel takes is
+    reported to the size query, so that it answers for the dense path)."""
+    real = ops._scratch
+
+    def scratch(fn, dev, *args):
+        if "scratch" not in fn:
+            return real(fn, dev, *args)
+        nb = ctypes.c_int64(0)
+        args = list(args)
+        args[4] = 7
+        nat.call(fn, *args, ctypes.byref(nb))
+        assert nb.value > 0
+        return torch.full((nb.value,), 0xFF, dtype=torch.uint8, device=dev)  # NaN patterns: contents must not matter
+
+    monkeypatch.setattr(ops, "_scratch", scratch)
+
+
+@pytest.mark.parametrize("M,K,N,block,rank,dtype,storage", FORWARD)
+def test_dense_forward(dev, always_dense, M, K, N, block, rank, dtype, storage):
+    print(f"dense forward {M} {K} {N} {block} {rank} {dtype} {storage}", flush=True)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    g = torch.Generator().manual_seed(M + K + N)
+    packed, s, kw, wf = _weight(g, N, K, block, storage, dev)
+    x, bias = _randn(g, M, K).to(dt), _randn(g, N, scale=0.1)
+    a, b = _randn(g, rank, K, scale=0.05), _randn(g, N, rank, scale=0.05)
+    y = ops.nf4_linear(x.to(dev), packed, s, N, block, bias.to(dt).to(dev), lora_a=a.to(dev) if rank else None,
+                       lora_b=b.to(dev) if rank else None, scaling=0.5, **kw)
+    ref = R.quant_linear_forward(x, wf.reshape(-1), bias, N, K)
+    if rank:
+        ref = R.lora_forward(x, ref, a, b, 0.5)
+    _check(y, ref)
+
+
+@pytest.mark.parametrize("M,K,N,block,rank,dtype,storage,masked",
+                         [(*c, m) for c in FORWARD for m in (False, True) if c[4] or not m])
+def test_dense_dx(dev, always_dense, M, K, N, block, rank, dtype, storage, masked):
+    print(f"dense dx {M} {K} {N} {block} {rank} {dtype} {storage} {masked}", flush=True)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    g = torch.Generator().manual_seed(M + K + N + 1)
+    packed, s, kw, wf = _weight(g, N, K, block, storage, dev)
+    dy = _randn(g, M, N, scale=0.05).to(dt)
+    a, b = _randn(g, rank, K, scale=0.05), _randn(g, N, rank, scale=0.05)
+    mask = torch.rand(M, K, generator=g) < 0.8
+    dx = ops.nf4_linear_dx(dy.to(dev), packed, s, K, block, lora_a=a.to(dev) if rank else None,
+                           lora_b=b.to(dev) if rank else None, scaling=0.5,
+                           lora_mask=mask.to(dev) if masked else None, mask_scale=1.25 if masked else 1.0, **kw)
+    ref = dy.float() @ wf.to(dt).float()
+    ref = ref.to(dt)
+    if rank:
+        l = (dy * 0.5) @ b.to(dt) @ a.to(dt)
+        ref = ref + (l * (mask.to(dt) * 1.25) if masked else l)
+    _check(dx, ref, relative=True)
+
+
+@pytest.mark.parametrize("M,K,N,block", [(17, 64, 64, 0), (130, 320, 192, 64), (300, 129, 257, 0), (20, 96, 64, 32),
+                                         (257, 2048, 96, 128), (3, 73, 37, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_int8(dev, always_dense, M, K, N, block, dtype):
+    print(f"dense int8 {M} {K} {N} {block} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(M + K + N + 2)
+    w = _randn(g, N, K, scale=0.02).to(dev)
+    q, s = quantize_int8(w, per_channel=True) if block == 0 else quantize_int8(w, block)
+    wf = R.dequantize_int8(q.cpu(), s.cpu().reshape(-1), block or 64).reshape(-1)[:N * K].reshape(N, K).to(dtype)
+    x, dy, bias = _randn(g, M, K).to(dtype), _randn(g, M, N, scale=0.05).to(dtype), _randn(g, N, scale=0.1)
+    y = ops.int8_linear(x.to(dev), q, s, N, block, bias.to(dtype).to(dev))
+    _check(y, torch.nn.functional.linear(x, wf, bias.to(dtype)))
+    dx = ops.int8_linear_dx(dy.to(dev), q, s, K, block)
+    _check(dx, (dy.float() @ wf.float()).to(dtype), relative=True)
+
+
+def test_dense_rule_matches_general_path(dev):
+    """Calls that the rule sends to the dense path against the same calls
+    without scratch memory (the fused and generic kernels), strided and
+    misaligned activations among them: the operands round alike, so the
+    results differ by the order of fp32 sums and its effect on one rounding."""
+    g = torch.Generator().manual_seed(5)
+    N, K, M = 4096, 1024, 4096
+    w = _randn(g, N, K, scale=0.02).to(dev)
+    packed, s = quantize_int4(w, 64)
+    q, qs = quantize_int8(w, 64)
+    wide = _randn(g, M, K + 4).to(torch.bfloat16).to(dev)
+    dy = _randn(g, M, N, scale=0.05).to(torch.bfloat16).to(dev)
+    real = ops._scratch
+    for x in (wide[:, :K].contiguous(), wide[:, :K], wide[:, 1:K + 1]):
+        calls = [lambda: ops.nf4_linear(x, packed, s, N, 64), lambda: ops.nf4_linear_dx(dy, packed, s, K, 64),
+                 lambda: ops.int8_linear(x, q, qs, N, 64), lambda: ops.int8_linear_dx(dy, q, qs, K, 64)]
+        for i, call in enumerate(calls):
+            sizes = []
+
+            def spy(fn, dev_, *args):
+                r = real(fn, dev_, *args)
+                if "scratch" in fn:
+                    sizes.append(0 if r is None else r.numel())
+                return r
+
+            ops._scratch = spy
+            try:
+                got = call()
+                assert sizes and sizes[0] > 0, f"call {i} is expected on the dense path"
+                ops._scratch = lambda fn, dev_, *args: None if "scratch" in fn else real(fn, dev_, *args)
+                ref = call()
+            finally:
+                ops._scratch = real
+            # one bf16 rounding may fall the other way: 2^-8 of the value
+            d = (got.float() - ref.float()).abs()
+            assert bool((d <= 2.0 ** -7 * ref.float().abs() + 1e-5 * float(ref.abs().max())).all()), f"call {i}"
