@@ -182,11 +182,11 @@ int rq_nf4_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                   hipStream_t stream);
 
 /* rq_nf4_linear with optional scratch memory (256-byte aligned device memory,
- * contents ignored, free again once the call's kernels are done).  A 16-bit
- * call given the bytes it needs decodes the weight into it once and multiplies
+ * contents ignored, free again once the call's kernels are done).  A call
+ * given the bytes it needs decodes the weight into it once and multiplies
  * by the dense MFMA GEMM (same operand roundings, another order of fp32 sums);
  * any other call is rq_nf4_linear.  rq_nf4_linear_scratch_size reports those
- * bytes where that is the faster route (many rows, and the calls that
+ * bytes where that is the faster route (many rows, and most calls that
  * otherwise run on the generic kernels), 0 elsewhere. */
 int rq_nf4_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int64_t rank,
                                int64_t* bytes);

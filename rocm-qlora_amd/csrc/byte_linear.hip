@@ -404,7 +404,7 @@ extern "C" int rq_int8_linear_scratch_size(int x_dtype, int64_t M, int64_t K, in
   if (!bytes) return RQ_ERR_NULL_POINTER;
   if (!rq::valid_float_dtype(x_dtype)) return RQ_ERR_BAD_DTYPE;
   if (M < 0 || N < 1 || K < 1 || block_size < 0) return RQ_ERR_BAD_SHAPE;
-  const bool fast = !dx && K % 64 == 0 &&
+  const bool fast = !dx && x_dtype != RQ_DTYPE_F32 && K % 64 == 0 &&
                     (block_size == 0 ||
                      (block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0));
   const int64_t C = dx ? K : N, R = dx ? N : K;

@@ -62,13 +62,34 @@ struct BlockOf {
 
 constexpr int kDecThreads = 256;
 
+// Eight values in the operand type at p (16-byte aligned): 16 or 32 bytes.
+template <int XT>
+__device__ __forceinline__ void store8(void* p, const float (&v)[8]) {
+  u32x4* o = static_cast<u32x4*>(p);
+  if constexpr (XT == RQ_DTYPE_F32) {
+    o[0] = u32x4{f2u(v[0]), f2u(v[1]), f2u(v[2]), f2u(v[3])};
+    o[1] = u32x4{f2u(v[4]), f2u(v[5]), f2u(v[6]), f2u(v[7])};
+  } else {
+    o[0] = u32x4{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3]), cvt_pk<XT>(v[4], v[5]), cvt_pk<XT>(v[6], v[7])};
+  }
+}
+
+// one value in the operand type, as its storage word
+template <int XT>
+using Word = std::conditional_t<XT == RQ_DTYPE_F32, uint32_t, uint16_t>;
+template <int XT>
+__device__ __forceinline__ Word<XT> to_word(float v) {
+  if constexpr (XT == RQ_DTYPE_F32) return f2u(v);
+  else return uint16_t(to_x16<XT>(v));
+}
+
 // W rows, K % 64 == 0 and blocks of at least 8 inside a row: the output is
 // the flat weight.  A lane takes 8 codes (one 16-byte store, consecutive
 // lanes consecutive bytes), four such per thread, all loads first.  HBM and
 // MALL writes bound it (measured at 4096 x 14336: see launch_decode).
 template <int XT, class Src, class Scale>
 __global__ __launch_bounds__(kDecThreads) void decode_rows_kernel(Src src, Scale scale, BlockOf blk, uint32_t n_chunks,
-                                                                  uint32_t row_chunks, u32x4* __restrict__ out) {
+                                                                  uint32_t row_chunks, uint8_t* __restrict__ out) {
   __shared__ float lut[16];
   if (threadIdx.x < 16) lut[threadIdx.x] = u2f(kNF4Bits[threadIdx.x]);
   __syncthreads();
@@ -91,10 +112,9 @@ __global__ __launch_bounds__(kDecThreads) void decode_rows_kernel(Src src, Scale
     if (c >= n_chunks) break;
     float v[8];
     Src::expand8(w[j], lut, v);
-    uint32_t o[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o[k] = cvt_pk<XT>(__fmul_rn(v[2 * k], s[j]), __fmul_rn(v[2 * k + 1], s[j]));
-    out[c] = u32x4{o[0], o[1], o[2], o[3]};
+    for (int k = 0; k < 8; ++k) v[k] = __fmul_rn(v[k], s[j]);
+    store8<XT>(out + size_t(c) * (8 * DnEl<XT>::kSize), v);
   }
 }
 
@@ -105,9 +125,10 @@ __global__ __launch_bounds__(kDecThreads) void decode_rows_kernel(Src src, Scale
 // row), which leaves as 128-byte runs of the output's rows.
 template <int XT, class Src, class Scale>
 __global__ __launch_bounds__(kDecThreads) void decode_cols_kernel(Src src, Scale scale, BlockOf blk, int64_t K,
-                                                                  int64_t ldo, uint16_t* __restrict__ out) {
+                                                                  int64_t ldo, uint8_t* __restrict__ out) {
+  constexpr int ES = DnEl<XT>::kSize, kRow = 64 * ES;  // bytes of 64 rows' values of one column
   __shared__ float lut[16];
-  __shared__ __attribute__((aligned(16))) uint8_t tile[256 * 128];
+  __shared__ __attribute__((aligned(16))) uint8_t tile[256 * kRow];
   const int t = threadIdx.x, p = t & 31;
   if (t < 16) lut[t] = u2f(kNF4Bits[t]);
   __syncthreads();
@@ -130,18 +151,22 @@ __global__ __launch_bounds__(kDecThreads) void decode_cols_kernel(Src src, Scale
 #pragma unroll
       for (int i = 0; i < 2; ++i) Src::expand8(Src::piece(w[i], j), lut, v[i]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        *reinterpret_cast<uint32_t*>(tile + (32 * (t >> 5) + 8 * j + e) * 128 + 4 * p) =
-            cvt_pk<XT>(__fmul_rn(v[0][e], s[0]), __fmul_rn(v[1][e], s[1]));
+      for (int e = 0; e < 8; ++e) {
+        uint8_t* o = tile + (32 * (t >> 5) + 8 * j + e) * kRow + 2 * ES * p;
+        const float a = __fmul_rn(v[0][e], s[0]), b = __fmul_rn(v[1][e], s[1]);
+        if constexpr (XT == RQ_DTYPE_F32) *reinterpret_cast<u32x2*>(o) = u32x2{f2u(a), f2u(b)};
+        else *reinterpret_cast<uint32_t*>(o) = cvt_pk<XT>(a, b);
+      }
     }
   }
   __syncthreads();
+  constexpr int kLanes = kRow / 16;  // 16-byte chunks per column
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int r = 32 * it + (t >> 3);
+  for (int it = 0; it < kLanes; ++it) {
+    const int r = (kDecThreads / kLanes) * it + t / kLanes, c = t % kLanes;
     if (k0 + r < K)
-      *reinterpret_cast<u32x4*>(out + (k0 + r) * ldo + n0 + 8 * (t & 7)) =
-          *reinterpret_cast<const u32x4*>(tile + r * 128 + 16 * (t & 7));
+      *reinterpret_cast<u32x4*>(out + ((k0 + r) * ldo + n0) * ES + 16 * c) =
+          *reinterpret_cast<const u32x4*>(tile + r * kRow + 16 * c);
   }
 }
 
@@ -151,9 +176,9 @@ __global__ __launch_bounds__(kDecThreads) void decode_cols_kernel(Src src, Scale
 template <int XT, class Src, class Scale, bool TRANS>
 __global__ __launch_bounds__(kDecThreads) void decode_any_kernel(Src src, Scale scale, BlockOf blk, int64_t N,
                                                                  int64_t K, int64_t rows, int64_t ldo,
-                                                                 uint16_t* __restrict__ out) {
+                                                                 Word<XT>* __restrict__ out) {
   __shared__ float lut[16];
-  __shared__ uint16_t tile[64][66];
+  __shared__ Word<XT> tile[64][64 + 4 / sizeof(Word<XT>)];
   const int t = threadIdx.x, c = t & 63;
   if (t < 16) lut[t] = u2f(kNF4Bits[t]);
   __syncthreads();
@@ -167,7 +192,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_any_kernel(Src src, Scale 
       const int64_t f = n * K + k;
       v = __fmul_rn(src.at(f, lut), scale(blk(f, n)));
     }
-    tile[r][c] = uint16_t(to_x16<XT>(v));
+    tile[r][c] = to_word<XT>(v);
   }
   __syncthreads();
 #pragma unroll 4
@@ -178,18 +203,17 @@ __global__ __launch_bounds__(kDecThreads) void decode_any_kernel(Src src, Scale 
   }
 }
 
-// The small operands, one launch: `cnt` words zeroed, and up to four 16-bit
-// copies out[r][c] = RND(in[r * sr + c * sc]) with zeros past the source's
+// The small operands, one launch: `cnt` words zeroed, and up to four copies out[r][c] = RND(in[r * sr + c * sc]) with zeros past the source's
 // rows and columns -- the GEMM's second LoRA operand, and for reduction lengths
-// that are not multiples of 64 the activations, the LoRA input and the first
-// LoRA factor.
+// that are not whole k steps the activations, the LoRA input and the first
+// LoRA factor (fp32: always the first factor).
 struct PadCopy {
   const void* in;
   int dt;
   int64_t sr, sc;
   int64_t rows, cols;          // live part
   int64_t out_rows, out_cols;  // out_cols a multiple of 8
-  uint16_t* out;
+  void* out;
   int64_t first;               // first workgroup
 };
 struct PadCopies {
@@ -223,24 +247,92 @@ __global__ __launch_bounds__(kDecThreads) void pad_copy_kernel(PadCopies P) {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
       v[e] = r < c.rows && c8 + e < c.cols ? load_as_f32(c.in, r * c.sr + (c8 + e) * c.sc, c.dt) : 0.0f;
-    *reinterpret_cast<u32x4*>(c.out + r * c.out_cols + c8) =
-        u32x4{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3]), cvt_pk<XT>(v[4], v[5]), cvt_pk<XT>(v[6], v[7])};
+    store8<XT>(static_cast<uint8_t*>(c.out) + (r * c.out_cols + c8) * DnEl<XT>::kSize, v);
   }
+}
+
+// u = RN(xl * pre) . S^T in fp32 on v_mfma_f32_16x16x4_f32, as K-split partials
+// part[split][m][j] (the split's k steps of 32 in order): four waves of 16 rows
+// per workgroup, up to 64 ranks; then their sum in split order into rows of
+// rankp (zeros past the rank).  Lane (i, q) loads 16 bytes of row i at k = 16 t +
+// 4 q in both operands, four MFMAs' k.  Latency bound: 16-64 ranks of a few
+// hundred rows, so the splits spread it over the compute units.
+template <int JB>
+__global__ __launch_bounds__(256) void lora_rows_f32_kernel(const float* __restrict__ x, int64_t ldx, int64_t M,
+                                                            const float* __restrict__ s, int64_t lds_, int rank,
+                                                            float pre, int steps, int steps_per,
+                                                            float* __restrict__ part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, q = lane >> 4;
+  const int64_t m0 = int64_t(blockIdx.x) * 64 + 16 * wave;
+  const int j0 = blockIdx.y * 16 * JB, b = blockIdx.z * steps_per;
+  const int e = b + steps_per < steps ? b + steps_per : steps;
+  int64_t m = m0 + i16;
+  m = m < M ? m : M - 1;
+  const float* xr = x + m * ldx + 4 * q;
+  const float* sr[JB];
+#pragma unroll
+  for (int jb = 0; jb < JB; ++jb) {
+    const int j = j0 + 16 * jb + i16;
+    sr[jb] = s + int64_t(j < rank ? j : rank - 1) * lds_ + 4 * q;  // ranks past the end: never stored
+  }
+  f32x4 acc[JB];
+#pragma unroll
+  for (int jb = 0; jb < JB; ++jb) acc[jb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = b; t < e; ++t) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t k = 32 * int64_t(t) + 16 * h;
+      const f32x4 xv = *reinterpret_cast<const f32x4*>(xr + k);
+#pragma unroll
+      for (int jb = 0; jb < JB; ++jb) {
+        const f32x4 sv = *reinterpret_cast<const f32x4*>(sr[jb] + k);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(__fmul_rn(xv[c], pre), sv[c], acc[jb], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int jb = 0; jb < JB; ++jb) {
+    const int j = j0 + 16 * jb + i16;
+    if (j >= rank) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t mo = m0 + 4 * q + r;
+      if (mo < M) part[(int64_t(blockIdx.z) * M + mo) * rank + j] = acc[jb][r];
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void lora_sum_f32_kernel(const float* __restrict__ part, int splits, int64_t M,
+                                                           int rank, int rankp, float* __restrict__ u) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= M * rankp) return;
+  const int64_t m = i / rankp;
+  const int j = int(i - m * rankp);
+  float v = 0.0f;
+  if (j < rank) {
+#pragma unroll 8
+    for (int k = 0; k < splits; ++k) v = __fadd_rn(v, part[(int64_t(k) * M + m) * rank + j]);
+  }
+  u[i] = v;
 }
 
 // ---------------------------------------------------------------------------
 // Plan
 // ---------------------------------------------------------------------------
-constexpr int kDnMaxSplits = 4;
 constexpr size_t kPad = 256;
 size_t up(size_t b) { return (b + kPad - 1) / kPad * kPad; }
+int el_size(int dt) { return dt == RQ_DTYPE_F32 ? 4 : 2; }
+int64_t step_len(int dt) { return 128 / el_size(dt); }
 
 struct DensePlan {
   int halves, tiles_m, tiles_n, whole, splits;
-  int64_t Rp, r16;
+  int64_t Rp, rankp;
   bool pad;  // the reduction length is padded: activations and factors copied
-  LoraRowsPlan lr;
-  size_t w, cnt, b16, u16, lpart, x, xl, s16, part, bytes;
+  LoraRowsPlan lr;          // 16-bit
+  int u_splits, u_steps;    // fp32: K splits of u and their k steps
+  size_t w, cnt, b, u, lpart, x, xl, s, part, bytes;
 };
 
 // Microseconds of a tiling, from measurements with all 256 compute units busy:
@@ -248,14 +340,16 @@ struct DensePlan {
 // (N(0, 1) operands; power bound), K splits adding 20 and 8 us for their
 // partial tiles (2048 x 4096 x 4096: 128 tiles of 256 in two splits 77 us,
 // 512 tiles of 128 unsplit 69 us; 1024 x 4096 x 4096: 55.6 and 35.5 us;
-// 4096 x 4096 x 14336: 347 and 429 us).
-double pick_tiles(DensePlan& p, int64_t M, int64_t C, int nk, int cus) {
+// 4096 x 4096 x 14336: 347 and 429 us).  fp32: 128 x 128 tiles, 2 us per 32-k
+// step, up to 8 splits (fp32 MFMA bound).
+double pick_tiles(DensePlan& p, int xt, int64_t M, int64_t C, int nk, int cus) {
+  const bool f32 = xt == RQ_DTYPE_F32;
   double best = 1e300;
-  for (int h = 2; h >= 1; --h) {
+  for (int h = f32 ? 1 : 2; h >= 1; --h) {
     const int64_t B = 128 * h, tm = ceil_div(M, B), tn = ceil_div(C, B), T = tm * tn;
-    const double step = h == 2 ? 1.5 : 0.55, extra = h == 2 ? 20.0 : 8.0;
+    const double step = f32 ? 2.0 : (h == 2 ? 1.5 : 0.55), extra = h == 2 ? 20.0 : 8.0;
     const int64_t lt = T % cus, lf = T - lt;
-    for (int s = 1; s <= kDnMaxSplits; s *= 2) {
+    for (int s = 1; s <= (f32 ? 8 : 4); s *= 2) {
       if (s > 1 && (lt == 0 || lt * s > cus || nk / s < 4)) break;
       const double t = step * (double(lf / cus) * nk + (lt ? double(ceil_div(nk, s)) : 0.0)) + (s > 1 ? extra : 0.0);
       if (t < best) {
@@ -271,35 +365,46 @@ double pick_tiles(DensePlan& p, int64_t M, int64_t C, int nk, int cus) {
   return best;
 }
 
-DensePlan plan_dense(int64_t M, int64_t C, int64_t R, int64_t rank, int cus) {
+DensePlan plan_dense(int xt, int64_t M, int64_t C, int64_t R, int64_t rank, int cus) {
   DensePlan p{};
-  p.Rp = (R + 63) / 64 * 64;
+  const int64_t sl = step_len(xt), rp = xt == RQ_DTYPE_F32 ? 8 : 16;
+  const size_t es = size_t(el_size(xt));
+  p.Rp = ceil_div(R, sl) * sl;
   p.pad = p.Rp != R;
-  p.r16 = rank > 0 ? (rank + 15) / 16 * 16 : 0;
-  pick_tiles(p, M, C, int(p.Rp / 64), cus);
+  p.rankp = rank > 0 ? ceil_div(rank, rp) * rp : 0;
+  pick_tiles(p, xt, M, C, int(p.Rp / sl), cus);
   size_t off = 0;
   auto take = [&](size_t b) {
     const size_t o = off;
     off += up(b);
     return o;
   };
-  p.w = take(size_t(C) * p.Rp * 2);
-  p.cnt = take(size_t(p.tiles_m) * p.tiles_n - p.whole ? (size_t(p.tiles_m) * p.tiles_n - p.whole) * 4 : 4);
+  const size_t lt = size_t(p.tiles_m) * p.tiles_n - p.whole;
+  p.w = take(size_t(C) * p.Rp * es);
+  p.cnt = take(lt * 4 + 4);
   if (rank > 0) {
-    p.lr = plan_lora_rows(M, p.Rp, rank, cus);
-    p.b16 = take(size_t(C) * p.r16 * 2);
-    p.u16 = take(size_t(M) * p.r16 * 2);
-    p.lpart = take(p.lr.part_bytes);
-  }
-  if (p.pad) {
-    p.x = take(size_t(M) * p.Rp * 2);
-    if (rank > 0) {
-      p.xl = take(size_t(M) * p.Rp * 2);
-      p.s16 = take(size_t(rank) * p.Rp * 2);
+    p.b = take(size_t(C) * p.rankp * es);
+    p.u = take(size_t(M) * p.rankp * es);
+    if (xt == RQ_DTYPE_F32) {
+      // about two workgroups per compute unit, at least two steps each
+      const int64_t steps = p.Rp / sl, wgs = ceil_div(M, 64) * ceil_div(rank, 64);
+      int64_t ks = std::min(std::max<int64_t>(2 * cus / wgs, 1), std::max<int64_t>(steps / 2, 1));
+      ks = std::min<int64_t>(ks, 64);
+      p.u_steps = int(ceil_div(steps, ks));
+      p.u_splits = int(ceil_div(steps, p.u_steps));
+      p.lpart = take(size_t(p.u_splits) * M * rank * 4);
+    } else {
+      p.lr = plan_lora_rows(M, p.Rp, rank, cus);
+      p.lpart = take(p.lr.part_bytes);
     }
   }
+  if (p.pad) {
+    p.x = take(size_t(M) * p.Rp * es);
+    if (rank > 0) p.xl = take(size_t(M) * p.Rp * es);
+  }
+  if (rank > 0 && (p.pad || xt == RQ_DTYPE_F32)) p.s = take(size_t(rank) * p.Rp * es);
   if (p.splits > 1) {
-    const size_t B = 128 * p.halves, lt = size_t(p.tiles_m) * p.tiles_n - p.whole;
+    const size_t B = 128 * p.halves;
     p.part = take(size_t(p.splits) * lt * B * B * 4);
   }
   p.bytes = off;
@@ -319,7 +424,7 @@ struct Product {
   const void* s;
   int64_t s_j, s_r;
   bool prescale;
-  float pre;
+  float pre = 1.0f;
   const void* f;
   int64_t f_c, f_j;
   int lora_dt;
@@ -327,26 +432,29 @@ struct Product {
 };
 
 template <int XT, class Src, class Scale>
-int launch_decode(Src src, Scale scale, int64_t N, int64_t K, int64_t bs, bool trans, int64_t Rp, uint16_t* out,
+int launch_decode(Src src, Scale scale, int64_t N, int64_t K, int64_t bs, bool trans, int64_t Rp, void* w,
                   hipStream_t stream) {
+  uint8_t* const out = static_cast<uint8_t*>(w);
   const BlockOf blk{bs, bs > 0 ? pow2_shift(bs) : -1};
   const bool blocks_ok = bs == 0 || (blk.log2 >= 5 && K % bs == 0);
   const int64_t chunks = N * (K / 8);
   if (!trans && K % 64 == 0 && blocks_ok && aligned(src.p, 8) && chunks < int64_t(UINT32_MAX) - 4096) {
     decode_rows_kernel<XT, Src, Scale><<<unsigned(ceil_div(chunks, 4 * kDecThreads)), kDecThreads, 0, stream>>>(
-        src, scale, blk, uint32_t(chunks), uint32_t(K / 8), reinterpret_cast<u32x4*>(out));
+        src, scale, blk, uint32_t(chunks), uint32_t(K / 8), out);
   } else if (trans && K % 64 == 0 && N % 64 == 0 && blocks_ok && aligned(src.p, 16) && N / 64 <= 65535) {
     decode_cols_kernel<XT, Src, Scale>
         <<<dim3(unsigned(ceil_div(K, 256)), unsigned(N / 64)), kDecThreads, 0, stream>>>(src, scale, blk, K, Rp, out);
   } else {
     // tiles over the output: its padded reduction index and its rows
-    const int64_t tk = trans ? ceil_div(K, 64) : Rp / 64, tn = trans ? Rp / 64 : ceil_div(N, 64);
+    const int64_t tk = ceil_div(trans ? K : Rp, 64), tn = ceil_div(trans ? Rp : N, 64);
     if (tn > 65535) return RQ_ERR_UNSUPPORTED;
     const dim3 grid{unsigned(tk), unsigned(tn)};
     if (trans)
-      decode_any_kernel<XT, Src, Scale, true><<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, K, Rp, out);
+      decode_any_kernel<XT, Src, Scale, true>
+          <<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, K, Rp, static_cast<Word<XT>*>(w));
     else
-      decode_any_kernel<XT, Src, Scale, false><<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, N, Rp, out);
+      decode_any_kernel<XT, Src, Scale, false>
+          <<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, N, Rp, static_cast<Word<XT>*>(w));
   }
   return rq_check_launch();
 }
@@ -354,20 +462,20 @@ int launch_decode(Src src, Scale scale, int64_t N, int64_t K, int64_t bs, bool t
 // The launches of a product whose weight `decode` writes into w16.
 template <int XT, class Decode>
 int run_product(const Product& P, const Decode& decode, void* scratch, size_t bytes, hipStream_t stream) {
-  const DensePlan p = plan_dense(P.M, P.C, P.R, P.rank, device_cus());
+  constexpr bool kF32 = XT == RQ_DTYPE_F32;
+  const DensePlan p = plan_dense(XT, P.M, P.C, P.R, P.rank, device_cus());
   if (!scratch || bytes < p.bytes) return RQ_ERR_WORKSPACE;
   if (!aligned(scratch, 256)) return RQ_ERR_BAD_ALIGNMENT;
   char* ws = static_cast<char*>(scratch);
-  uint16_t* w16 = reinterpret_cast<uint16_t*>(ws + p.w);
   uint32_t* cnt = reinterpret_cast<uint32_t*>(ws + p.cnt);
-  int st = decode(w16, p.Rp);
+  int st = decode(static_cast<void*>(ws + p.w), p.Rp);
   if (st != RQ_OK) return st;
 
   DenseEpi e = P.e;
   DenseGemmArgs a{};
-  a.x = static_cast<const uint16_t*>(P.x);
+  a.x = P.x;
   a.ldx = P.ldx;
-  const uint16_t* xl = static_cast<const uint16_t*>(P.xl);
+  const void* xl = P.xl;
   int64_t ldxl = P.ldxl;
   const void* s = P.s;
   int64_t s_j = P.s_j, s_r = P.s_r;
@@ -376,16 +484,15 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
   PadCopies pc{};
   int64_t groups = 0;
   auto copy = [&](const void* in, int dt, int64_t sr, int64_t sc, int64_t rows, int64_t cols, int64_t out_rows,
-                  int64_t out_cols, size_t off) {
-    PadCopy& c = pc.c[pc.n++];
-    c = PadCopy{in, dt, sr, sc, rows, cols, out_rows, out_cols, reinterpret_cast<uint16_t*>(ws + off), groups};
+                  int64_t out_cols, size_t off) -> const void* {
+    pc.c[pc.n++] = PadCopy{in, dt, sr, sc, rows, cols, out_rows, out_cols, ws + off, groups};
     groups += ceil_div(out_rows * (out_cols / 8), kDecThreads);
-    return reinterpret_cast<uint16_t*>(ws + off);
+    return ws + off;
   };
   if (P.rank > 0) {
-    e.rank16 = int(p.r16);
-    e.u = reinterpret_cast<uint16_t*>(ws + p.u16);
-    e.b = copy(P.f, P.lora_dt, P.f_c, P.f_j, P.C, P.rank, P.C, p.r16, p.b16);
+    e.rankp = int(p.rankp);
+    e.u = ws + p.u;
+    e.b = copy(P.f, P.lora_dt, P.f_c, P.f_j, P.C, P.rank, P.C, p.rankp, p.b);
   }
   if (p.pad) {
     const bool same = P.xl == P.x && P.ldxl == P.ldx;
@@ -394,11 +501,13 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
     if (P.rank > 0) {
       xl = same ? a.x : copy(P.xl, XT, P.ldxl, 1, P.M, P.R, P.M, p.Rp, p.xl);
       ldxl = p.Rp;
-      s = copy(P.s, P.lora_dt, P.s_j, P.s_r, P.rank, P.R, P.rank, p.Rp, p.s16);
-      s_j = p.Rp;
-      s_r = 1;
-      s_dt = XT;
     }
+  }
+  if (P.rank > 0 && (p.pad || kF32)) {
+    s = copy(P.s, P.lora_dt, P.s_j, P.s_r, P.rank, P.R, P.rank, p.Rp, p.s);
+    s_j = p.Rp;
+    s_r = 1;
+    s_dt = XT;
   }
   if (p.splits > 1) {
     pc.cnt = cnt;
@@ -410,16 +519,31 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
     if ((st = rq_check_launch()) != RQ_OK) return st;
   }
   if (P.rank > 0) {
-    st = run_lora_rows(XT, xl, ldxl, P.M, p.Rp, s, s_dt, s_j, s_r, int(P.rank), P.prescale, P.pre, p.lr,
-                       reinterpret_cast<float*>(ws + p.lpart), reinterpret_cast<uint16_t*>(ws + p.u16), int(p.r16),
-                       stream);
+    float* lpart = reinterpret_cast<float*>(ws + p.lpart);
+    if constexpr (kF32) {
+      const int rank = int(P.rank), jb = rank <= 16 ? 1 : (rank <= 32 ? 2 : 4);
+      const dim3 grid(unsigned(ceil_div(P.M, 64)), unsigned(ceil_div(rank, 16 * jb)), unsigned(p.u_splits));
+      auto launch = [&](auto kernel) {
+        kernel<<<grid, 256, 0, stream>>>(static_cast<const float*>(xl), ldxl, P.M, static_cast<const float*>(s), s_j,
+                                         rank, P.pre, int(p.Rp / 32), p.u_steps, lpart);
+      };
+      if (jb == 1) launch(lora_rows_f32_kernel<1>);
+      else if (jb == 2) launch(lora_rows_f32_kernel<2>);
+      else launch(lora_rows_f32_kernel<4>);
+      lora_sum_f32_kernel<<<unsigned(ceil_div(P.M * p.rankp, 256)), 256, 0, stream>>>(
+          lpart, p.u_splits, P.M, rank, int(p.rankp), reinterpret_cast<float*>(ws + p.u));
+      st = rq_check_launch();
+    } else {
+      st = run_lora_rows(XT, static_cast<const uint16_t*>(xl), ldxl, P.M, p.Rp, s, s_dt, s_j, s_r, int(P.rank),
+                         P.prescale, P.pre, p.lr, lpart, reinterpret_cast<uint16_t*>(ws + p.u), int(p.rankp), stream);
+    }
     if (st != RQ_OK) return st;
   }
-  a.w = w16;
+  a.w = ws + p.w;
   a.ldw = p.Rp;
   a.M = P.M;
   a.N = P.C;
-  a.nk = int(p.Rp / 64);
+  a.nk = int(p.Rp / step_len(XT));
   a.tiles_m = p.tiles_m;
   a.tiles_n = p.tiles_n;
   a.whole = p.whole;
@@ -428,8 +552,12 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
   a.tile_cnt = cnt;
   const int64_t T = int64_t(p.tiles_m) * p.tiles_n;
   const unsigned grid = unsigned(p.whole + (T - p.whole) * p.splits);
-  if (p.halves == 2) dense_gemm_kernel<XT, 2><<<grid, kDnThreads, 0, stream>>>(a, e);
-  else dense_gemm_kernel<XT, 1><<<grid, kDnThreads, 0, stream>>>(a, e);
+  if constexpr (kF32) {
+    dense_gemm_kernel<XT, 1><<<grid, kDnThreads, 0, stream>>>(a, e);
+  } else {
+    if (p.halves == 2) dense_gemm_kernel<XT, 2><<<grid, kDnThreads, 0, stream>>>(a, e);
+    else dense_gemm_kernel<XT, 1><<<grid, kDnThreads, 0, stream>>>(a, e);
+  }
   return rq_check_launch();
 }
 
@@ -456,28 +584,40 @@ int run_weight(const Product& P, const Src& src, const WithScale& with_scale, in
                bool trans, void* scratch, size_t bytes, hipStream_t stream) {
   return run_product<XT>(
       P,
-      [&](uint16_t* w16, int64_t Rp) {
-        return with_scale([&](auto sc) { return launch_decode<XT>(src, sc, N, K, bs, trans, Rp, w16, stream); });
+      [&](void* w, int64_t Rp) {
+        return with_scale([&](auto sc) { return launch_decode<XT>(src, sc, N, K, bs, trans, Rp, w, stream); });
       },
       scratch, bytes, stream);
 }
 
-bool x16(int dt) { return dt == RQ_DTYPE_BF16 || dt == RQ_DTYPE_F16; }
+// run_weight for the activation dtype
+template <class Src, class WithScale>
+int run_any(const Product& P, const Src& src, const WithScale& ws, int64_t N, int64_t K, int64_t bs, bool trans,
+            void* scratch, size_t bytes, hipStream_t stream) {
+  switch (P.xt) {
+    case RQ_DTYPE_F32: return run_weight<RQ_DTYPE_F32>(P, src, ws, N, K, bs, trans, scratch, bytes, stream);
+    case RQ_DTYPE_BF16: return run_weight<RQ_DTYPE_BF16>(P, src, ws, N, K, bs, trans, scratch, bytes, stream);
+    default: return run_weight<RQ_DTYPE_F16>(P, src, ws, N, K, bs, trans, scratch, bytes, stream);
+  }
+}
 
 // 16-byte activation loads when the reduction is not copied into padded rows
-bool act_ok(const void* x, int64_t ldx, int64_t M, int64_t R) {
-  return R % 64 != 0 || (aligned(x, 16) && ldx % 8 == 0 && double(M) * double(ldx) * 2.0 < 4294967296.0);
+bool act_ok(int dt, const void* x, int64_t ldx, int64_t M, int64_t R) {
+  const int64_t es = el_size(dt);
+  return R % step_len(dt) != 0 ||
+         (aligned(x, 16) && ldx * es % 16 == 0 && double(M) * double(ldx) * double(es) < 4294967296.0);
 }
 
 }  // namespace
 
 size_t dense_scratch_bytes(int x_dtype, int64_t M, int64_t C, int64_t R, int64_t rank) {
-  const int64_t Rp = (R + 63) / 64 * 64;
-  if (!x16(x_dtype) || M < 1 || rank < 0 || rank > 256) return 0;
+  const int64_t Rp = ceil_div(R, step_len(x_dtype)) * step_len(x_dtype);
+  if (M < 1 || rank < 0 || rank > 256) return 0;
   // 32-bit byte offsets into both operands, tile counts in an int
-  if (double(C) * double(Rp) * 2.0 >= 4294967296.0 || double(M) * double(Rp) * 2.0 >= 4294967296.0) return 0;
+  const double es = el_size(x_dtype);
+  if (double(C) * double(Rp) * es >= 4294967296.0 || double(M) * double(Rp) * es >= 4294967296.0) return 0;
   if (ceil_div(M, 128) * ceil_div(C, 128) > int64_t(1) << 28) return 0;
-  return plan_dense(M, C, R, rank > 0 ? rank : 0, device_cus()).bytes;
+  return plan_dense(x_dtype, M, C, R, rank > 0 ? rank : 0, device_cus()).bytes;
 }
 
 // Estimates in microseconds from measurements on the Llama-3-8B shapes (M = 64
@@ -496,32 +636,42 @@ bool dense_beats_fused(int64_t M, int64_t C, int64_t R, bool splits) {
   const double waves = f.splits > 1 ? double(f.lf * 8 / cus) + 1.0 / f.splits : double(ceil_div(T, cus));
   const double fused = nk * step * waves + (f.splits > 1 ? 12.0 : 0.0);
   DensePlan p{};
-  const double dense = pick_tiles(p, M, C, int((R + 63) / 64), cus);
+  const double dense = pick_tiles(p, RQ_DTYPE_BF16, M, C, int((R + 63) / 64), cus);
   return dense + 6.0 + 0.5e-6 * double(C) * double(R) < fused;
 }
 
-bool dense_nf4_linear_ok(const LinearArgs& L) {
-  return act_ok(L.x, L.ldx, L.M, L.K) && (L.rank == 0 || act_ok(L.lora_x, L.ld_lora_x, L.M, L.K));
+// fp32 forward against the GEMV kernels over blocks of 16 rows, about 1.2 us per
+// million weights and block (4096 x 4096: 20 us a block with the LoRA operand):
+// decoding takes 1 us per million weights and its launches 10 us.
+bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R) {
+  if (M <= kGemvMaxM) return false;
+  DensePlan p{};
+  const double mw = 1e-6 * double(C) * double(R);
+  return pick_tiles(p, RQ_DTYPE_F32, M, C, int(ceil_div(R, 32)), device_cus()) + 10.0 + 1.0 * mw <
+         1.2 * mw * double(ceil_div(M, 16));
 }
-bool dense_nf4_dx_ok(const DxArgs& D) { return act_ok(D.dy, D.lddy, D.M, D.N); }
-bool dense_int8_ok(const GenericInt8& A, bool dx) { return act_ok(A.x, A.ldx, A.M, dx ? A.N : A.K); }
+
+bool dense_nf4_linear_ok(const LinearArgs& L) {
+  return act_ok(L.x_dtype, L.x, L.ldx, L.M, L.K) &&
+         (L.rank == 0 || act_ok(L.x_dtype, L.lora_x, L.ld_lora_x, L.M, L.K));
+}
+bool dense_nf4_dx_ok(const DxArgs& D) { return act_ok(D.dy_dtype, D.dy, D.lddy, D.M, D.N); }
+bool dense_int8_ok(const GenericInt8& A, bool dx) { return act_ok(A.x_dtype, A.x, A.ldx, A.M, dx ? A.N : A.K); }
 
 int run_dense_nf4_linear(const LinearArgs& L, void* scratch, size_t bytes, hipStream_t stream) {
   Product P{};
   P.xt = L.x_dtype; P.x = L.x; P.ldx = L.ldx; P.M = L.M; P.C = L.N; P.R = L.K;
   if (L.rank > 0) {
     P.rank = L.rank; P.xl = L.lora_x; P.ldxl = L.ld_lora_x;
-    P.s = L.lora_a; P.s_j = L.K; P.s_r = 1; P.pre = 1.0f;
+    P.s = L.lora_a; P.s_j = L.K; P.s_r = 1;
     P.f = L.lora_b; P.f_c = L.ld_lora_b; P.f_j = 1;
     P.lora_dt = L.lora_dtype;
   }
   P.e.bias = L.bias; P.e.bias_dt = L.bias_dtype; P.e.scaling = L.scaling;
-  P.e.y = static_cast<uint16_t*>(L.y); P.e.ldy = L.ldy;
+  P.e.y = L.y; P.e.ldy = L.ldy;
   auto ws = [&](auto fn) { return with_nf4_scale(L.absmax, L.absmax_dtype, L.c2, L.c2_format, L.block2, fn); };
   const SrcNF4 src{L.w_packed};
-  return L.x_dtype == RQ_DTYPE_BF16
-             ? run_weight<RQ_DTYPE_BF16>(P, src, ws, L.N, L.K, L.block_size, false, scratch, bytes, stream)
-             : run_weight<RQ_DTYPE_F16>(P, src, ws, L.N, L.K, L.block_size, false, scratch, bytes, stream);
+  return run_any(P, src, ws, L.N, L.K, L.block_size, false, scratch, bytes, stream);
 }
 
 int run_dense_nf4_dx(const DxArgs& D, void* scratch, size_t bytes, hipStream_t stream) {
@@ -536,26 +686,22 @@ int run_dense_nf4_dx(const DxArgs& D, void* scratch, size_t bytes, hipStream_t s
     P.e.mask = D.lora_mask; P.e.ldm = D.ld_lora_mask; P.e.mask_scale = D.mask_scale;
   }
   P.e.scaling = 1.0f;
-  P.e.y = static_cast<uint16_t*>(D.dx); P.e.ldy = D.lddx;
+  P.e.y = D.dx; P.e.ldy = D.lddx;
   auto ws = [&](auto fn) { return with_nf4_scale(D.absmax, D.absmax_dtype, D.c2, D.c2_format, D.block2, fn); };
   const SrcNF4 src{D.w_packed};
-  return D.dy_dtype == RQ_DTYPE_BF16
-             ? run_weight<RQ_DTYPE_BF16>(P, src, ws, D.N, D.K, D.block_size, true, scratch, bytes, stream)
-             : run_weight<RQ_DTYPE_F16>(P, src, ws, D.N, D.K, D.block_size, true, scratch, bytes, stream);
+  return run_any(P, src, ws, D.N, D.K, D.block_size, true, scratch, bytes, stream);
 }
 
 int run_dense_int8(const GenericInt8& A, bool dx, void* scratch, size_t bytes, hipStream_t stream) {
   Product P{};
   P.xt = A.x_dtype; P.x = A.x; P.ldx = A.ldx; P.M = A.M; P.C = dx ? A.K : A.N; P.R = dx ? A.N : A.K;
   P.e.bias = dx ? nullptr : A.bias; P.e.bias_dt = A.bias_dtype; P.e.scaling = 1.0f;
-  P.e.y = static_cast<uint16_t*>(A.y); P.e.ldy = A.ldy;
+  P.e.y = A.y; P.e.ldy = A.ldy;
   auto ws = [&](auto fn) {
     return with_nf4_scale(A.scales, A.scales_dtype, nullptr, 0, 1, fn);
   };
   const SrcInt8 src{reinterpret_cast<const uint8_t*>(A.q)};
-  return A.x_dtype == RQ_DTYPE_BF16
-             ? run_weight<RQ_DTYPE_BF16>(P, src, ws, A.N, A.K, A.block_size, dx, scratch, bytes, stream)
-             : run_weight<RQ_DTYPE_F16>(P, src, ws, A.N, A.K, A.block_size, dx, scratch, bytes, stream);
+  return run_any(P, src, ws, A.N, A.K, A.block_size, dx, scratch, bytes, stream);
 }
 
 }  // namespace rq

@@ -1648,8 +1648,11 @@ extern "C" int rq_nf4_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int
   if (!bytes) return RQ_ERR_NULL_POINTER;
   if (!valid_float_dtype(x_dtype)) return RQ_ERR_BAD_DTYPE;
   if (M < 0 || N < 1 || K < 1 || block_size < 1 || rank < 0 || rank > 256) return RQ_ERR_BAD_SHAPE;
-  const bool fast = K % 64 == 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0;
-  *bytes = fast && !dense_beats_fused(M, N, K, true) ? 0 : int64_t(dense_scratch_bytes(x_dtype, M, N, K, rank));
+  const bool f32 = x_dtype == RQ_DTYPE_F32;
+  const bool fast = K % 64 == 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0 &&
+                    (!f32 || rank <= 64);
+  const bool faster = !fast || (f32 ? dense_beats_f32_blocks(M, N, K) : dense_beats_fused(M, N, K, true));
+  *bytes = faster ? int64_t(dense_scratch_bytes(x_dtype, M, N, K, rank)) : 0;
   return RQ_OK;
 }
 

@@ -1,7 +1,7 @@
 // Host interface of the dequantize-once linears (dense_gemm.hip): the weight
 // is decoded into scratch memory by one launch and multiplied by the dense
 // MFMA GEMM (rq_dense_gemm.h).  For NF4 and INT8 weights, forward and dX,
-// 16-bit activations, any sizes, block sizes and alignments.
+// any activation dtype, sizes, block sizes and alignments.
 #pragma once
 
 #include <stddef.h>
@@ -21,6 +21,9 @@ size_t dense_scratch_bytes(int x_dtype, int64_t M, int64_t C, int64_t R, int64_t
 // Whether the dense path is the faster one for a call the fused GEMM takes
 // (splits: that call's GEMM splits K for the last wave's tiles).
 bool dense_beats_fused(int64_t M, int64_t C, int64_t R, bool splits);
+
+// The same for fp32 activations and the row-block GEMV kernels (forward).
+bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R);
 
 // Whether the operands' alignment suits the dense path (any, once the
 // reduction is padded; else activation rows of 16-byte chunks).

@@ -1,7 +1,9 @@
-// Dense 16-bit MFMA GEMM for gfx950: out[M, N] = X[M, K] . W[N, K]^T with the
+// Dense MFMA GEMM for gfx950: out[M, N] = X[M, K] . W[N, K]^T with the
 // quantized linears' epilogue (bias, LoRA term, the reference's roundings),
-// where W is the 16-bit weight RND(W_deq) that a launch before it wrote into
-// scratch memory (dense_gemm.hip), as W rows (forward) or W^T rows (dX).
+// where W is the weight RND(W_deq) that a launch before it wrote into scratch
+// memory (dense_gemm.hip), as W rows (forward) or W^T rows (dX).  bf16 and
+// fp16 (v_mfma_f32_32x32x16), and fp32 (v_mfma_f32_32x32x2_f32, 128 x 128
+// tiles only, everything in fp32).
 //
 // Tile 256 x 256 (HALVES = 2) or 128 x 128 (HALVES = 1), 64 k per step,
 // eight waves, two per SIMD: wave (wr, wc) = (wave / 4, wave % 4) owns rows
@@ -30,24 +32,33 @@ namespace rq {
 constexpr int kDnThreads = 512;
 constexpr int kDnHalf = 128 * 128;  // bytes of a half tile: 128 rows x 64 k
 
+// Element bytes of an operand type, and the elements of one k step (128-byte
+// rows).
+template <int XT>
+struct DnEl {
+  static constexpr int kSize = XT == RQ_DTYPE_F32 ? 4 : 2;
+  static constexpr int kStep = 128 / kSize;
+  static constexpr int kRankPad = XT == RQ_DTYPE_F32 ? 8 : 16;  // one LoRA epilogue step
+};
+
 // LDS: two buffers of X0 X1 W0 W1 (256 x 256 tiles), or four of X W (128 x
 // 128); the epilogue stages the output tile in it (16-byte padded rows).
-template <int HALVES>
+template <int XT, int HALVES>
 struct DnTile {
   static constexpr int kB = 128 * HALVES;           // tile rows and columns
   static constexpr int kBuf = 2 * HALVES * kDnHalf;  // one k step
   static constexpr int kBufs = 4 / HALVES;
-  static constexpr int kOutPitch = kB * 2 + 16;
+  static constexpr int kOutPitch = kB * DnEl<XT>::kSize + 16;
   static constexpr int kLds = kB * kOutPitch > kBufs * kBuf ? kB * kOutPitch : kBufs * kBuf;
   static_assert(kLds <= 160 * 1024, "LDS plan");
 };
 
 struct DenseGemmArgs {
-  const uint16_t* x;  // [M][ldx]
-  const uint16_t* w;  // [N][ldw]
+  const void* x;  // [M][ldx]
+  const void* w;  // [N][ldw]
   int64_t ldx, ldw;
   int64_t M, N;
-  int nk;             // k steps of 64 (the operands are zero past K)
+  int nk;             // k steps of 128 bytes (the operands are zero past K)
   int tiles_m, tiles_n;
   int whole;          // tiles run whole; the other tiles - whole run as `splits` workgroups
   int splits;
@@ -58,21 +69,42 @@ struct DenseGemmArgs {
 struct DenseEpi {
   const void* bias;
   int bias_dt;
-  int rank16;          // LoRA rank rounded up to 16 (0: none)
-  const uint16_t* u;   // [M][rank16]
-  const uint16_t* b;   // [N][rank16]
+  int rankp;           // LoRA rank rounded up to kRankPad (0: none)
+  const void* u;       // [M][rankp]
+  const void* b;       // [N][rankp]
   float scaling;
   const uint8_t* mask;  // dX with LoRA dropout
   int64_t ldm;
   float mask_scale;
-  uint16_t* y;
+  void* y;
   int64_t ldy;
 };
+
+// RND: rounding to the result type (none for fp32)
+template <int XT>
+__device__ __forceinline__ void dn_round2(float& x, float& y) {
+  if constexpr (XT != RQ_DTYPE_F32) round2<XT>(x, y);
+}
+
+// The products of one 16-byte operand chunk pair per lane: 8 16-bit values (one
+// MFMA), or 4 fp32 values (four 32x32x2 MFMAs; lanes 0-31 and 32-63 hold
+// different k in both operands alike, so any order of k serves).
+template <int XT>
+__device__ __forceinline__ f32x16 dn_mfma(const u32x4& w, const u32x4& x, f32x16 c) {
+  if constexpr (XT == RQ_DTYPE_F32) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(w[j]), u2f(x[j]), c, 0, 0, 0);
+    return c;
+  } else {
+    return mfma32x32x16<XT>(w, x, c);
+  }
+}
 
 template <int XT, int HALVES>
 __global__ __launch_bounds__(kDnThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void dense_gemm_kernel(DenseGemmArgs a, DenseEpi e) {
-  using Tile = DnTile<HALVES>;
+  using Tile = DnTile<XT, HALVES>;
+  constexpr int ES = DnEl<XT>::kSize;
   constexpr int H = HALVES, kBuf = Tile::kBuf, kOutPitch = Tile::kOutPitch;
   __shared__ __attribute__((aligned(16))) uint8_t lds[Tile::kLds];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -118,17 +150,17 @@ void dense_gemm_kernel(DenseGemmArgs a, DenseEpi e) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int r = 16 * wave + 8 * i + (lane >> 3);
-      const uint32_t c = uint32_t(8 * ((lane & 7) ^ ((r >> 1) & 7)));
+      const uint32_t c = uint32_t(16 * ((lane & 7) ^ ((r >> 1) & 7)));
       int64_t m = m0 + 128 * h + r, n = n0 + 128 * h + r;
       m = m < a.M ? m : a.M - 1;
       n = n < a.N ? n : a.N - 1;
-      xo[h][i] = uint32_t(m * a.ldx + c) * 2u;
-      wo[h][i] = uint32_t(n * a.ldw + c) * 2u;
+      xo[h][i] = uint32_t(m * a.ldx) * uint32_t(ES) + c;
+      wo[h][i] = uint32_t(n * a.ldw) * uint32_t(ES) + c;
     }
   const uint32_t dst0 = __builtin_amdgcn_readfirstlane(uint32_t(wave) * 2048u);
-  auto load_half = [&](const uint16_t* base, const uint32_t (&off)[2], int step, uint32_t lds_off) {
+  auto load_half = [&](const void* base, const uint32_t (&off)[2], int step, uint32_t lds_off) {
     const int st = step < nk ? step : nk - 1;  // past the end: a live step again, never used
-    const uint8_t* p = reinterpret_cast<const uint8_t*>(base) + int64_t(kbeg + st) * 128;
+    const uint8_t* p = static_cast<const uint8_t*>(base) + int64_t(kbeg + st) * 128;
     dma16(p, off[0], dst0 + lds_off);
     dma16(p, off[1], dst0 + lds_off + 1024u);
   };
@@ -136,7 +168,7 @@ void dense_gemm_kernel(DenseGemmArgs a, DenseEpi e) {
   auto xoff = [](int b, int h) { return uint32_t(b * kBuf + h * kDnHalf); };
   auto woff = [](int b, int h) { return uint32_t(b * kBuf + (H + h) * kDnHalf); };
 
-  // operand read offsets of sub-step s (16 k): chunk 2 s + q of the lane's row
+  // operand read offsets of sub-step s: chunk 2 s + q of the lane's row
   uint32_t xr[4], wrd[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
@@ -167,9 +199,18 @@ void dense_gemm_kernel(DenseGemmArgs a, DenseEpi e) {
   auto mma = [&](f32x16 (&c)[2], const u32x4 (&wv)[4]) {
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < 4; ++s) {
+      if constexpr (XT == RQ_DTYPE_F32) {  // the two blocks in turn: no MFMA waits for the one before it
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb) c[mb] = mfma32x32x16<XT>(wv[s], xa[mb][s], c[mb]);
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int mb = 0; mb < 2; ++mb)
+            c[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(u2f(wv[s][j]), u2f(xa[mb][s][j]), c[mb], 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) c[mb] = mfma32x32x16<XT>(wv[s], xa[mb][s], c[mb]);
+      }
+    }
     __builtin_amdgcn_s_setprio(0);
   };
 #define RQ_DN_MEM_END(N)                                                      \
@@ -330,32 +371,35 @@ void dense_gemm_kernel(DenseGemmArgs a, DenseEpi e) {
       for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) lo[mb][r] = 0.0f;
-      if (e.rank16 > 0) {
+      if (e.rankp > 0) {
         int64_t n = nq + i32;
         n = n < a.N ? n : a.N - 1;
-        const uint16_t* bp = e.b + n * e.rank16 + 8 * q;
-        const uint16_t* up[2];
+        const uint8_t* bp = static_cast<const uint8_t*>(e.b) + n * e.rankp * ES + 16 * q;
+        const uint8_t* up[2];
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) {
           int64_t m = mq + 32 * mb + i32;
           m = m < a.M ? m : a.M - 1;
-          up[mb] = e.u + m * e.rank16 + 8 * q;
+          up[mb] = static_cast<const uint8_t*>(e.u) + m * e.rankp * ES + 16 * q;
         }
-        for (int s = 0; s < e.rank16; s += 16) {
+        for (int s = 0; s < e.rankp * ES; s += 32) {
           const u32x4 bv = *reinterpret_cast<const u32x4*>(bp + s);
 #pragma unroll
           for (int mb = 0; mb < 2; ++mb)
-            lo[mb] = mfma32x32x16<XT>(bv, *reinterpret_cast<const u32x4*>(up[mb] + s), lo[mb]);
+            lo[mb] = dn_mfma<XT>(bv, *reinterpret_cast<const u32x4*>(up[mb] + s), lo[mb]);
         }
       }
       float bias[4][4];
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
+      for (int h = 0; h < 4; ++h) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const int64_t n = nq + 8 * h + 4 * q + c;
-          bias[h][c] = e.bias && n < a.N ? round_x<XT>(load_as_f32(e.bias, n, e.bias_dt)) : -0.0f;
+          bias[h][c] = e.bias && n < a.N ? load_as_f32(e.bias, n, e.bias_dt) : -0.0f;
         }
+        dn_round2<XT>(bias[h][0], bias[h][1]);
+        dn_round2<XT>(bias[h][2], bias[h][3]);
+      }
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -363,9 +407,9 @@ void dense_gemm_kernel(DenseGemmArgs a, DenseEpi e) {
           float v[4];
 #pragma unroll
           for (int c = 0; c < 4; ++c) v[c] = __fadd_rn(acc[hm][hn][mb][4 * h + c], bias[h][c]);
-          if (e.rank16 > 0) {
-            round2<XT>(v[0], v[1]);
-            round2<XT>(v[2], v[3]);
+          if (e.rankp > 0) {
+            dn_round2<XT>(v[0], v[1]);
+            dn_round2<XT>(v[2], v[3]);
             float l[4], s[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -378,38 +422,46 @@ void dense_gemm_kernel(DenseGemmArgs a, DenseEpi e) {
               for (int c = 0; c < 4; ++c)
                 s[c] = m < a.M && n + c < a.N && e.mask[m * e.ldm + n + c] ? e.mask_scale : 0.0f;
             }
-            round2<XT>(l[0], l[1]);
-            round2<XT>(l[2], l[3]);
+            dn_round2<XT>(l[0], l[1]);
+            dn_round2<XT>(l[2], l[3]);
 #pragma unroll
             for (int c = 0; c < 4; ++c) l[c] = __fmul_rn(l[c], s[c]);
-            round2<XT>(l[0], l[1]);
-            round2<XT>(l[2], l[3]);
+            dn_round2<XT>(l[0], l[1]);
+            dn_round2<XT>(l[2], l[3]);
 #pragma unroll
             for (int c = 0; c < 4; ++c) v[c] = __fadd_rn(v[c], l[c]);
           }
-          *reinterpret_cast<u32x2*>(lds + (128 * hm + 64 * wr + 32 * mb + i32) * kOutPitch +
-                                    (128 * hn + 32 * wc + 8 * h + 4 * q) * 2) =
-              u32x2{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3])};
+          uint8_t* o = lds + (128 * hm + 64 * wr + 32 * mb + i32) * kOutPitch +
+                       (128 * hn + 32 * wc + 8 * h + 4 * q) * ES;
+          if constexpr (XT == RQ_DTYPE_F32)
+            *reinterpret_cast<u32x4*>(o) = u32x4{f2u(v[0]), f2u(v[1]), f2u(v[2]), f2u(v[3])};
+          else
+            *reinterpret_cast<u32x2*>(o) = u32x2{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3])};
         }
     }
   __syncthreads();
   // 16 H rows per wave, whole rows of the tile per instruction
-  constexpr int kLpr = Tile::kB / 8;  // lanes (16-byte chunks) per row
-  const bool vec = (reinterpret_cast<uintptr_t>(e.y) & 15u) == 0 && (e.ldy & 7) == 0;
-  const int64_t nc = n0 + 8 * (lane & (kLpr - 1));
+  constexpr int kPer = 16 / ES;            // outputs per 16-byte chunk
+  constexpr int kLpr = Tile::kB / kPer;    // lanes per row
+  constexpr int kRows = 64 / kLpr;         // rows per instruction
+  const bool vec = (reinterpret_cast<uintptr_t>(e.y) & 15u) == 0 && e.ldy % kPer == 0;
+  const int64_t nc = n0 + kPer * (lane & (kLpr - 1));
 #pragma unroll 4
-  for (int it = 0; it < Tile::kB / 8 / (64 / kLpr); ++it) {
-    const int r = (Tile::kB / 8) * wave + (64 / kLpr) * it + lane / kLpr;
+  for (int it = 0; it < Tile::kB / 8 / kRows; ++it) {
+    const int r = (Tile::kB / 8) * wave + kRows * it + lane / kLpr;
     const int64_t m = m0 + r;
     if (m >= a.M) continue;
     const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * kOutPitch + 16 * (lane & (kLpr - 1)));
-    uint16_t* yp = e.y + m * e.ldy + nc;
-    if (vec && nc + 8 <= a.N) {
+    uint8_t* yp = static_cast<uint8_t*>(e.y) + (m * e.ldy + nc) * ES;
+    if (vec && nc + kPer <= a.N) {
       *reinterpret_cast<u32x4*>(yp) = v;
     } else {
 #pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (nc + c < a.N) yp[c] = uint16_t(v[c >> 1] >> (16 * (c & 1)));
+      for (int c = 0; c < kPer; ++c) {
+        if (nc + c >= a.N) break;
+        if constexpr (ES == 4) reinterpret_cast<uint32_t*>(yp)[c] = v[c];
+        else reinterpret_cast<uint16_t*>(yp)[c] = uint16_t(v[c >> 1] >> (16 * (c & 1)));
+      }
     }
   }
 }

@@ -139,6 +139,11 @@ def _workspace(x_dtype: torch.dtype, M: int, K: int, N: int, rank: int, dev) -> 
     return ws
 
 
+def _step(dtype: torch.dtype) -> int:
+    """Elements of one 128-byte k step of the dense GEMM's activations."""
+    return 32 if dtype == torch.float32 else 64
+
+
 def _scratch(size_fn: str, dev, *args) -> Optional[torch.Tensor]:
     """Scratch memory for one call, of the size `size_fn` reports (None when
     none is used): from torch's caching allocator, which hands it out again in
@@ -188,9 +193,9 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
         x2, ldx = _rows(x, K)
         M = x2.shape[0]
         # the decode GEMV reads any alignment; every other kernel whose rows are
-        # whole 64-element steps reads activations 16 bytes at a time
+        # whole 128-byte steps reads activations 16 bytes at a time
         fast_shape = K % 64 == 0 and block_size >= 64 and not block_size & (block_size - 1) and K % block_size == 0
-        wide = K % 64 == 0 and (M > GEMV_MAX_M or x.dtype == torch.float32 or not fast_shape)
+        wide = K % _step(x.dtype) == 0 and (M > GEMV_MAX_M or x.dtype == torch.float32 or not fast_shape)
         if wide:
             x2, ldx = _aligned_rows(x2, K)
         y = torch.empty((M, N), dtype=x.dtype, device=dev)
@@ -221,7 +226,7 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
                 xl, ldxl = (_aligned_rows if wide else _rows)(lora_x.to(x.dtype), K)
         b = bias.contiguous() if bias is not None else None
         scratch = None
-        if (M > GEMV_MAX_M or not fast_shape) and max(ldx, ldxl) * M < 1 << 31:
+        if (M > GEMV_MAX_M or not fast_shape) and max(ldx, ldxl) * M * x.element_size() < 1 << 32:
             scratch = _scratch("rq_nf4_linear_scratch_size", dev, xcode, M, K, N, block_size, rank)
         # a call with scratch memory needs no workspace of its own
         ws = _workspace(x.dtype, M, K, N, rank, dev) if scratch is None else None
@@ -265,8 +270,8 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
     scales = scales.reshape(-1).contiguous()
     lead = dy.shape[:-1]
     with on(dev):
-        # the dX kernel loads dY rows 16 bytes at a time
-        dy2, lddy = _aligned_rows(dy, N) if N % 64 == 0 else _rows(dy, N)
+        # the dX kernels load dY rows 16 bytes at a time
+        dy2, lddy = _aligned_rows(dy, N) if N % _step(dy.dtype) == 0 else _rows(dy, N)
         M = dy2.shape[0]
         dx = torch.empty((M, K), dtype=dy.dtype, device=dev)
         if M == 0:
@@ -295,7 +300,7 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
                 raise RuntimeError(f"lora_mask has {mk.shape[0]} rows, dY {M}")
         code = nat.dtype_code(dy.dtype)
         scratch = ws = None
-        if lddy * M < 1 << 31:
+        if lddy * M * dy.element_size() < 1 << 32:
             scratch = _scratch("rq_nf4_linear_dx_scratch_size", dev, code, M, N, K, block_size, rank)
         if scratch is None:
             ws = _scratch("rq_nf4_linear_dx_workspace_size", dev, code, M, N, K, rank)
@@ -343,7 +348,7 @@ def int8_linear(x: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, out_feat
         raise RuntimeError(f"scales hold {sc.numel()} values, need {need}")
     lead = x.shape[:-1]
     with on(dev):
-        x2, ldx = _aligned_rows(x, K) if K % 64 == 0 and x.dtype != torch.float32 else _rows(x, K)
+        x2, ldx = _aligned_rows(x, K) if K % _step(x.dtype) == 0 else _rows(x, K)
         M = x2.shape[0]
         y = torch.empty((M, N), dtype=x.dtype, device=dev)
         if M == 0:
@@ -379,7 +384,7 @@ def int8_linear_dx(dy: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, in_f
         raise RuntimeError(f"scales hold {sc.numel()} values, need {need}")
     lead = dy.shape[:-1]
     with on(dev):
-        dy2, lddy = _aligned_rows(dy, N) if N % 64 == 0 and dy.dtype != torch.float32 else _rows(dy, N)
+        dy2, lddy = _aligned_rows(dy, N) if N % _step(dy.dtype) == 0 else _rows(dy, N)
         M = dy2.shape[0]
         dx = torch.empty((M, K), dtype=dy.dtype, device=dev)
         if M == 0:
