@@ -271,7 +271,9 @@ int rq_nf4_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t
                      float mask_scale, void* dx, int64_t lddx,
                      void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
-/* rq_nf4_linear_dx with optional scratch memory, as rq_nf4_linear_scratch. */
+/* rq_nf4_linear_dx with optional scratch memory, as rq_nf4_linear_scratch, and
+ * optionally (16-bit dY) with the adapter's RND(RND(dY * scaling) . RND(B)) as
+ * rq_lora_grads leaves it: lora_g [M, rank rounded up to 16], or NULL. */
 int rq_nf4_linear_dx_scratch_size(int dy_dtype, int64_t M, int64_t N, int64_t K, int64_t block_size, int64_t rank,
                                   int64_t* bytes);
 int rq_nf4_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy,
@@ -281,8 +283,26 @@ int rq_nf4_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N,
                              const void* lora_a, const void* lora_b, int64_t ld_lora_b, int lora_dtype,
                              int64_t rank, float scaling, const uint8_t* lora_mask, int64_t ld_lora_mask,
                              float mask_scale, void* dx, int64_t lddx,
-                             void* workspace, int64_t workspace_bytes, void* scratch, int64_t scratch_bytes,
+                             const void* lora_g, void* workspace, int64_t workspace_bytes, void* scratch,
+                             int64_t scratch_bytes,
                              hipStream_t stream);
+
+/* Gradients of the LoRA adapters (lora_layer.py:67 differentiated), 16-bit
+ * activations, rank <= 64:
+ *   u = RND(x RND(A)^T), dv = RND(dY * scaling), g = RND(dv RND(B)),
+ *   dB = RND(dv^T u) [N, rank], dA = RND(g^T x) [rank, K]
+ * in lora_dtype (fp32 or x_dtype; the values rounded to x_dtype).  x [M, K]
+ * (the adapter's input) stride ldx, dy [M, N] stride lddy, A [rank, K], B [N,
+ * rank] stride ld_lora_b.  da, db, g ([M, rank rounded up to 16], x_dtype): each
+ * may be NULL.  Rows of x (dy) are read 16 bytes at a time when K (N) is a
+ * multiple of 64.  scratch: 256-byte aligned, rq_lora_grads_scratch_size bytes
+ * (0: not supported here -- fp32 activations, rank > 64). */
+int rq_lora_grads_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t rank, int64_t* bytes);
+int rq_lora_grads(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
+                  const void* dy, int64_t N, int64_t lddy,
+                  const void* lora_a, const void* lora_b, int64_t ld_lora_b, int lora_dtype, int64_t rank,
+                  float scaling, void* da, void* db, void* g, void* scratch, int64_t scratch_bytes,
+                  hipStream_t stream);
 
 /* ------------------------------------------------------------------------
  * INT8 and FP8 linears

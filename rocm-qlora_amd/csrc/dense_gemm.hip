@@ -428,6 +428,7 @@ struct Product {
   const void* f;
   int64_t f_c, f_j;
   int lora_dt;
+  const void* u;  // u itself ([M][rankp]) when the caller has it
   DenseEpi e;
 };
 
@@ -491,19 +492,19 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
   };
   if (P.rank > 0) {
     e.rankp = int(p.rankp);
-    e.u = ws + p.u;
+    e.u = P.u ? P.u : ws + p.u;
     e.b = copy(P.f, P.lora_dt, P.f_c, P.f_j, P.C, P.rank, P.C, p.rankp, p.b);
   }
   if (p.pad) {
     const bool same = P.xl == P.x && P.ldxl == P.ldx;
     a.x = copy(P.x, XT, P.ldx, 1, P.M, P.R, P.M, p.Rp, p.x);
     a.ldx = p.Rp;
-    if (P.rank > 0) {
+    if (P.rank > 0 && !P.u) {
       xl = same ? a.x : copy(P.xl, XT, P.ldxl, 1, P.M, P.R, P.M, p.Rp, p.xl);
       ldxl = p.Rp;
     }
   }
-  if (P.rank > 0 && (p.pad || kF32)) {
+  if (P.rank > 0 && !P.u && (p.pad || kF32)) {
     s = copy(P.s, P.lora_dt, P.s_j, P.s_r, P.rank, P.R, P.rank, p.Rp, p.s);
     s_j = p.Rp;
     s_r = 1;
@@ -518,7 +519,7 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
     pad_copy_kernel<XT><<<unsigned(std::max<int64_t>(groups, 1)), kDecThreads, 0, stream>>>(pc);
     if ((st = rq_check_launch()) != RQ_OK) return st;
   }
-  if (P.rank > 0) {
+  if (P.rank > 0 && !P.u) {
     float* lpart = reinterpret_cast<float*>(ws + p.lpart);
     if constexpr (kF32) {
       const int rank = int(P.rank), jb = rank <= 16 ? 1 : (rank <= 32 ? 2 : 4);
@@ -683,6 +684,7 @@ int run_dense_nf4_dx(const DxArgs& D, void* scratch, size_t bytes, hipStream_t s
     P.s = D.lora_b; P.s_j = 1; P.s_r = D.ld_lora_b; P.prescale = true; P.pre = D.scaling;
     P.f = D.lora_a; P.f_c = 1; P.f_j = D.K;
     P.lora_dt = D.lora_dtype;
+    P.u = D.lora_g;
     P.e.mask = D.lora_mask; P.e.ldm = D.ld_lora_mask; P.e.mask_scale = D.mask_scale;
   }
   P.e.scaling = 1.0f;

@@ -378,13 +378,13 @@ int gen_nf4_dx(const DxArgs& D, Scale sc, void* v, hipStream_t stream) {
     GenEpi ev{};
     ev.y = v;
     ev.ldy = rank;
-    const int st = launch_generic<XT, false, true, kEpiRound>(XPlain<XT>{D.dy, D.lddy, D.scaling, true},
+    const int st = D.lora_g ? RQ_OK : launch_generic<XT, false, true, kEpiRound>(XPlain<XT>{D.dy, D.lddy, D.scaling, true},
                                                               WDense{D.lora_b, D.lora_dtype, D.ld_lora_b, 1}, D.M,
                                                               rank, D.N, ev, stream);
     if (st != RQ_OK) return st;
     e.rank = int(rank);
-    e.u = v;
-    e.ldu = rank;
+    e.u = D.lora_g ? D.lora_g : v;
+    e.ldu = D.lora_g ? (rank + 15) / 16 * 16 : rank;
     e.lf = WDense{D.lora_a, D.lora_dtype, 1, D.K};  // RND(A)[j, k] as element (k, j)
     e.mask = D.lora_mask;
     e.ldm = D.ld_lora_mask;

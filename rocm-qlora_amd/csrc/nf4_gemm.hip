@@ -438,13 +438,15 @@ int run_nf4_dx(const DxArgs& D, void* workspace, size_t ws_bytes, hipStream_t st
     char* ws = static_cast<char*>(workspace);
     uint16_t* g16 = reinterpret_cast<uint16_t*>(ws + p.u16_offset);
     // g = RND(RND(dY * s) . RND(B)): S[j][n] = B[n][j]
-    st = run_lora_rows(D.dy_dtype, static_cast<const uint16_t*>(D.dy), D.lddy, D.M, D.N, D.lora_b, D.lora_dtype, 1,
-                       D.ld_lora_b, int(rank), true, D.scaling, p.lr, reinterpret_cast<float*>(ws), g16, p.rank16,
-                       stream);
-    if (st != RQ_OK) return st;
+    if (!D.lora_g) {
+      st = run_lora_rows(D.dy_dtype, static_cast<const uint16_t*>(D.dy), D.lddy, D.M, D.N, D.lora_b, D.lora_dtype, 1,
+                         D.ld_lora_b, int(rank), true, D.scaling, p.lr, reinterpret_cast<float*>(ws), g16, p.rank16,
+                         stream);
+      if (st != RQ_OK) return st;
+    }
     // RND(A^T) [K][r]: element (k, j) = A[j][k], A [r][K] row-major, rounded
     // as the epilogue stages it
-    e.u = g16;
+    e.u = D.lora_g ? static_cast<const uint16_t*>(D.lora_g) : g16;
     e.braw = D.lora_a;
     e.b_dt = D.lora_dtype;
     e.b_sn = 1;
@@ -514,6 +516,7 @@ static rq::DxArgs pack_dx_args(const void* dy, int dy_dtype, int64_t M, int64_t 
   D.rank = (lora_a && lora_b) ? rank : 0; D.scaling = scaling;
   D.lora_mask = lora_mask; D.ld_lora_mask = ld_lora_mask; D.mask_scale = mask_scale;
   D.dx = dx; D.lddx = lddx;
+  D.lora_g = nullptr;
   return D;
 }
 
@@ -547,14 +550,16 @@ extern "C" int rq_nf4_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M,
                                         int absmax_dtype, const uint8_t* c2, int c2_format, int64_t block2,
                                         const void* lora_a, const void* lora_b, int64_t ld_lora_b, int lora_dtype,
                                         int64_t rank, float scaling, const uint8_t* lora_mask, int64_t ld_lora_mask,
-                                        float mask_scale, void* dx, int64_t lddx, void* workspace,
-                                        int64_t workspace_bytes, void* scratch, int64_t scratch_bytes,
+                                        float mask_scale, void* dx, int64_t lddx, const void* lora_g,
+                                        void* workspace, int64_t workspace_bytes, void* scratch, int64_t scratch_bytes,
                                         hipStream_t stream) {
-  const rq::DxArgs D = pack_dx_args(dy, dy_dtype, M, N, lddy, w_packed, K, block_size, absmax, absmax_dtype, c2,
+  rq::DxArgs D = pack_dx_args(dy, dy_dtype, M, N, lddy, w_packed, K, block_size, absmax, absmax_dtype, c2,
                                     c2_format, block2, lora_a, lora_b, ld_lora_b, lora_dtype, rank, scaling,
                                     lora_mask, ld_lora_mask, mask_scale, dx, lddx);
   const int st = rq::validate_dx(D);
   if (st != RQ_OK) return st;
+  if (dy_dtype != RQ_DTYPE_F32) D.lora_g = D.rank > 0 ? lora_g : nullptr;
+  if (D.lora_g && !rq::aligned(lora_g, 16)) return RQ_ERR_BAD_ALIGNMENT;
   if (scratch && scratch_bytes > 0 && M > 0) {
     const size_t need = rq::dense_scratch_bytes(dy_dtype, M, K, N, D.rank > 0 ? D.rank : 0);
     if (need > 0 && size_t(scratch_bytes) >= need && rq::dense_nf4_dx_ok(D))

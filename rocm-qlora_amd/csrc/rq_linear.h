@@ -128,6 +128,7 @@ struct DxArgs {
   float mask_scale;
   void* dx;
   int64_t lddx;
+  const void* lora_g;  // RND(RND(dY * s) . RND(B)) [M][rank rounded up to 16] when the caller has it (16-bit dY)
 };
 
 int validate_dx(const DxArgs& D);

@@ -25,4 +25,9 @@ int run_lora_rows(int xt, const uint16_t* x, int64_t ldx, int64_t M, int64_t K, 
                   int64_t s_j, int64_t s_k, int R, bool prescale, float scale, const LoraRowsPlan& p, float* part,
                   uint16_t* out, int R16, hipStream_t stream);
 
+// The same product's fp32 partials alone, part[split][m][j].
+int run_lora_rows_parts(int xt, const uint16_t* x, int64_t ldx, int64_t M, int64_t K, const void* s, int s_dt,
+                        int64_t s_j, int64_t s_k, int R, bool prescale, float scale, const LoraRowsPlan& p,
+                        float* part, hipStream_t stream);
+
 }  // namespace rq

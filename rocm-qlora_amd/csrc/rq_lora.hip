@@ -22,6 +22,9 @@ namespace rq {
 constexpr int kLoraChunkK = 256;   // k per LDS stage of S
 constexpr int kLoraSPitch = kLoraChunkK + 8;
 constexpr int kLoraMaxSplits = 16;
+// how S is read: value by value, fp32 16 bytes at a time, or already in the
+// activation dtype, 16 bytes at a time
+constexpr int kVecNone = 0, kVecF32 = 1, kVecX = 2;
 
 // X[m, k] (16-bit, row stride ldx) times RND(S)[j, k] over k in this split's
 // range, for the 16 W activation rows (W waves of 16) and the 16 JB ranks
@@ -35,7 +38,7 @@ constexpr int kLoraMaxSplits = 16;
 template <int XT, bool PRESCALE, int JB, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void lora_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M,
                                                         int64_t K, const void* __restrict__ s, int sdt, int64_t s_j,
-                                                        int64_t s_k, bool s_rows, bool svec, int R, float prescale,
+                                                        int64_t s_k, bool s_rows, int svec, int R, float prescale,
                                                         int64_t k_per_split, float* __restrict__ part) {
   __shared__ __attribute__((aligned(16))) uint16_t ss[16 * JB * kLoraSPitch];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -52,14 +55,17 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
   f32x4 acc[JB];
 #pragma unroll
   for (int jb = 0; jb < JB; ++jb) acc[jb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int64_t kc = k0; kc < k1; kc += kLoraChunkK) {
-    const int len = int(k1 - kc < kLoraChunkK ? k1 - kc : kLoraChunkK);  // multiple of 64
-    // this lane's activation fragments of the whole chunk, issued before the
-    // staging so that their latency overlaps it
-    u32x4 xf[kLoraChunkK / 32];
+  // this lane's activation fragments of a whole chunk: the first chunk's
+  // issued before its staging, the next one's before the current one's MFMAs
+  u32x4 xn[kLoraChunkK / 32];
+  auto load_x = [&](int64_t kc) {
 #pragma unroll
     for (int t = 0; t < kLoraChunkK / 32; ++t)
-      if (32 * t < len) xf[t] = *reinterpret_cast<const u32x4*>(xr + kc + 32 * t + 8 * q4);
+      if (kc + 32 * t < k1) xn[t] = *reinterpret_cast<const u32x4*>(xr + kc + 32 * t + 8 * q4);
+  };
+  load_x(k0);
+  for (int64_t kc = k0; kc < k1; kc += kLoraChunkK) {
+    const int len = int(k1 - kc < kLoraChunkK ? k1 - kc : kLoraChunkK);  // multiple of 64
     __syncthreads();
     if (s_rows) {
       // 16 JB ranks x len in 16-byte chunks, CPR per rank: thread tid takes
@@ -70,7 +76,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
       for (int i = 0; i < 16 * JB / (NT / CPR); ++i) {
         const int jj = tid / CPR + (NT / CPR) * i, j = j0 + jj;
         if (8 * c < len) {
-          const u32x4 v = load_a8<XT>(s, sdt, int64_t(j) * s_j + kc + 8 * c, j < R, svec);
+          const int64_t off = int64_t(j) * s_j + kc + 8 * c;
+          u32x4 v;
+          if (svec == kVecX)
+            v = j < R ? *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(s) + off) : u32x4{0u, 0u, 0u, 0u};
+          else
+            v = load_a8<XT>(s, sdt, off, j < R, svec == kVecF32);
           *reinterpret_cast<u32x4*>(ss + jj * kLoraSPitch + 8 * c) = v;
         }
       }
@@ -86,7 +97,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
           const int i = tid / 256 + (NT / 256) * n;
           if (i >= 2 * JB) break;
           const int j = j0 + 8 * i;
-          const u32x4 v = j < R ? load_a8_masked<XT>(s, sdt, (kc + kk) * s_k + j, R - j, svec)
+          const u32x4 v = j < R ? load_a8_masked<XT>(s, sdt, (kc + kk) * s_k + j, R - j, svec == kVecF32)
                                 : u32x4{0u, 0u, 0u, 0u};
           const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -96,6 +107,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
       }
     }
     __syncthreads();
+    u32x4 xf[kLoraChunkK / 32];
+#pragma unroll
+    for (int t = 0; t < kLoraChunkK / 32; ++t) xf[t] = xn[t];
+    load_x(kc + kLoraChunkK);
 #pragma unroll
     for (int t = 0; t < kLoraChunkK / 32; ++t) {
       if (32 * t >= len) break;
@@ -201,7 +216,7 @@ LoraRowsPlan plan_lora_rows(int64_t M, int64_t K, int64_t R, int cus) {
 
 template <int XT, bool PRESCALE, int JB, int W>
 static void launch_rows_jb(const uint16_t* x, int64_t ldx, int64_t M, int64_t K, const void* s, int sdt,
-                           int64_t s_j, int64_t s_k, bool s_rows, bool svec, int R, float prescale,
+                           int64_t s_j, int64_t s_k, bool s_rows, int svec, int R, float prescale,
                            const LoraRowsPlan& p, float* part, hipStream_t stream) {
   dim3 grid(unsigned((M + 16 * W - 1) / (16 * W)), unsigned((R + 16 * JB - 1) / (16 * JB)), unsigned(p.splits));
   lora_rows_kernel<XT, PRESCALE, JB, W><<<grid, 64 * W, 0, stream>>>(x, ldx, M, K, s, sdt, s_j, s_k, s_rows, svec, R,
@@ -210,7 +225,7 @@ static void launch_rows_jb(const uint16_t* x, int64_t ldx, int64_t M, int64_t K,
 
 template <int XT, bool PRESCALE>
 static void launch_rows_t(const uint16_t* x, int64_t ldx, int64_t M, int64_t K, const void* s, int sdt, int64_t s_j,
-                          int64_t s_k, bool s_rows, bool svec, int R, float prescale, const LoraRowsPlan& p,
+                          int64_t s_k, bool s_rows, int svec, int R, float prescale, const LoraRowsPlan& p,
                           float* part, hipStream_t stream) {
   if (p.jb == 1)
     launch_rows_jb<XT, PRESCALE, 1, 4>(x, ldx, M, K, s, sdt, s_j, s_k, s_rows, svec, R, prescale, p, part, stream);
@@ -220,15 +235,17 @@ static void launch_rows_t(const uint16_t* x, int64_t ldx, int64_t M, int64_t K, 
     launch_rows_jb<XT, PRESCALE, 4, 8>(x, ldx, M, K, s, sdt, s_j, s_k, s_rows, svec, R, prescale, p, part, stream);
 }
 
-int run_lora_rows(int xt, const uint16_t* x, int64_t ldx, int64_t M, int64_t K, const void* s, int s_dt,
-                  int64_t s_j, int64_t s_k, int R, bool prescale, float scale, const LoraRowsPlan& p, float* part,
-                  uint16_t* out, int R16, hipStream_t stream) {
+int run_lora_rows_parts(int xt, const uint16_t* x, int64_t ldx, int64_t M, int64_t K, const void* s, int s_dt,
+                        int64_t s_j, int64_t s_k, int R, bool prescale, float scale, const LoraRowsPlan& p,
+                        float* part, hipStream_t stream) {
   if (!aligned(x, 16) || ldx % 8 != 0 || K % 64 != 0) return RQ_ERR_BAD_ALIGNMENT;
   if (s_k != 1 && s_j != 1) return RQ_ERR_BAD_SHAPE;
   // contiguous runs of S are read 16 bytes at a time when aligned
   const bool s_rows = s_k == 1;
   const int64_t run_stride = s_rows ? s_j : s_k;
-  const bool svec = aligned(s, 16) && (s_dt != RQ_DTYPE_F32 || run_stride % 4 == 0);
+  const int svec = !aligned(s, 16) ? kVecNone
+                   : s_dt == RQ_DTYPE_F32 ? (run_stride % 4 == 0 ? kVecF32 : kVecNone)
+                   : s_dt == xt && s_rows && run_stride % 8 == 0 ? kVecX : kVecNone;
   if (xt == RQ_DTYPE_BF16) {
     if (prescale)
       launch_rows_t<RQ_DTYPE_BF16, true>(x, ldx, M, K, s, s_dt, s_j, s_k, s_rows, svec, R, scale, p, part, stream);
@@ -240,7 +257,13 @@ int run_lora_rows(int xt, const uint16_t* x, int64_t ldx, int64_t M, int64_t K, 
     else
       launch_rows_t<RQ_DTYPE_F16, false>(x, ldx, M, K, s, s_dt, s_j, s_k, s_rows, svec, R, scale, p, part, stream);
   }
-  int st = rq_check_launch();
+  return rq_check_launch();
+}
+
+int run_lora_rows(int xt, const uint16_t* x, int64_t ldx, int64_t M, int64_t K, const void* s, int s_dt,
+                  int64_t s_j, int64_t s_k, int R, bool prescale, float scale, const LoraRowsPlan& p, float* part,
+                  uint16_t* out, int R16, hipStream_t stream) {
+  const int st = run_lora_rows_parts(xt, x, ldx, M, K, s, s_dt, s_j, s_k, R, prescale, scale, p, part, stream);
   if (st != RQ_OK) return st;
   const unsigned blocks = unsigned((M * (R16 / 4) + 255) / 256);
   if (xt == RQ_DTYPE_BF16)

@@ -72,7 +72,11 @@ SIGNATURES = {
                                  _P, _I32, _I64,                     # c2, c2 format, block2
                                  _P, _P, _I64, _I32, _I64, _F32,     # A, B, ldB, dtype, rank, scaling
                                  _P, _I64, _F32,                     # dropout mask, ld, mask scale
-                                 _P, _I64, _P, _I64, _P, _I64, _P],  # dx, lddx, workspace, bytes, scratch, bytes, stream
+                                 _P, _I64, _P, _P, _I64, _P, _I64, _P],  # dx, lddx, g, workspace, bytes, scratch, bytes, stream
+    "rq_lora_grads_scratch_size": [_I32, _I64, _I64, _I64, _I64, _P],
+    "rq_lora_grads": [_P, _I32, _I64, _I64, _I64, _P, _I64, _I64,  # x, dtype, M, K, ldx, dy, N, lddy
+                      _P, _P, _I64, _I32, _I64, _F32,        # A, B, ldB, dtype, rank, scaling
+                      _P, _P, _P, _P, _I64, _P],             # dA, dB, g, scratch, bytes, stream
     "rq_int8_linear": [_P, _I32, _I64, _I64, _I64,           # x, dtype, M, K, ldx
                        _P, _I64, _I64, _P, _I32,             # q, N, block, scales, dtype
                        _P, _I32, _P, _I64, _P],              # bias, dtype, y, ldy, stream

@@ -23,6 +23,7 @@ from typing import Optional
 import torch
 
 from rocm_qlora import _native as nat
+from rocm_qlora import ops
 from rocm_qlora import torch_ops
 
 # activation dtypes of the HIP linear kernels
@@ -103,6 +104,27 @@ def _lora_term(x, lora_a, lora_b, scaling):
     return x @ lora_a.to(x.dtype).T @ lora_b.to(x.dtype).T * scaling
 
 
+def _lora_backward(dy, x, A, B, s, need_a, need_b, need_g):
+    """Gradients of (x A^T) B^T * s in x's dtype, cast to the parameters':
+    dv = dY * s, dB = dv^T (x A^T), dA = (dv B)^T x; and dv B (None where the
+    torch path runs), which dX's LoRA term starts from.  The HIP kernels run in
+    eager first-order backward passes; tracing, create_graph (whose result is
+    differentiated again), fp32 and ranks past 64 run on torch."""
+    if not torch_ops.compiling() and not torch.is_grad_enabled() and dy.dtype == x.dtype and \
+            ops.lora_grads_supported(x, A):
+        return ops.lora_grads(x, dy, A, B, s, need_a, need_b, need_g)
+    da = db = None
+    dt = x.dtype
+    x2 = x.reshape(-1, x.shape[-1])
+    dv = dy.reshape(-1, dy.shape[-1]).to(dt) * s
+    if need_b:
+        u = x2 @ A.to(dt).T
+        db = (dv.T @ u).to(B.dtype)
+    if need_a:
+        da = ((dv @ B.to(dt)).T @ x2).to(A.dtype)
+    return da, db, None
+
+
 class _FusedNF4LinearFunc(torch.autograd.Function):
     """y = x . W_deq^T + bias (+ LoRA) by the HIP kernels; backward gives dX
     (NF4 dX kernel, LoRA term fused) and the adapters' gradients.
@@ -136,23 +158,14 @@ class _FusedNF4LinearFunc(torch.autograd.Function):
         w: NF4Weight = ctx.w
         s = ctx.scaling
         need_x, need_a, need_b = ctx.needs_input_grad[:3]
-        dx = da = db = None
+        dx = da = db = g = None
+        grads = ctx.lora and (need_a or need_b)
+        if grads:
+            da, db, g = _lora_backward(dy, xl if xl is not None else x, A, B, s, need_a, need_b, need_x)
         if need_x:
             dx = torch_ops.call_nf4_linear_dx(dy, w.packed, w.scales, w.K, w.block_size,
                                               lora_a=A, lora_b=B, scaling=s, lora_mask=mask,
-                                              mask_scale=ctx.mask_scale, **w.dq_kwargs())
-        if ctx.lora and (need_a or need_b):
-            # lora_out = ((xl A^T) B^T) * s in x's dtype, xl = drop(x) or x:
-            # dv = dY * s, dB = dv^T (xl A^T), dA = (dv B)^T xl, cast to the
-            # parameters' dtype
-            dt = x.dtype
-            x2 = (xl if xl is not None else x).reshape(-1, x.shape[-1])
-            dv = dy.reshape(-1, dy.shape[-1]).to(dt) * s
-            if need_b:
-                u = x2 @ A.to(dt).T
-                db = (dv.T @ u).to(B.dtype)
-            if need_a:
-                da = ((dv @ B.to(dt)).T @ x2).to(A.dtype)
+                                              mask_scale=ctx.mask_scale, lora_g=g, **w.dq_kwargs())
         return dx, da, db, None, None, None, None
 
 

@@ -248,12 +248,13 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
                   blocksize_2: int = 256, use_fp8_c2: bool = True,
                   lora_a: Optional[torch.Tensor] = None, lora_b: Optional[torch.Tensor] = None,
                   scaling: float = 0.0, lora_mask: Optional[torch.Tensor] = None,
-                  mask_scale: float = 1.0) -> torch.Tensor:
+                  mask_scale: float = 1.0, lora_g: Optional[torch.Tensor] = None) -> torch.Tensor:
     """dX = dY . dequant(W) (+ the LoRA term ((dY * s) . B) . A) for an NF4
     weight stored flat (dequant_matmul.py:338-351, lora_layer.py:67
     differentiated).  With lora_mask (the dropout mask of the adapter's input,
     [..., K] bool), the LoRA term goes through dropout's backward: times
-    mask * mask_scale.  dy: [..., N] fp32/bf16/fp16 on the GPU; output
+    mask * mask_scale.  lora_g: the adapter's (dY * s) . B as lora_grads returns
+    it, when the caller has it.  dy: [..., N] fp32/bf16/fp16 on the GPU; output
     [..., K] in dy's dtype.  Shapes outside the MFMA dX kernel's (N or K not
     multiples of 64, other block sizes, fp32 dy) run on the generic kernels."""
     N = dy.shape[-1]
@@ -311,9 +312,45 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
                  nat.ptr(codes), nat.C2_FP8_E4M3FNUZ if use_fp8_c2 else nat.C2_INT8, blocksize_2,
                  nat.ptr(la), nat.ptr(lb), ldb, lcode, rank, float(scaling),
                  nat.ptr(mk), ldm, float(mask_scale),
-                 dx.data_ptr(), K, nat.ptr(ws), ws.numel() if ws is not None else 0,
+                 dx.data_ptr(), K, nat.ptr(lora_g), nat.ptr(ws), ws.numel() if ws is not None else 0,
                  nat.ptr(scratch), scratch.numel() if scratch is not None else 0, nat.stream_handle(dev))
     return dx.reshape(*lead, K)
+
+
+def lora_grads_supported(x: torch.Tensor, lora_a: torch.Tensor) -> bool:
+    """Whether lora_grads takes activations and adapters like these."""
+    return x.dtype in (torch.bfloat16, torch.float16) and lora_a.shape[0] <= 64 and x.numel() > 0
+
+
+def lora_grads(x: torch.Tensor, dy: torch.Tensor, lora_a: torch.Tensor, lora_b: torch.Tensor, scaling: float,
+               need_a: bool = True, need_b: bool = True, need_g: bool = False):
+    """The adapters' gradients of x -> (x A^T) B^T * s (lora_layer.py:67
+    differentiated, every intermediate in x's dtype): dB = (dY s)^T (x A^T) and
+    dA = ((dY s) B)^T x, in the adapters' dtypes, and (dY s) B as nf4_linear_dx
+    takes it.  x: [..., K] bf16/fp16, dy: [..., N].  Returns (dA, dB, g), None
+    where not asked for."""
+    K, N, rank = x.shape[-1], dy.shape[-1], lora_a.shape[0]
+    dev = nat.require_gpu(x, dy, lora_a, lora_b)
+    if lora_a.shape[1] != K or lora_b.shape != (N, rank):
+        raise RuntimeError(f"LoRA shapes {tuple(lora_a.shape)} / {tuple(lora_b.shape)} do not fit {N}x{K}")
+    with on(dev):
+        x2, ldx = (_aligned_rows if K % 64 == 0 else _rows)(x, K)
+        dy2, lddy = (_aligned_rows if N % 64 == 0 else _rows)(dy.to(x.dtype), N)
+        M = x2.shape[0]
+        if dy2.shape[0] != M:
+            raise RuntimeError(f"dY has {dy2.shape[0]} rows, x {M}")
+        a = lora_a if lora_a.dtype in (torch.float32, x.dtype) else lora_a.float()
+        a = a.contiguous()
+        b, ldb = _rows(lora_b.to(a.dtype), rank)
+        da = torch.empty((rank, K), dtype=a.dtype, device=dev) if need_a else None
+        db = torch.empty((N, rank), dtype=a.dtype, device=dev) if need_b else None
+        g = torch.empty((M, -(-rank // 16) * 16), dtype=x.dtype, device=dev) if need_g else None
+        code = nat.dtype_code(x.dtype)
+        scratch = _scratch("rq_lora_grads_scratch_size", dev, code, M, K, N, rank)
+        nat.call("rq_lora_grads", x2.data_ptr(), code, M, K, ldx, dy2.data_ptr(), N, lddy,
+                 a.data_ptr(), b.data_ptr(), ldb, nat.dtype_code(a.dtype), rank, float(scaling),
+                 nat.ptr(da), nat.ptr(db), nat.ptr(g), scratch.data_ptr(), scratch.numel(), nat.stream_handle(dev))
+    return (da.to(lora_a.dtype) if need_a else None, db.to(lora_b.dtype) if need_b else None, g)
 
 
 def _aligned_rows(t: torch.Tensor, K: int) -> Tuple[torch.Tensor, int]:

@@ -117,7 +117,7 @@ def _int8_linear_w8a8_fake(x, q, scales, bias):
     return x.new_empty((*x.shape[:-1], n))
 
 
-def _compiling() -> bool:
+def compiling() -> bool:
     try:
         return torch.compiler.is_compiling()
     except AttributeError:  # older torch
@@ -128,7 +128,7 @@ def call_nf4_linear(x, weight_quant, weight_scales, out_features, block_size=64,
                     c2_scales=None, blocksize_2=256, use_fp8_c2=True, lora_a=None, lora_b=None, scaling=0.0,
                     lora_x=None):
     """ops.nf4_linear, through the registered operator while being traced."""
-    if _compiling():
+    if compiling():
         return torch.ops.rocm_qlora.nf4_linear(x, weight_quant, weight_scales, int(out_features), int(block_size),
                                                bias, c2, c2_scales, int(blocksize_2), bool(use_fp8_c2), lora_a,
                                                lora_b, float(scaling), lora_x)
@@ -139,48 +139,48 @@ def call_nf4_linear(x, weight_quant, weight_scales, out_features, block_size=64,
 
 def call_nf4_linear_dx(dy, weight_quant, weight_scales, in_features, block_size=64, *, c2=None, c2_scales=None,
                        blocksize_2=256, use_fp8_c2=True, lora_a=None, lora_b=None, scaling=0.0, lora_mask=None,
-                       mask_scale=1.0):
+                       mask_scale=1.0, lora_g=None):
     """ops.nf4_linear_dx, through the registered operator while being traced."""
-    if _compiling():
+    if compiling():
         return torch.ops.rocm_qlora.nf4_linear_dx(dy, weight_quant, weight_scales, int(in_features),
                                                   int(block_size), c2, c2_scales, int(blocksize_2),
                                                   bool(use_fp8_c2), lora_a, lora_b, float(scaling), lora_mask,
                                                   float(mask_scale))
     return ops.nf4_linear_dx(dy, weight_quant, weight_scales, in_features, block_size, c2=c2, c2_scales=c2_scales,
                              blocksize_2=blocksize_2, use_fp8_c2=use_fp8_c2, lora_a=lora_a, lora_b=lora_b,
-                             scaling=scaling, lora_mask=lora_mask, mask_scale=mask_scale)
+                             scaling=scaling, lora_mask=lora_mask, mask_scale=mask_scale, lora_g=lora_g)
 
 
 def call_int8_linear(x, q, scales, out_features, block_size=0, bias=None):
     """ops.int8_linear, through the registered operator while being traced."""
-    if _compiling():
+    if compiling():
         return torch.ops.rocm_qlora.int8_linear(x, q, scales, int(out_features), int(block_size), bias)
     return ops.int8_linear(x, q, scales, out_features, block_size, bias)
 
 
 def call_int8_linear_dx(dy, q, scales, in_features, block_size=0):
     """ops.int8_linear_dx, through the registered operator while being traced."""
-    if _compiling():
+    if compiling():
         return torch.ops.rocm_qlora.int8_linear_dx(dy, q, scales, int(in_features), int(block_size))
     return ops.int8_linear_dx(dy, q, scales, in_features, block_size)
 
 
 def call_fp8_quantize(t):
     """ops.fp8_quantize, through the registered operator while being traced."""
-    if _compiling():
+    if compiling():
         return torch.ops.rocm_qlora.fp8_quantize(t)
     return ops.fp8_quantize(t)
 
 
 def call_fp8_linear(x, w_codes, w_scale, bias=None):
     """ops.fp8_linear, through the registered operator while being traced."""
-    if _compiling():
+    if compiling():
         return torch.ops.rocm_qlora.fp8_linear(x, w_codes, w_scale, bias)
     return ops.fp8_linear(x, w_codes, w_scale, bias)
 
 
 def call_int8_linear_w8a8(x, q, scales, bias=None):
     """ops.int8_linear_w8a8, through the registered operator while being traced."""
-    if _compiling():
+    if compiling():
         return torch.ops.rocm_qlora.int8_linear_w8a8(x, q, scales, bias)
     return ops.int8_linear_w8a8(x, q, scales, bias)
