@@ -47,6 +47,7 @@
 #include "rq_gemm8.h"
 #include "rq_dense.h"
 #include "rq_generic.h"
+#include "rq_skinny.h"
 
 namespace rq {
 
@@ -299,6 +300,8 @@ static size_t dx_at_bytes(int64_t K, int64_t rank16) { return (size_t(K) * size_
 
 int gemm_workspace(const LinearArgs& L, size_t* bytes) {
   *bytes = plan_gemm(L.M, L.N, L.K, L.rank, device_cus(), true).ws_bytes;
+  if (skinny_takes(L.M, L.N, L.K, L.rank))
+    *bytes = std::max(*bytes, skinny_workspace(L.M, L.N, L.K, L.rank));
   return RQ_OK;
 }
 
@@ -311,6 +314,13 @@ int run_nf4_gemm(const LinearArgs& L, void* workspace, size_t ws_bytes, uint32_t
   // the activation operands are loaded 16 bytes at a time
   if (!aligned(L.x, 16) || L.ldx % 8 != 0) return RQ_ERR_BAD_ALIGNMENT;
   if (!offsets_fit(L.M, L.ldx, L.N, L.K)) return RQ_ERR_UNSUPPORTED;
+  // few rows: the skinny kernel, given room for its splits
+  if (skinny_takes(L.M, L.N, L.K, L.rank)) {
+    const size_t need = skinny_workspace(L.M, L.N, L.K, L.rank), counters = skinny_counters(L.M, L.N, L.K);
+    if ((need == 0 || (workspace && ws_bytes >= need && aligned(workspace, 256))) &&
+        (counters == 0 || (tile_cnt && counters <= n_cnt)) && aligned(L.w_packed, 16))
+      return run_skinny_nf4(L, workspace, ws_bytes, tile_cnt, stream);
+  }
   // K splits need the zeroed tile counts and room for their partial tiles;
   // without them the GEMM runs unsplit
   GemmPlan p = plan_gemm(L.M, L.N, L.K, L.rank, device_cus(), true);
