@@ -1,6 +1,8 @@
 // Device and host helpers shared by the NF4 linear kernels (GEMV, GEMM, dX).
 #pragma once
 
+#include <atomic>
+
 #include "rq_mfma.h"
 #include "rq_linear.h"
 
@@ -218,11 +220,17 @@ __device__ __forceinline__ u32x4 load_a8_strided(const void* p, int dt, int64_t 
 // ---------------------------------------------------------------------------
 // Host helpers
 // ---------------------------------------------------------------------------
+// Compute units of the current device, asked of the runtime once per device
+// (a launch plan otherwise costs several attribute queries per call; racing
+// threads store the same value).
 inline int device_cus() {
+  static std::atomic<int> known[64];
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev >= 0 && dev < 64 && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     return 256;
+  if (dev >= 0 && dev < 64) known[dev].store(cus, std::memory_order_relaxed);
   return cus;
 }
 

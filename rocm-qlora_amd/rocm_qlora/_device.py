@@ -9,7 +9,6 @@ raise: there is no CPU implementation in this package.
 """
 from __future__ import annotations
 
-from contextlib import contextmanager
 from typing import Tuple
 
 import torch
@@ -31,7 +30,18 @@ def to_gpu(t: torch.Tensor) -> Tuple[torch.Tensor, torch.device]:
     return (t if t.device == dev else t.to(dev)), t.device
 
 
-@contextmanager
-def on(device: torch.device):
-    with torch.cuda.device(device):
-        yield
+class on:
+    """`with on(device)`: that GPU current inside the block (nothing is changed
+    when it already is, which costs one query)."""
+    __slots__ = ("_guard",)
+
+    def __init__(self, device: torch.device):
+        same = device.index is not None and device.index == torch.cuda.current_device()
+        self._guard = None if same else torch.cuda.device(device)
+
+    def __enter__(self):
+        if self._guard is not None:
+            self._guard.__enter__()
+
+    def __exit__(self, *exc):
+        return None if self._guard is None else self._guard.__exit__(*exc)

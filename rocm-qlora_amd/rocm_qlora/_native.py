@@ -179,17 +179,23 @@ def stream_capture_id(handle: int) -> int:
     return int(cid.value)
 
 
+_DTYPE_CODES = {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16}
+
+
 def dtype_code(dt: torch.dtype) -> int:
-    if dt == torch.float32:
-        return DTYPE_F32
-    if dt == torch.bfloat16:
-        return DTYPE_BF16
-    if dt == torch.float16:
-        return DTYPE_F16
-    raise TypeError(f"unsupported dtype {dt}: expected float32, bfloat16 or float16")
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        raise TypeError(f"unsupported dtype {dt}: expected float32, bfloat16 or float16")
+    return code
+
+
+# the current stream's handle without building a Stream object
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_handle(device: torch.device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -203,13 +209,14 @@ def require_gpu(*tensors: Optional[torch.Tensor]) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 f"rocm_qlora_amd kernels run on the GPU; got a tensor on {t.device}")
+        d = t.device
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
+            dev = d
+        elif d != dev:
+            raise RuntimeError(f"tensors on different devices: {dev} and {d}")
     if dev is None:
         raise RuntimeError("no tensor given")
     return dev

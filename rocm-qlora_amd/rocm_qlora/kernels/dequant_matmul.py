@@ -21,6 +21,7 @@ from dataclasses import dataclass
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from rocm_qlora import _native as nat
 from rocm_qlora import ops
@@ -186,6 +187,19 @@ class _FusedInt8LinearFunc(torch.autograd.Function):
         return torch_ops.call_int8_linear_dx(dy, w.q, w.scales, w.K, w.block_size), None, None
 
 
+_functorch_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: True)
+
+
+def _nothing_recorded(*inputs) -> bool:
+    """Whether autograd records nothing for an op on these inputs, so that the
+    forward can run without its autograd function: no gradient asked for, and
+    neither tracing, a functorch transform nor forward-mode AD active (those go
+    through the function, which accepts or refuses them)."""
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs):
+        return False
+    return not torch_ops.compiling() and not _functorch_active() and forward_ad._current_level < 0
+
+
 def nf4_linear(x: torch.Tensor, w: NF4Weight, bias: Optional[torch.Tensor] = None,
                lora_a: Optional[torch.Tensor] = None, lora_b: Optional[torch.Tensor] = None,
                scaling: float = 0.0, dropout_p: float = 0.0) -> torch.Tensor:
@@ -196,6 +210,9 @@ def nf4_linear(x: torch.Tensor, w: NF4Weight, bias: Optional[torch.Tensor] = Non
         raise TypeError(f"NF4 linear takes fp32/bf16/fp16 activations, got {x.dtype}")
     # the reference adds bias.to(x.dtype) (quant_linear.py:196)
     bias = bias.to(x.dtype) if bias is not None else None
+    if dropout_p == 0.0 and _nothing_recorded(x, lora_a, lora_b, bias):
+        return ops.nf4_linear(x, w.packed, w.scales, w.N, w.block_size, bias, lora_a=lora_a, lora_b=lora_b,
+                              scaling=scaling, **w.dq_kwargs())
     return _FusedNF4LinearFunc.apply(x, lora_a, lora_b, bias, w, scaling, float(dropout_p))
 
 
@@ -205,6 +222,8 @@ def int8_linear(x: torch.Tensor, w: Int8Weight, bias: Optional[torch.Tensor] = N
     if not w.kernel_ok(x.dtype):
         raise TypeError(f"INT8 linear takes fp32/bf16/fp16 activations, got {x.dtype}")
     bias = bias.to(x.dtype) if bias is not None else None
+    if _nothing_recorded(x, bias):
+        return ops.int8_linear(x, w.q, w.scales, w.N, w.block_size, bias)
     return _FusedInt8LinearFunc.apply(x, bias, w)
 
 

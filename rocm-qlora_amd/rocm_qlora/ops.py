@@ -7,6 +7,8 @@ GPU, or a missing library, raises.
 """
 from __future__ import annotations
 
+import ctypes
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -23,10 +25,17 @@ GEMV_MAX_B_ELEMS = 1 << 29
 
 def _rows(t: torch.Tensor, K: int) -> Tuple[torch.Tensor, int]:
     """[..., K] -> 2-D [rows, K] view with unit inner stride, and its row stride."""
-    t2 = t.reshape(-1, K)
-    if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < K):
+    t2 = t if t.dim() == 2 and t.shape[1] == K else t.reshape(-1, K)
+    rows, (ld, inner) = t2.shape[0], t2.stride()
+    if inner != 1 or (rows > 1 and ld < K):
         t2 = t2.contiguous()
-    return t2, (t2.stride(0) if t2.shape[0] > 1 else K)
+        ld = t2.stride(0)
+    return t2, (ld if rows > 1 else K)
+
+
+def _flat(t: torch.Tensor) -> torch.Tensor:
+    """t as contiguous 1-D."""
+    return (t if t.dim() == 1 else t.reshape(-1)).contiguous()
 
 
 # rq_nf4_linear's workspace.  Its first RQ_LINEAR_SYNC_BYTES
@@ -68,11 +77,14 @@ _CAPTURE_POOL_LIMIT = 1 << 30  # pre-zeroed capture buffers per device, at most 
 _CAPTURE_POOL: dict = {}       # device index -> pre-zeroed buffers not yet handed out
 _CAPTURE_POOL_BASE: dict = {}  # device index -> the allocations they are views of (kept for good)
 _CAPTURE_POOL_TOTAL: dict = {}  # device index -> bytes of those allocations
+_CAPTURE_POOL_MAX: dict = {}   # device index -> size of the largest buffer not yet handed out
 
 
 def _ensure_capture_pool(dev, idx: int, need: int) -> None:
     """The device's pool exists and holds a free entry of at least `need`
     bytes (while the pool stays within _CAPTURE_POOL_LIMIT)."""
+    if _CAPTURE_POOL_MAX.get(idx, -1) >= need:
+        return
     if idx not in _CAPTURE_POOL_BASE:
         base = torch.zeros(_CAPTURE_POOL_ENTRIES * _CAPTURE_POOL_BYTES, dtype=torch.uint8, device=dev)
         torch.cuda.current_stream(dev).synchronize()  # zero before any later capture, on any stream, replays it
@@ -81,7 +93,8 @@ def _ensure_capture_pool(dev, idx: int, need: int) -> None:
         _CAPTURE_POOL[idx] = [base[i * _CAPTURE_POOL_BYTES:(i + 1) * _CAPTURE_POOL_BYTES]
                               for i in range(_CAPTURE_POOL_ENTRIES)]
     pool = _CAPTURE_POOL[idx]
-    if any(e.numel() >= need for e in pool):
+    _CAPTURE_POOL_MAX[idx] = max((e.numel() for e in pool), default=0)
+    if _CAPTURE_POOL_MAX[idx] >= need:
         return
     size = -(-max(need, _CAPTURE_POOL_BYTES) // _CAPTURE_POOL_BYTES) * _CAPTURE_POOL_BYTES
     if _CAPTURE_POOL_TOTAL[idx] + size > _CAPTURE_POOL_LIMIT:
@@ -91,6 +104,7 @@ def _ensure_capture_pool(dev, idx: int, need: int) -> None:
     _CAPTURE_POOL_BASE[idx].append(buf)
     _CAPTURE_POOL_TOTAL[idx] += size
     pool.append(buf)
+    _CAPTURE_POOL_MAX[idx] = size
 
 
 def _zeroed_area(nbytes: int, dev, min_bytes: int = _WS_MIN_BYTES) -> torch.Tensor:
@@ -100,14 +114,11 @@ def _zeroed_area(nbytes: int, dev, min_bytes: int = _WS_MIN_BYTES) -> torch.Tens
 
 
 def _workspace(x_dtype: torch.dtype, M: int, K: int, N: int, rank: int, dev) -> Optional[torch.Tensor]:
-    import ctypes
-    nbytes = ctypes.c_int64(0)
-    nat.call("rq_nf4_linear_workspace_size", nat.dtype_code(x_dtype), M, K, N, rank, ctypes.byref(nbytes))
-    need = nbytes.value
+    idx = dev.index if dev.index is not None else torch.cuda.current_device()
+    need = _bytes("rq_nf4_linear_workspace_size", idx, nat.dtype_code(x_dtype), M, K, N, rank)
     if need == 0:
         return None
-    idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = nat.stream_handle(dev)
     if torch.cuda.is_current_stream_capturing():
         cid = nat.capture_id(dev)
         # the buffers of captures that have ended belong to their graphs'
@@ -126,6 +137,7 @@ def _workspace(x_dtype: torch.dtype, M: int, K: int, N: int, rank: int, dev) -> 
             fits = [i for i, e in enumerate(pool) if e.numel() >= need]
             if fits:
                 ws = pool.pop(min(fits, key=lambda i: pool[i].numel()))
+                _CAPTURE_POOL_MAX[idx] = max((e.numel() for e in pool), default=0)
             else:
                 ws = _zeroed_area(need, dev, min_bytes=LINEAR_SYNC_BYTES)
             _CAPTURE_WS[key] = ws
@@ -139,6 +151,15 @@ def _workspace(x_dtype: torch.dtype, M: int, K: int, N: int, rank: int, dev) -> 
     return ws
 
 
+@functools.lru_cache(maxsize=4096)
+def _bytes(size_fn: str, device_index, *args) -> int:
+    """What the library's size query `size_fn` reports for sizes and dtype codes
+    (a function of those and the current device's compute units alone)."""
+    nbytes = ctypes.c_int64(0)
+    nat.call(size_fn, *args, ctypes.byref(nbytes))
+    return nbytes.value
+
+
 def _step(dtype: torch.dtype) -> int:
     """Elements of one 128-byte k step of the dense GEMM's activations."""
     return 32 if dtype == torch.float32 else 64
@@ -148,10 +169,8 @@ def _scratch(size_fn: str, dev, *args) -> Optional[torch.Tensor]:
     """Scratch memory for one call, of the size `size_fn` reports (None when
     none is used): from torch's caching allocator, which hands it out again in
     stream order once the tensor is dropped."""
-    import ctypes
-    nbytes = ctypes.c_int64(0)
-    nat.call(size_fn, *args, ctypes.byref(nbytes))
-    return torch.empty(nbytes.value, dtype=torch.uint8, device=dev) if nbytes.value else None
+    n = _bytes(size_fn, dev.index, *args)
+    return torch.empty(n, dtype=torch.uint8, device=dev) if n else None
 
 
 def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optional[torch.Tensor],
@@ -173,13 +192,11 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
     dq = c2 is not None
     scales = c2_scales if dq else weight_scales
     dev = nat.require_gpu(x, weight_quant, scales, bias, lora_a, lora_b, c2)
-    packed = weight_quant.reshape(-1)
-    if packed.dtype != torch.uint8:
-        raise TypeError(f"NF4 weight_quant must be uint8, got {packed.dtype}")
-    if packed.numel() * 2 < N * K:
-        raise RuntimeError(f"weight_quant holds {packed.numel() * 2} codes, need {N}x{K}")
-    packed = packed.contiguous()
-    scales = scales.reshape(-1).contiguous()
+    if weight_quant.dtype != torch.uint8:
+        raise TypeError(f"NF4 weight_quant must be uint8, got {weight_quant.dtype}")
+    if weight_quant.numel() * 2 < N * K:
+        raise RuntimeError(f"weight_quant holds {weight_quant.numel() * 2} codes, need {N}x{K}")
+    packed, scales = _flat(weight_quant), _flat(scales)
     if block_size < 1:
         raise RuntimeError(f"block_size must be positive, got {block_size}")
     n_blocks = -(-N * K // block_size)
@@ -188,7 +205,6 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
             raise RuntimeError("c2 / c2_scales too short for the weight")
     elif scales.numel() < n_blocks:
         raise RuntimeError(f"weight_scales holds {scales.numel()} values, need {n_blocks}")
-    lead = x.shape[:-1]
     with on(dev):
         x2, ldx = _rows(x, K)
         M = x2.shape[0]
@@ -200,7 +216,7 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
             x2, ldx = _aligned_rows(x2, K)
         y = torch.empty((M, N), dtype=x.dtype, device=dev)
         if M == 0:
-            return y.reshape(*lead, N)
+            return y.reshape(*x.shape[:-1], N)
         rank = 0
         la = lb = xl = None
         ldxl = ldb = 0
@@ -239,7 +255,7 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
                  nat.ptr(xl), ldxl, nat.ptr(la), nat.ptr(lb), ldb, lcode, rank, float(scaling),
                  y.data_ptr(), N, nat.ptr(ws), ws.numel() if ws is not None else 0,
                  nat.ptr(scratch), scratch.numel() if scratch is not None else 0, nat.stream_handle(dev))
-    return y.reshape(*lead, N)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
 
 
 def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optional[torch.Tensor],
@@ -262,13 +278,11 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
     dq = c2 is not None
     scales = c2_scales if dq else weight_scales
     dev = nat.require_gpu(dy, weight_quant, scales, lora_a, lora_b, c2)
-    packed = weight_quant.reshape(-1)
-    if packed.dtype != torch.uint8:
-        raise TypeError(f"NF4 weight_quant must be uint8, got {packed.dtype}")
-    if packed.numel() * 2 < N * K:
-        raise RuntimeError(f"weight_quant holds {packed.numel() * 2} codes, need {N}x{K}")
-    packed = packed.contiguous()
-    scales = scales.reshape(-1).contiguous()
+    if weight_quant.dtype != torch.uint8:
+        raise TypeError(f"NF4 weight_quant must be uint8, got {weight_quant.dtype}")
+    if weight_quant.numel() * 2 < N * K:
+        raise RuntimeError(f"weight_quant holds {weight_quant.numel() * 2} codes, need {N}x{K}")
+    packed, scales = _flat(weight_quant), _flat(scales)
     lead = dy.shape[:-1]
     with on(dev):
         # the dX kernels load dY rows 16 bytes at a time
@@ -445,10 +459,7 @@ def fp8_quantize(t: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         src, ld = _rows(t2, cols)
         codes = torch.empty((rows, cols), dtype=torch.uint8, device=dev)
         scale = torch.empty((), dtype=torch.float32, device=dev)
-        import ctypes
-        nb = ctypes.c_int64(0)
-        nat.call("rq_fp8_quantize_workspace_size", ctypes.byref(nb))
-        ws = torch.empty(nb.value, dtype=torch.uint8, device=dev)
+        ws = _scratch("rq_fp8_quantize_workspace_size", dev)
         nat.call("rq_fp8_quantize", src.data_ptr(), nat.dtype_code(t.dtype), rows, cols, ld,
                  codes.data_ptr(), scale.data_ptr(), ws.data_ptr(), ws.numel(), nat.stream_handle(dev))
     return codes.view(torch.float8_e4m3fnuz), scale
@@ -493,10 +504,7 @@ def fp8_linear(x: torch.Tensor, w_codes: torch.Tensor, w_scale: torch.Tensor,
         y = torch.empty((M, N), dtype=x.dtype, device=dev)
         if M == 0:
             return y.reshape(*lead, N)
-        import ctypes
-        nb = ctypes.c_int64(0)
-        nat.call("rq_fp8_linear_workspace_size", M, K, ctypes.byref(nb))
-        ws = torch.empty(nb.value, dtype=torch.uint8, device=dev)
+        ws = _scratch("rq_fp8_linear_workspace_size", dev, M, K)
         b = bias.to(x.dtype).contiguous() if bias is not None else None
         nat.call("rq_fp8_linear", x2.data_ptr(), nat.dtype_code(x.dtype), M, K, ldx,
                  wc.data_ptr(), N, ws_scale.data_ptr(), nat.ptr(b),
@@ -552,10 +560,7 @@ def int8_linear_w8a8(x: torch.Tensor, q: torch.Tensor, scales: torch.Tensor,
         y = torch.empty((M, N), dtype=x.dtype, device=dev)
         if M == 0:
             return y.reshape(*lead, N)
-        import ctypes
-        nb = ctypes.c_int64(0)
-        nat.call("rq_int8_linear_w8a8_workspace_size", M, K, ctypes.byref(nb))
-        ws = torch.empty(nb.value, dtype=torch.uint8, device=dev)
+        ws = _scratch("rq_int8_linear_w8a8_workspace_size", dev, M, K)
         b = bias.to(x.dtype).contiguous() if bias is not None else None
         nat.call("rq_int8_linear_w8a8", x2.data_ptr(), nat.dtype_code(x.dtype), M, K, ldx,
                  wq.data_ptr(), N, sc.data_ptr(), nat.dtype_code(sc.dtype), nat.ptr(b),
