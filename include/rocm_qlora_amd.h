@@ -338,16 +338,32 @@ int rq_int8_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_
                       int64_t lddx, hipStream_t stream);
 
 /* rq_int8_linear and rq_int8_linear_dx with optional scratch memory, as
- * rq_nf4_linear_scratch (dx: 0 the forward, 1 dX). */
+ * rq_nf4_linear_scratch (dx: 0 the forward, 1 dX).  dX also takes the adapter's
+ * term, RND(dX + RND(RND(g RND(A)) * d)), with rank > 0: g [M, rank rounded up to
+ * 16] as rq_lora_grads leaves it, A [rank, K] of lora_dtype (fp32 or dy_dtype), d
+ * = 1, or mask_scale where lora_mask [M, K] (stride ld_lora_mask) is non-zero and
+ * 0 elsewhere; that needs 16-bit dY and the scratch memory. */
 int rq_int8_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int dx,
-                                int64_t* bytes);
+                                int64_t rank, int64_t* bytes);
 int rq_int8_linear_scratch(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* q,
                            int64_t N, int64_t block_size, const void* scales, int scales_dtype, const void* bias,
                            int bias_dtype, void* y, int64_t ldy, void* scratch, int64_t scratch_bytes,
                            hipStream_t stream);
 int rq_int8_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy, const int8_t* q,
-                              int64_t K, int64_t block_size, const void* scales, int scales_dtype, void* dx,
-                              int64_t lddx, void* scratch, int64_t scratch_bytes, hipStream_t stream);
+                              int64_t K, int64_t block_size, const void* scales, int scales_dtype,
+                              const void* lora_g, const void* lora_a, int lora_dtype, int64_t rank,
+                              const uint8_t* lora_mask, int64_t ld_lora_mask, float mask_scale,
+                              void* dx, int64_t lddx, void* scratch, int64_t scratch_bytes, hipStream_t stream);
+
+/* The adapter's term added in place (lora_layer.py:67-70), 16-bit activations:
+ *   y = RND(y + RND(RND(RND(x RND(A)^T) RND(B)^T) * scaling))
+ * x [M, K] (K a multiple of 64, rows 16-byte aligned) stride ldx, A [rank, K], B
+ * [N, rank] stride ld_lora_b, both of lora_dtype (fp32 or x_dtype), rank <= 256;
+ * y [M, N] stride ldy, x_dtype.  workspace: 256-byte aligned. */
+int rq_lora_add_workspace_size(int64_t M, int64_t K, int64_t rank, int64_t* bytes);
+int rq_lora_add(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const void* lora_a,
+                const void* lora_b, int64_t ld_lora_b, int lora_dtype, int64_t rank, float scaling,
+                void* y, int64_t N, int64_t ldy, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
 /* Bytes of workspace rq_fp8_quantize needs. */
 int rq_fp8_quantize_workspace_size(int64_t* bytes);

@@ -400,45 +400,56 @@ extern "C" int rq_int8_linear(const void* x, int x_dtype, int64_t M, int64_t K, 
 }
 
 extern "C" int rq_int8_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int dx,
-                                           int64_t* bytes) {
+                                           int64_t rank, int64_t* bytes) {
   if (!bytes) return RQ_ERR_NULL_POINTER;
   if (!rq::valid_float_dtype(x_dtype)) return RQ_ERR_BAD_DTYPE;
-  if (M < 0 || N < 1 || K < 1 || block_size < 0) return RQ_ERR_BAD_SHAPE;
+  if (M < 0 || N < 1 || K < 1 || block_size < 0 || rank < 0 || rank > 256) return RQ_ERR_BAD_SHAPE;
   const bool fast = !dx && x_dtype != RQ_DTYPE_F32 && K % 64 == 0 &&
                     (block_size == 0 ||
                      (block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0));
   const int64_t C = dx ? K : N, R = dx ? N : K;
-  *bytes = fast && !rq::dense_beats_fused(M, C, R, false) ? 0 : int64_t(rq::dense_scratch_bytes(x_dtype, M, C, R, 0));
+  *bytes = fast && !rq::dense_beats_fused(M, C, R, false) ? 0 : int64_t(rq::dense_scratch_bytes(x_dtype, M, C, R, dx ? rank : 0));
   return RQ_OK;
 }
 
 extern "C" int rq_int8_linear_dx_scratch(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy,
                                          const int8_t* q, int64_t K, int64_t block_size, const void* scales,
-                                         int scales_dtype, void* dx, int64_t lddx, void* scratch,
+                                         int scales_dtype, const void* lora_g, const void* lora_a, int lora_dtype,
+                                         int64_t rank, const uint8_t* lora_mask, int64_t ld_lora_mask,
+                                         float mask_scale, void* dx, int64_t lddx, void* scratch,
                                          int64_t scratch_bytes, hipStream_t stream) {
   if (!dy || !q || !scales || !dx) return RQ_ERR_NULL_POINTER;
   if (!rq::valid_float_dtype(dy_dtype) || !rq::valid_float_dtype(scales_dtype)) return RQ_ERR_BAD_DTYPE;
   if (M < 0 || N <= 0 || K <= 0 || block_size < 0 || lddy < N || lddx < K) return RQ_ERR_BAD_SHAPE;
   if (!rq::aligned(dy, rq::dtype_size(dy_dtype)) || !rq::aligned(dx, rq::dtype_size(dy_dtype)))
     return RQ_ERR_BAD_ALIGNMENT;
+  if (rank < 0 || rank > 256 || (lora_mask && ld_lora_mask < K)) return RQ_ERR_BAD_SHAPE;
+  if (rank > 0) {
+    if (!lora_g || !lora_a) return RQ_ERR_NULL_POINTER;
+    if (dy_dtype == RQ_DTYPE_F32 || (lora_dtype != RQ_DTYPE_F32 && lora_dtype != dy_dtype)) return RQ_ERR_BAD_DTYPE;
+    if (!rq::aligned(lora_g, 16)) return RQ_ERR_BAD_ALIGNMENT;
+  }
   if (M == 0) return RQ_OK;
   rq::GenericInt8 g{};
+  g.rank = rank; g.lora_g = lora_g; g.lora_a = lora_a; g.lora_dtype = lora_dtype;
+  g.lora_mask = lora_mask; g.ld_lora_mask = ld_lora_mask; g.mask_scale = mask_scale;
   g.x = dy; g.x_dtype = dy_dtype; g.M = M; g.K = K; g.N = N; g.ldx = lddy;
   g.q = q; g.block_size = block_size; g.scales = scales; g.scales_dtype = scales_dtype;
   g.y = dx; g.ldy = lddx;
   if (scratch && scratch_bytes > 0) {
-    const size_t need = rq::dense_scratch_bytes(dy_dtype, M, K, N, 0);
+    const size_t need = rq::dense_scratch_bytes(dy_dtype, M, K, N, rank);
     if (need > 0 && size_t(scratch_bytes) >= need && rq::dense_int8_ok(g, true))
       return rq::run_dense_int8(g, true, scratch, size_t(scratch_bytes), stream);
   }
+  if (rank > 0) return RQ_ERR_WORKSPACE;  // the generic kernels add no adapter term here
   return rq::run_generic_int8_dx(g, stream);
 }
 
 extern "C" int rq_int8_linear_dx(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t lddy, const int8_t* q,
                                  int64_t K, int64_t block_size, const void* scales, int scales_dtype, void* dx,
                                  int64_t lddx, hipStream_t stream) {
-  return rq_int8_linear_dx_scratch(dy, dy_dtype, M, N, lddy, q, K, block_size, scales, scales_dtype, dx, lddx, nullptr,
-                                   0, stream);
+  return rq_int8_linear_dx_scratch(dy, dy_dtype, M, N, lddy, q, K, block_size, scales, scales_dtype, nullptr,
+                                   nullptr, 0, 0, nullptr, 0, 1.0f, dx, lddx, nullptr, 0, stream);
 }
 
 extern "C" int rq_fp8_quantize_workspace_size(int64_t* bytes) {

@@ -336,22 +336,23 @@ struct DensePlan {
 };
 
 // Microseconds of a tiling, from measurements with all 256 compute units busy:
-// 1.5 us per 64-k step of a 256 x 256 tile and 0.55 us of a 128 x 128 one
-// (N(0, 1) operands; power bound), K splits adding 20 and 8 us for their
-// partial tiles (2048 x 4096 x 4096: 128 tiles of 256 in two splits 77 us,
-// 512 tiles of 128 unsplit 69 us; 1024 x 4096 x 4096: 55.6 and 35.5 us;
-// 4096 x 4096 x 14336: 347 and 429 us).  fp32: 128 x 128 tiles, 2 us per 32-k
-// step, up to 8 splits (fp32 MFMA bound).
+// 1.45 us per 64-k step of a 256 x 256 tile and 8 us per round of tiles, 0.55 us
+// per step of a 128 x 128 one (N(0, 1) operands; power bound), K splits adding
+// 20 and 8 us for their partial tiles (2048 x 4096 x 4096: 128 tiles of 256 in
+// two splits 77 us, 512 tiles of 128 unsplit 69 us; 1024 x 4096 x 4096: 55.6 and
+// 35.5 us; 4096 x 4096 x 14336: 347 and 429 us).  fp32: 128 x 128 tiles, 2 us per
+// 32-k step, up to 8 splits (fp32 MFMA bound).
 double pick_tiles(DensePlan& p, int xt, int64_t M, int64_t C, int nk, int cus) {
   const bool f32 = xt == RQ_DTYPE_F32;
   double best = 1e300;
   for (int h = f32 ? 1 : 2; h >= 1; --h) {
     const int64_t B = 128 * h, tm = ceil_div(M, B), tn = ceil_div(C, B), T = tm * tn;
-    const double step = f32 ? 2.0 : (h == 2 ? 1.5 : 0.55), extra = h == 2 ? 20.0 : 8.0;
+    const double step = f32 ? 2.0 : (h == 2 ? 1.45 : 0.55), round = h == 2 ? 8.0 : 0.0, extra = h == 2 ? 20.0 : 8.0;
     const int64_t lt = T % cus, lf = T - lt;
     for (int s = 1; s <= (f32 ? 8 : 4); s *= 2) {
       if (s > 1 && (lt == 0 || lt * s > cus || nk / s < 4)) break;
-      const double t = step * (double(lf / cus) * nk + (lt ? double(ceil_div(nk, s)) : 0.0)) + (s > 1 ? extra : 0.0);
+      const double t = double(lf / cus) * (step * nk + round) + (lt ? step * double(ceil_div(nk, s)) + round : 0.0) +
+                       (s > 1 ? extra : 0.0);
       if (t < best) {
         best = t;
         p.halves = h;
@@ -623,9 +624,9 @@ size_t dense_scratch_bytes(int x_dtype, int64_t M, int64_t C, int64_t R, int64_t
 
 // Estimates in microseconds from measurements on the Llama-3-8B shapes (M = 64
 // .. 2048): the fused GEMM takes 1.15 us per 64-k step of a full wave of
-// 256 x 128 tiles (0.9 us while fewer than half the compute units have one)
-// and 12 us for its K splits; decoding takes 0.5 us per million weights and its
-// launches 6 us.  Both sides near the line, fused against dense: q forward M =
+// 256 x 128 tiles (0.9 us while fewer than half the compute units have one),
+// 6 us per wave of tiles and 12 us for its K splits; decoding takes 0.5 us per million weights and its
+// launches 8 us.  Both sides near the line, fused against dense: q forward M =
 // 2048 93 / 105 us, gate forward M = 512 86 / 111 us and M = 1024 165 / 142 us,
 // q dX M = 1024 90 / 62 us, down dX M = 512 98 / 116 us, M = 1024 183 / 145 us.
 bool dense_beats_fused(int64_t M, int64_t C, int64_t R, bool splits) {
@@ -635,10 +636,10 @@ bool dense_beats_fused(int64_t M, int64_t C, int64_t R, bool splits) {
   const int64_t T = int64_t(f.tiles_m) * f.tiles_n;
   const double nk = double(R) / 64.0, step = T * f.splits >= cus / 2 ? 1.15 : 0.9;
   const double waves = f.splits > 1 ? double(f.lf * 8 / cus) + 1.0 / f.splits : double(ceil_div(T, cus));
-  const double fused = nk * step * waves + (f.splits > 1 ? 12.0 : 0.0);
+  const double fused = nk * step * waves + 6.0 * double(ceil_div(T, cus)) + (f.splits > 1 ? 12.0 : 0.0);
   DensePlan p{};
   const double dense = pick_tiles(p, RQ_DTYPE_BF16, M, C, int((R + 63) / 64), cus);
-  return dense + 6.0 + 0.5e-6 * double(C) * double(R) < fused;
+  return dense + 8.0 + 0.5e-6 * double(C) * double(R) < fused;
 }
 
 // fp32 forward against the GEMV kernels over blocks of 16 rows, about 1.2 us per
@@ -699,6 +700,12 @@ int run_dense_int8(const GenericInt8& A, bool dx, void* scratch, size_t bytes, h
   P.xt = A.x_dtype; P.x = A.x; P.ldx = A.ldx; P.M = A.M; P.C = dx ? A.K : A.N; P.R = dx ? A.N : A.K;
   P.e.bias = dx ? nullptr : A.bias; P.e.bias_dt = A.bias_dtype; P.e.scaling = 1.0f;
   P.e.y = A.y; P.e.ldy = A.ldy;
+  if (dx && A.rank > 0) {
+    P.rank = A.rank; P.u = A.lora_g;
+    P.f = A.lora_a; P.f_c = 1; P.f_j = A.K;
+    P.lora_dt = A.lora_dtype;
+    P.e.mask = A.lora_mask; P.e.ldm = A.ld_lora_mask; P.e.mask_scale = A.mask_scale;
+  }
   auto ws = [&](auto fn) {
     return with_nf4_scale(A.scales, A.scales_dtype, nullptr, 0, 1, fn);
   };

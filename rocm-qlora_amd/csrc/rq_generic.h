@@ -38,6 +38,16 @@ struct GenericInt8 {
   int bias_dtype;
   void* y;  // [M, N] (forward) or [M, K] (dX), row stride ldy
   int64_t ldy;
+  // dX through the dense path only: the adapter's term RND(RND(g . RND(A)) * d),
+  // g [M, rank rounded up to 16] as rq_lora_grads leaves it, A [rank, K], d = mask
+  // ? mask_scale : 0 (1 without a mask)
+  int64_t rank;
+  const void* lora_g;
+  const void* lora_a;
+  int lora_dtype;
+  const uint8_t* lora_mask;
+  int64_t ld_lora_mask;
+  float mask_scale;
 };
 int run_generic_int8_linear(const GenericInt8& A, hipStream_t stream);
 int run_generic_int8_dx(const GenericInt8& A, hipStream_t stream);

@@ -185,6 +185,77 @@ __global__ __launch_bounds__(256) void lora_finish_kernel(const float* __restric
   *reinterpret_cast<uint2*>(out + m * R16 + j0) = uint2{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3])};
 }
 
+// y[m][n] = RND(y + RND(RND(sum_j u[m][j] RND(B[n][j])) * s)) in place: the
+// adapter's term added to a linear whose kernel has no LoRA epilogue (INT8,
+// FP8).  A workgroup takes 32 rows x 256 columns, a wave 64 of the columns as
+// 16x16x32 MFMAs with B's rows as the A operand (a lane's four results along a
+// row); the terms go through LDS so that y moves in whole 512-byte row pieces.
+// Bound by reading and writing y (512 x 28672: see rq_lora_add).
+constexpr int kAddRows = 32, kAddCols = 256, kAddPitch = kAddCols + 8;
+
+template <int XT>
+__global__ __launch_bounds__(256) void lora_add_kernel(const uint16_t* __restrict__ u, int R16, const void* b, int b_dt,
+                                                       int64_t ldb, bool b_vec, int rank, float s, int64_t M, int64_t N,
+                                                       uint16_t* y, int64_t ldy) {
+  __shared__ __attribute__((aligned(16))) uint16_t t[kAddRows * kAddPitch];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, q = lane >> 4;
+  const int64_t n0 = int64_t(blockIdx.x) * kAddCols, m0 = int64_t(blockIdx.y) * kAddRows;
+  const uint16_t* up[2];
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int64_t m = m0 + 16 * mb + i16;
+    up[mb] = u + (m < M ? m : M - 1) * R16 + 8 * q;
+  }
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    const int64_t n = n0 + 64 * wave + 16 * nb + i16, nl = n < N ? n : N - 1;
+    f32x4 lo[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    for (int j0 = 0; j0 < R16; j0 += 32) {
+      const int left = rank - j0 - 8 * q;
+      const u32x4 bv = left > 0 ? load_a8_masked<XT>(b, b_dt, nl * ldb + j0 + 8 * q, left, b_vec)
+                                : u32x4{0u, 0u, 0u, 0u};
+      const bool in = j0 + 8 * q < R16;  // R16 is a multiple of 16
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+        lo[mb] = mfma16x16x32<XT>(bv, in ? *reinterpret_cast<const u32x4*>(up[mb] + j0) : u32x4{0u, 0u, 0u, 0u},
+                                  lo[mb]);
+    }
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = __fmul_rn(round_x<XT>(lo[mb][r]), s);
+      *reinterpret_cast<u32x2*>(t + (16 * mb + i16) * kAddPitch + 64 * wave + 16 * nb + 4 * q) =
+          u32x2{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3])};
+    }
+  }
+  __syncthreads();
+  const bool vec = (reinterpret_cast<uintptr_t>(y) & 15u) == 0 && (ldy & 7) == 0;
+  const int64_t n = n0 + 8 * (tid & 31);
+#pragma unroll
+  for (int it = 0; it < 4; ++it) {
+    const int r = 8 * it + (tid >> 5);
+    const int64_t m = m0 + r;
+    if (m >= M || n >= N) continue;
+    const u32x4 l = *reinterpret_cast<const u32x4*>(t + r * kAddPitch + 8 * (tid & 31));
+    uint16_t* yp = y + m * ldy + n;
+    if (vec && n + 8 <= N) {
+      const u32x4 a = *reinterpret_cast<const u32x4*>(yp);
+      u32x4 o;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        o[c] = cvt_pk<XT>(__fadd_rn(from_x16<XT>(a[c] & 0xFFFFu), from_x16<XT>(l[c] & 0xFFFFu)),
+                          __fadd_rn(from_x16<XT>(a[c] >> 16), from_x16<XT>(l[c] >> 16)));
+      *reinterpret_cast<u32x4*>(yp) = o;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        if (n + c < N)
+          yp[c] = uint16_t(to_x16<XT>(__fadd_rn(from_x16<XT>(yp[c]), from_x16<XT>((l[c >> 1] >> (16 * (c & 1))) & 0xFFFFu))));
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -274,3 +345,60 @@ int run_lora_rows(int xt, const uint16_t* x, int64_t ldx, int64_t M, int64_t K, 
 }
 
 }  // namespace rq
+
+// ---------------------------------------------------------------------------
+// C ABI
+// ---------------------------------------------------------------------------
+namespace {
+struct AddPlan {
+  rq::LoraRowsPlan lr;
+  int64_t r16;
+  size_t u, bytes;
+};
+AddPlan plan_add(int64_t M, int64_t K, int64_t rank) {
+  AddPlan p{};
+  p.r16 = (rank + 15) / 16 * 16;
+  p.lr = rq::plan_lora_rows(M, K, rank, rq::device_cus());
+  p.u = p.lr.part_bytes;
+  p.bytes = p.u + ((size_t(M) * p.r16 * 2 + 255) & ~size_t(255));
+  return p;
+}
+}  // namespace
+
+extern "C" int rq_lora_add_workspace_size(int64_t M, int64_t K, int64_t rank, int64_t* bytes) {
+  if (!bytes) return RQ_ERR_NULL_POINTER;
+  if (M < 1 || K < 1 || K % 64 != 0 || rank < 1 || rank > 256) return RQ_ERR_BAD_SHAPE;
+  *bytes = int64_t(plan_add(M, K, rank).bytes);
+  return RQ_OK;
+}
+
+extern "C" int rq_lora_add(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const void* lora_a,
+                           const void* lora_b, int64_t ld_lora_b, int lora_dtype, int64_t rank, float scaling,
+                           void* y, int64_t N, int64_t ldy, void* workspace, int64_t workspace_bytes,
+                           hipStream_t stream) {
+  using namespace rq;
+  if (x_dtype != RQ_DTYPE_BF16 && x_dtype != RQ_DTYPE_F16) return RQ_ERR_BAD_DTYPE;
+  if (lora_dtype != RQ_DTYPE_F32 && lora_dtype != x_dtype) return RQ_ERR_BAD_DTYPE;
+  if (M < 1 || K < 1 || K % 64 != 0 || N < 1 || rank < 1 || rank > 256 || ldx < K || ldy < N || ld_lora_b < rank)
+    return RQ_ERR_BAD_SHAPE;
+  if (!x || !lora_a || !lora_b || !y || !workspace) return RQ_ERR_NULL_POINTER;
+  if (!aligned(x, 16) || ldx % 8 != 0 || !aligned(y, 2) || !aligned(workspace, 256)) return RQ_ERR_BAD_ALIGNMENT;
+  const int64_t gy = (M + kAddRows - 1) / kAddRows;
+  if (gy > 65535) return RQ_ERR_UNSUPPORTED;
+  const AddPlan p = plan_add(M, K, rank);
+  if (workspace_bytes < 0 || size_t(workspace_bytes) < p.bytes) return RQ_ERR_WORKSPACE;
+  uint16_t* u = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + p.u);
+  const int st = run_lora_rows(x_dtype, static_cast<const uint16_t*>(x), ldx, M, K, lora_a, lora_dtype, K, 1,
+                               int(rank), false, 1.0f, p.lr, static_cast<float*>(workspace), u, int(p.r16), stream);
+  if (st != RQ_OK) return st;
+  const bool bvec = aligned(lora_b, 16) && (lora_dtype != RQ_DTYPE_F32 || ld_lora_b % 4 == 0);
+  const dim3 grid(unsigned((N + kAddCols - 1) / kAddCols), unsigned(gy));
+  uint16_t* yp = static_cast<uint16_t*>(y);
+  if (x_dtype == RQ_DTYPE_BF16)
+    lora_add_kernel<RQ_DTYPE_BF16><<<grid, 256, 0, stream>>>(u, int(p.r16), lora_b, lora_dtype, ld_lora_b, bvec,
+                                                             int(rank), scaling, M, N, yp, ldy);
+  else
+    lora_add_kernel<RQ_DTYPE_F16><<<grid, 256, 0, stream>>>(u, int(p.r16), lora_b, lora_dtype, ld_lora_b, bvec,
+                                                            int(rank), scaling, M, N, yp, ldy);
+  return rq_check_launch();
+}

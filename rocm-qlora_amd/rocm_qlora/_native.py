@@ -83,14 +83,18 @@ SIGNATURES = {
     "rq_int8_linear_dx": [_P, _I32, _I64, _I64, _I64,        # dy, dtype, M, N, lddy
                           _P, _I64, _I64, _P, _I32,          # q, K, block, scales, dtype
                           _P, _I64, _P],                     # dx, lddx, stream
-    "rq_int8_linear_scratch_size": [_I32, _I64, _I64, _I64, _I64, _I32, _P],
+    "rq_int8_linear_scratch_size": [_I32, _I64, _I64, _I64, _I64, _I32, _I64, _P],
     "rq_int8_linear_scratch": [_P, _I32, _I64, _I64, _I64,   # x, dtype, M, K, ldx
                                _P, _I64, _I64, _P, _I32,     # q, N, block, scales, dtype
                                _P, _I32, _P, _I64,           # bias, dtype, y, ldy
                                _P, _I64, _P],                # scratch, bytes, stream
     "rq_int8_linear_dx_scratch": [_P, _I32, _I64, _I64, _I64,  # dy, dtype, M, N, lddy
                                   _P, _I64, _I64, _P, _I32,    # q, K, block, scales, dtype
+                                  _P, _P, _I32, _I64, _P, _I64, _F32,  # g, A, dtype, rank, mask, ld, mask scale
                                   _P, _I64, _P, _I64, _P],     # dx, lddx, scratch, bytes, stream
+    "rq_lora_add_workspace_size": [_I64, _I64, _I64, _P],
+    "rq_lora_add": [_P, _I32, _I64, _I64, _I64, _P, _P, _I64, _I32, _I64, _F32,  # x, dtype, M, K, ldx, A, B, ldB, dtype, rank, scaling
+                    _P, _I64, _I64, _P, _I64, _P],           # y, N, ldy, workspace, bytes, stream
     "rq_merge_lora": [_P, _I32, _I64, _I64, _I64,           # w, format, N, K, block
                       _P, _I32, _P, _I32, _I64,             # scales, dtype, c2, c2 format, block2
                       _P, _P, _I64, _I32, _I64, _F32,       # A, B, ldB, dtype, rank, scaling

@@ -21,6 +21,7 @@ import torch.nn as nn
 from rocm_qlora import ops
 from rocm_qlora import torch_ops
 from rocm_qlora.fp8.fp8_config import detect_fp8_support, FP8Config
+from rocm_qlora.kernels import dequant_matmul as dm
 from rocm_qlora.lora.lora_layer import LoRALinear
 
 _FNUZ_MAX = 240.0
@@ -33,6 +34,15 @@ def _fp8_forward(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     # products (fp8_linear.py:44-52)
     wc, ws = w_q if w_q is not None else torch_ops.call_fp8_quantize(w)
     return torch_ops.call_fp8_linear(x, wc, ws, bias)
+
+
+def _stored_dx(dy: torch.Tensor, qw) -> torch.Tensor:
+    """dX = dY . W from the layer's stored NF4 / INT8 codes."""
+    if not qw.kernel_ok(dy.dtype):
+        raise TypeError(f"FP8 backward takes fp32/bf16/fp16 gradients, got {dy.dtype}")
+    if isinstance(qw, dm.NF4Weight):
+        return torch_ops.call_nf4_linear_dx(dy, qw.packed, qw.scales, qw.K, qw.block_size, **qw.dq_kwargs())
+    return dm.int8_dx(dy, qw)
 
 
 class _FP8LinearFunc(torch.autograd.Function):
@@ -50,16 +60,7 @@ class _FP8LinearFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        from rocm_qlora.kernels.dequant_matmul import NF4Weight
-        qw = ctx.qw
-        if not qw.kernel_ok(grad_output.dtype):
-            raise TypeError(f"FP8 backward takes fp32/bf16/fp16 gradients, got {grad_output.dtype}")
-        if isinstance(qw, NF4Weight):
-            dx = torch_ops.call_nf4_linear_dx(grad_output, qw.packed, qw.scales, qw.K, qw.block_size,
-                                              **qw.dq_kwargs())
-        else:
-            dx = torch_ops.call_int8_linear_dx(grad_output, qw.q, qw.scales, qw.K, qw.block_size)
-        return dx, None, None, None, None
+        return _stored_dx(grad_output, ctx.qw), None, None, None, None
 
 
 class FP8LinearWrapper(nn.Module):
@@ -99,6 +100,22 @@ class FP8LinearWrapper(nn.Module):
             w_q = self._weight(x.dtype)
             bias = ql.bias.to(x.dtype) if ql.bias is not None else None
             qw = ql.nf4_weight() if ql.bits == 4 else ql.int8_weight()
+            lora = self.base
+            if dm.native_adapter(x, lora.lora_A) and type(lora.lora_dropout) in (nn.Dropout, nn.Identity):
+                p = lora.lora_dropout.p if lora._dropout_active() else 0.0
+
+                def base_dx(dy, A, B, s, g, mask, mask_scale):
+                    if g is None:
+                        return dm.composed_dx(_stored_dx(dy, qw), dy, A, B, s, mask, mask_scale)
+                    if isinstance(qw, dm.NF4Weight):
+                        return ops.nf4_linear_dx(dy, qw.packed, qw.scales, qw.K, qw.block_size, lora_a=A, lora_b=B,
+                                                 scaling=s, lora_mask=mask, mask_scale=mask_scale, lora_g=g,
+                                                 **qw.dq_kwargs())
+                    return ops.int8_linear_dx(dy, qw.q, qw.scales, qw.K, qw.block_size, lora_a=A, lora_g=g,
+                                              lora_mask=mask, mask_scale=mask_scale)
+
+                return dm.base_lora_linear(x, lora.lora_A, lora.lora_B, lora.scaling, p,
+                                           lambda t: _fp8_forward(t, None, bias, w_q), base_dx)
             base_out = _FP8LinearFunc.apply(x, None, bias, w_q, qw)
             lora_out = (self.base.lora_dropout(x) @ self.base.lora_A.t().to(x.dtype)
                         @ self.base.lora_B.t().to(x.dtype) * self.base.scaling)

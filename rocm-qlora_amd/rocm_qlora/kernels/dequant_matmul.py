@@ -187,6 +187,83 @@ class _FusedInt8LinearFunc(torch.autograd.Function):
         return torch_ops.call_int8_linear_dx(dy, w.q, w.scales, w.K, w.block_size), None, None
 
 
+def native_adapter(x, lora_a) -> bool:
+    """Whether the adapter of an INT8 or FP8 layer runs on the LoRA kernels, both
+    ways (eager, 16-bit activations, K a multiple of 64, rank <= 64)."""
+    return not torch_ops.compiling() and not _functorch_active() and forward_ad._current_level < 0 and \
+        ops.lora_add_supported(x, lora_a) and ops.lora_grads_supported(x, lora_a)
+
+
+class _BaseLoRALinearFunc(torch.autograd.Function):
+    """base(x) + (drop(x) A^T) B^T * s where base is a HIP linear without a LoRA
+    epilogue (INT8, FP8): the term is added in place by the LoRA kernels, and
+    the backward is the adapters' gradient kernels and base's dX with the
+    adapter's input gradient in its epilogue.  base_dx(dy, A, B, s, g, mask,
+    mask_scale) returns that dX, or None where it cannot include the term."""
+
+    @staticmethod
+    def forward(ctx, x, lora_a, lora_b, scaling: float, dropout_p: float, base, base_dx):
+        xl, mask = x, None
+        if dropout_p > 0.0:
+            xl, mask = torch.ops.aten.native_dropout(x, float(dropout_p), True)
+        ctx.base_dx = base_dx
+        ctx.scaling = float(scaling)
+        ctx.mask_scale = 1.0 / (1.0 - dropout_p) if mask is not None else 1.0
+        ctx.save_for_backward(xl, lora_a, lora_b, mask)
+        return ops.lora_add_(base(x), xl, lora_a, lora_b, scaling)
+
+    @staticmethod
+    def backward(ctx, dy):
+        xl, A, B, mask = ctx.saved_tensors
+        need_x, need_a, need_b = ctx.needs_input_grad[:3]
+        da, db, g = _lora_backward(dy, xl, A, B, ctx.scaling, need_a, need_b, need_x)
+        dx = ctx.base_dx(dy, A, B, ctx.scaling, g, mask, ctx.mask_scale) if need_x else None
+        return dx, da, db, None, None, None, None
+
+
+def int8_lora_linear(x: torch.Tensor, w: Int8Weight, bias, lora_a, lora_b, scaling: float,
+                     dropout_p: float = 0.0) -> torch.Tensor:
+    """The INT8 linear plus the adapter's term, each rounded as the composed
+    layers round them (lora_layer.py:58-70)."""
+    if not native_adapter(x, lora_a):
+        y = int8_linear(x, w, bias)
+        xl = torch.nn.functional.dropout(x, dropout_p, True) if dropout_p > 0.0 else x
+        return y + _lora_term(xl, lora_a, lora_b, scaling).to(y.dtype)
+    nat.require_gpu(x, w.q)
+    bias = bias.to(x.dtype) if bias is not None else None
+
+    def base(x):
+        return ops.int8_linear(x, w.q, w.scales, w.N, w.block_size, bias)
+
+    def base_dx(dy, A, B, s, g, mask, mask_scale):
+        if g is not None:
+            return ops.int8_linear_dx(dy, w.q, w.scales, w.K, w.block_size, lora_a=A, lora_g=g, lora_mask=mask,
+                                      mask_scale=mask_scale)
+        return composed_dx(int8_dx(dy, w), dy, A, B, s, mask, mask_scale)
+
+    return base_lora_linear(x, lora_a, lora_b, scaling, dropout_p, base, base_dx)
+
+
+def base_lora_linear(x, lora_a, lora_b, scaling, dropout_p, base, base_dx):
+    """_BaseLoRALinearFunc, or its forward alone where nothing is recorded."""
+    if dropout_p == 0.0 and not (torch.is_grad_enabled() and
+                                 (x.requires_grad or lora_a.requires_grad or lora_b.requires_grad)):
+        return ops.lora_add_(base(x), x, lora_a, lora_b, scaling)
+    return _BaseLoRALinearFunc.apply(x, lora_a, lora_b, float(scaling), float(dropout_p), base, base_dx)
+
+
+def int8_dx(dy, w: Int8Weight):
+    return torch_ops.call_int8_linear_dx(dy, w.q, w.scales, w.K, w.block_size)
+
+
+def composed_dx(dx, dy, A, B, s, mask, mask_scale):
+    """dx plus the adapter's input gradient ((dY s) B) A (times the dropout mask)
+    by torch operators, which are differentiable again."""
+    dt = dy.dtype
+    t = (dy * s) @ B.to(dt) @ A.to(dt)
+    return dx + (t * (mask.to(dt) * mask_scale) if mask is not None else t)
+
+
 _functorch_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: True)
 
 

@@ -405,7 +405,7 @@ def int8_linear(x: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, out_feat
         if M == 0:
             return y.reshape(*lead, N)
         b = bias.contiguous() if bias is not None else None
-        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(x.dtype), M, K, N, block_size, 0)
+        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(x.dtype), M, K, N, block_size, 0, 0)
         nat.call("rq_int8_linear_scratch", x2.data_ptr(), nat.dtype_code(x.dtype), M, K, ldx,
                  qf.data_ptr(), N, block_size, sc.data_ptr(), nat.dtype_code(sc.dtype),
                  nat.ptr(b), nat.dtype_code(b.dtype) if b is not None else 0,
@@ -415,37 +415,83 @@ def int8_linear(x: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, out_feat
 
 
 def int8_linear_dx(dy: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, in_features: int,
-                   block_size: int = 0) -> torch.Tensor:
+                   block_size: int = 0, *, lora_a: Optional[torch.Tensor] = None,
+                   lora_g: Optional[torch.Tensor] = None, lora_mask: Optional[torch.Tensor] = None,
+                   mask_scale: float = 1.0) -> torch.Tensor:
     """dX = dY . (q * scale) for int8 weights (the backward of
     dequant_matmul.py:308-324: the dequantized weight rounded to dY's dtype,
     then the product), decoded inside the multiply.  q: [N, K] (or flat)
     int8, scales as for int8_linear; dy: [..., N] fp32/bf16/fp16 on the GPU;
-    output [..., K] in dy's dtype."""
+    output [..., K] in dy's dtype.  With lora_g (lora_grads' (dY s) B, 16-bit
+    dY) and lora_a, plus the adapter's g . A, through dropout's backward with
+    lora_mask as in nf4_linear_dx."""
     N = dy.shape[-1]
     K = int(in_features)
-    dev = nat.require_gpu(dy, q, scales)
+    dev = nat.require_gpu(dy, q, scales, lora_a, lora_g)
     if q.dtype != torch.int8:
         raise TypeError(f"int8 weights expected, got {q.dtype}")
-    qf = q.reshape(-1).contiguous()
-    if qf.numel() < N * K:
-        raise RuntimeError(f"q holds {qf.numel()} values, need {N}x{K}")
-    sc = scales.reshape(-1).contiguous()
+    if q.numel() < N * K:
+        raise RuntimeError(f"q holds {q.numel()} values, need {N}x{K}")
+    qf, sc = _flat(q), _flat(scales)
     need = N if block_size == 0 else -(-N * K // block_size)
     if sc.numel() < need:
         raise RuntimeError(f"scales hold {sc.numel()} values, need {need}")
-    lead = dy.shape[:-1]
     with on(dev):
         dy2, lddy = _aligned_rows(dy, N) if N % _step(dy.dtype) == 0 else _rows(dy, N)
         M = dy2.shape[0]
         dx = torch.empty((M, K), dtype=dy.dtype, device=dev)
         if M == 0:
-            return dx.reshape(*lead, K)
-        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(dy.dtype), M, K, N, block_size, 1)
+            return dx.reshape(*dy.shape[:-1], K)
+        rank, la, lcode, mk, ldm = 0, None, 0, None, 0
+        if lora_g is not None:
+            rank = lora_a.shape[0]
+            if lora_a.shape[1] != K or lora_g.shape != (M, -(-rank // 16) * 16) or lora_g.dtype != dy.dtype:
+                raise RuntimeError(f"LoRA shapes {tuple(lora_a.shape)} / {tuple(lora_g.shape)} do not fit {M}x{K}")
+            la = (lora_a if lora_a.dtype in (torch.float32, dy.dtype) else lora_a.float()).contiguous()
+            lcode = nat.dtype_code(la.dtype)
+            if lora_mask is not None:
+                mk, ldm = _rows(lora_mask.reshape(-1, K).view(torch.uint8), K)
+        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(dy.dtype), M, K, N, block_size, 1, rank)
+        if rank and (scratch is None or lddy * M * dy.element_size() >= 1 << 32):
+            # past the dense kernel's 32-bit offsets: the adapter's term by torch
+            t = lora_g[:, :rank] @ lora_a.to(dy.dtype)
+            if lora_mask is not None:
+                t = t * (lora_mask.reshape(-1, K).to(dy.dtype) * mask_scale)
+            return int8_linear_dx(dy, q, scales, K, block_size) + t.reshape(*dy.shape[:-1], K)
         nat.call("rq_int8_linear_dx_scratch", dy2.data_ptr(), nat.dtype_code(dy.dtype), M, N, lddy,
                  qf.data_ptr(), K, block_size, sc.data_ptr(), nat.dtype_code(sc.dtype),
+                 nat.ptr(lora_g) if rank else None, nat.ptr(la), lcode, rank, nat.ptr(mk), ldm, float(mask_scale),
                  dx.data_ptr(), K, nat.ptr(scratch), scratch.numel() if scratch is not None else 0,
                  nat.stream_handle(dev))
-    return dx.reshape(*lead, K)
+    return dx.reshape(*dy.shape[:-1], K)
+
+
+def lora_add_supported(x: torch.Tensor, lora_a: torch.Tensor) -> bool:
+    """Whether lora_add_ takes activations and adapters like these."""
+    return x.dtype in (torch.bfloat16, torch.float16) and x.shape[-1] % 64 == 0 and 0 < lora_a.shape[0] <= 256 \
+        and 0 < x.numel() // x.shape[-1] <= 1 << 20
+
+
+def lora_add_(y: torch.Tensor, x: torch.Tensor, lora_a: torch.Tensor, lora_b: torch.Tensor,
+              scaling: float) -> torch.Tensor:
+    """y += (x A^T) B^T * s in place (lora_layer.py:67-70: every intermediate in
+    x's dtype), for a contiguous y [..., N] in x's dtype; returns y."""
+    K, N, rank = x.shape[-1], y.shape[-1], lora_a.shape[0]
+    dev = nat.require_gpu(y, x, lora_a, lora_b)
+    if lora_a.shape[1] != K or lora_b.shape != (N, rank):
+        raise RuntimeError(f"LoRA shapes {tuple(lora_a.shape)} / {tuple(lora_b.shape)} do not fit {N}x{K}")
+    if y.dtype != x.dtype or not y.is_contiguous() or y.numel() // N != x.numel() // K:
+        raise RuntimeError(f"y must be contiguous [..., {N}] in {x.dtype} with x's rows")
+    with on(dev):
+        x2, ldx = _aligned_rows(x, K)
+        M = x2.shape[0]
+        a = (lora_a if lora_a.dtype in (torch.float32, x.dtype) else lora_a.float()).contiguous()
+        b, ldb = _rows(lora_b.to(a.dtype), rank)
+        ws = _scratch("rq_lora_add_workspace_size", dev, M, K, rank)
+        nat.call("rq_lora_add", x2.data_ptr(), nat.dtype_code(x.dtype), M, K, ldx, a.data_ptr(), b.data_ptr(), ldb,
+                 nat.dtype_code(a.dtype), rank, float(scaling), y.data_ptr(), N, N, ws.data_ptr(), ws.numel(),
+                 nat.stream_handle(dev))
+    return y
 
 
 def fp8_quantize(t: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -166,11 +166,10 @@ class QuantLinear(nn.Module):
         from rocm_qlora.kernels import dequant_matmul as dm
         if self.bits == 4:
             return dm.nf4_linear(x, self.nf4_weight(), self.bias, lora_a, lora_b, scaling, dropout_p)
-        y = dm.int8_linear(x, self.int8_weight(), self.bias)
+        w = self.int8_weight()
         if lora_a is not None and lora_b is not None and lora_a.shape[0] > 0:
-            xl = torch.nn.functional.dropout(x, dropout_p, True) if dropout_p > 0.0 else x
-            y = y + dm._lora_term(xl, lora_a, lora_b, scaling).to(y.dtype)
-        return y
+            return dm.int8_lora_linear(x, w, self.bias, lora_a, lora_b, scaling, dropout_p)
+        return dm.int8_linear(x, w, self.bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """y = x . W^T + bias in x's dtype, any leading dims (quant_linear.py:121-197)."""

@@ -56,3 +56,67 @@ def test_lora_grads_strided_and_partial(dev):
         alone = (ops.lora_grads(x, y, a, b, 2.0, True, False)[0], ops.lora_grads(x, y, a, b, 2.0, False, True)[1])
         assert all(torch.equal(p, q) for p, q in zip(ref, got))
         assert torch.equal(alone[0], ref[0]) and torch.equal(alone[1], ref[1])
+
+
+@pytest.mark.parametrize("M,K,N,rank,dtype", [(1, 64, 8, 8, "bf16"), (31, 128, 255, 17, "fp16"), (33, 320, 256, 16, "bf16"),
+                                              (100, 4096, 300, 80, "bf16"), (300, 192, 1000, 64, "fp16")])
+@pytest.mark.parametrize("lora32", [True, False])
+def test_lora_add(dev, M, K, N, rank, dtype, lora32):
+    """y += term in place: 32-row and 256-column tile edges, rows that are not
+    16-byte aligned (N odd), ranks of one to several MFMA steps.  Each of the
+    four roundings (u, the product, the scaling, the sum) is the reference's;
+    bound 4 * 2^-9 (2^-12) of the result."""
+    print(f"lora add {M} {K} {N} {rank} {dtype} {lora32}", flush=True)
+    dt = DT[dtype]
+    g = torch.Generator().manual_seed(M + K + N + rank)
+    x, y = torch.randn(M, K, generator=g).to(dt), torch.randn(M, N, generator=g).to(dt)
+    a, b = torch.randn(rank, K, generator=g) / K ** 0.5, torch.randn(N, rank, generator=g) / rank ** 0.5
+    if not lora32:
+        a, b = a.to(dt), b.to(dt)
+    got = y.to(dev).clone()
+    out = ops.lora_add_(got, x.to(dev), a.to(dev), b.to(dev), 0.75)
+    assert out is got
+    ref = y.double() + 0.75 * (x.double() @ a.to(dt).double().T) @ b.to(dt).double().T
+    err = float((got.cpu().double() - ref).norm() / ref.norm())
+    assert err <= 4 * 2.0 ** (-9 if dtype == "bf16" else -12), err
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8_nf4", "fp8_int8"])
+@pytest.mark.parametrize("p", [0.0, 0.25])
+@pytest.mark.parametrize("M", [5, 40])
+def test_byte_layers_with_adapter(dev, kind, p, M):
+    """LoRALinear on an INT8 layer and FP8LinearWrapper: output and gradients of
+    the fused adapter path against the same module composed by torch (its own
+    path under create_graph), with and without dropout (same seed, same mask).
+    The composed path rounds alike; sums in another order move a rounding by
+    one unit: 2^-7 of the value plus 2^-7 of the rms covers two such."""
+    import torch.nn as nn
+    from rocm_qlora import LoRALinear, QuantLinear
+    from rocm_qlora.fp8 import FP8LinearWrapper
+    from rocm_qlora.kernels import dequant_matmul as dm
+    torch.manual_seed(7)
+    layer = LoRALinear(QuantLinear.from_linear(nn.Linear(192, 136).to(dev), bits=4 if kind == "fp8_nf4" else 8, block_size=64),
+                       r=12, lora_alpha=24, lora_dropout=p).to(dev)
+    with torch.no_grad():
+        layer.lora_B.normal_(0, 0.05)
+    module = layer if kind == "int8" else FP8LinearWrapper(layer)
+    x = torch.randn(M, 192, device=dev, dtype=torch.bfloat16)
+    dy = torch.randn(M, 136, device=dev, dtype=torch.bfloat16)
+
+    def run():
+        torch.manual_seed(11)
+        xi = x.clone().requires_grad_(True)
+        y = module(xi)
+        return [y.detach(), *torch.autograd.grad(y, (xi, layer.lora_A, layer.lora_B), dy)]
+
+    got = run()
+    real = dm.native_adapter
+    dm.native_adapter = lambda *a: False
+    try:
+        ref = run()
+    finally:
+        dm.native_adapter = real
+    for name, a, b in zip(("y", "dx", "dA", "dB"), got, ref):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        d, f = (a.float() - b.float()).abs(), b.float()
+        assert bool((d <= 2.0 ** -7 * (f.abs() + f.square().mean().sqrt())).all()), (name, float(d.max()))
