@@ -433,6 +433,38 @@ __global__ __launch_bounds__(256) void nf4_dequant16_kernel(const uint32_t* __re
   }
 }
 
+// The fp32 output's counterpart: a quad is 4 weights, half a dword of codes and
+// one 16-byte output vector, so that a wave's store writes 1 KiB of consecutive
+// bytes here too (two adjacent lanes read the same dword and take a half each).
+// Wave v' owns quads 512 v' .. + 511, lane l quads 64 j + l, j = 0..7.  Bound by
+// the writes; with 16 weights per lane in four stores 64 bytes apart and the
+// scale behind runtime dtype branches, double_dequantize of 11008 x 4096 took 128
+// us (1.6 TB/s).
+template <class Scale>
+__global__ __launch_bounds__(256) void nf4_dequant32_kernel(const uint32_t* __restrict__ packed, Scale scale,
+                                                            int bs_log2, f32x4* __restrict__ out) {
+  __shared__ float lut[16];
+  if (threadIdx.x < 16) lut[threadIdx.x] = u2f(kNF4Bits[threadIdx.x]);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int64_t c0 = (int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6)) * 512 + lane;
+  uint32_t p[8];
+  float s[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) p[j] = __builtin_nontemporal_load(packed + ((c0 + 64 * j) >> 1));
+#pragma unroll
+  for (int j = 0; j < 8; ++j) s[j] = scale(((c0 + 64 * j) * 4) >> bs_log2);
+  const int sh = 16 * (lane & 1);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t w = p[j] >> sh;
+    f32x4 v;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = __fmul_rn(lut[(w >> (4 * k)) & 15u], s[j]);
+    __builtin_nontemporal_store(v, out + c0 + 64 * j);
+  }
+}
+
 template <int ODT, class Scale>
 __global__ __launch_bounds__(256) void nf4_dequant_generic(const uint8_t* __restrict__ packed, Scale scale,
                                                            int64_t bs, void* __restrict__ out,
@@ -719,13 +751,13 @@ extern "C" int rq_nf4_quantize(const void* w, int w_dtype, int64_t numel, int64_
 
 static int64_t dtype_bytes(int dt) { return dt == RQ_DTYPE_F32 ? 4 : 2; }
 
-// Runs nf4_dequant16_kernel over the whole workgroups that fit (1024 chunks
-// of 8 weights each) and returns the number of weights covered (0 when the
+// Runs nf4_dequant16_kernel (fp32 output: nf4_dequant32_kernel) over the whole
+// workgroups that fit (8192 weights each) and returns the number of weights covered (0 when the
 // call does not qualify); the rest goes through nf4_dequant_launch.
 template <class Scale>
-static int64_t nf4_dequant16_prefix(const uint8_t* packed, Scale scale, int64_t n_packed, int64_t bs,
+static int64_t nf4_dequant_prefix(const uint8_t* packed, Scale scale, int64_t n_packed, int64_t bs,
                                     void* out, int out_dtype, int64_t n_out, hipStream_t stream) {
-  if (out_dtype == RQ_DTYPE_F32 || bs < 16 || (bs & (bs - 1)) || !aligned(packed, 4) || !aligned(out, 16))
+  if (bs < 16 || (bs & (bs - 1)) || !aligned(packed, 4) || !aligned(out, 16))
     return 0;
   const int64_t chunks = n_packed / 4 < n_out / 8 ? n_packed / 4 : n_out / 8;
   const int64_t wgs = chunks / 1024;
@@ -735,6 +767,8 @@ static int64_t nf4_dequant16_prefix(const uint8_t* packed, Scale scale, int64_t 
   uint32_t* o = static_cast<uint32_t*>(out);
   if (out_dtype == RQ_DTYPE_BF16)
     nf4_dequant16_kernel<RQ_DTYPE_BF16, Scale><<<unsigned(wgs), 256, 0, stream>>>(p, scale, bs_log2, o);
+  else if (out_dtype == RQ_DTYPE_F32)
+    nf4_dequant32_kernel<Scale><<<unsigned(wgs), 256, 0, stream>>>(p, scale, bs_log2, static_cast<f32x4*>(out));
   else
     nf4_dequant16_kernel<RQ_DTYPE_F16, Scale><<<unsigned(wgs), 256, 0, stream>>>(p, scale, bs_log2, o);
   return wgs * 1024 * 8;
@@ -770,13 +804,13 @@ extern "C" int rq_nf4_dequantize(const uint8_t* packed, const void* absmax, int 
   int64_t done = 0;
   if (block_size <= 8192) {
     if (absmax_dtype == RQ_DTYPE_F32)
-      done = nf4_dequant16_prefix(packed, DqScaleAbs<RQ_DTYPE_F32>{absmax}, n_packed, block_size, out, out_dtype,
+      done = nf4_dequant_prefix(packed, DqScaleAbs<RQ_DTYPE_F32>{absmax}, n_packed, block_size, out, out_dtype,
                                   n_out, stream);
     else if (absmax_dtype == RQ_DTYPE_BF16)
-      done = nf4_dequant16_prefix(packed, DqScaleAbs<RQ_DTYPE_BF16>{absmax}, n_packed, block_size, out,
+      done = nf4_dequant_prefix(packed, DqScaleAbs<RQ_DTYPE_BF16>{absmax}, n_packed, block_size, out,
                                   out_dtype, n_out, stream);
     else
-      done = nf4_dequant16_prefix(packed, DqScaleAbs<RQ_DTYPE_F16>{absmax}, n_packed, block_size, out,
+      done = nf4_dequant_prefix(packed, DqScaleAbs<RQ_DTYPE_F16>{absmax}, n_packed, block_size, out,
                                   out_dtype, n_out, stream);
   }
   if (done == n_out) return rq_check_launch();
@@ -813,7 +847,7 @@ extern "C" int rq_dq_dequantize(const uint8_t* packed, const uint8_t* c2, int c2
   int64_t done = 0;
   if (block1 <= 8192 && (block2 & (block2 - 1)) == 0) {
     const int b2 = __builtin_ctzll(uint64_t(block2));
-    auto run = [&](auto sc) { return nf4_dequant16_prefix(packed, sc, n_packed, block1, out, out_dtype, n_out, stream); };
+    auto run = [&](auto sc) { return nf4_dequant_prefix(packed, sc, n_packed, block1, out, out_dtype, n_out, stream); };
     const bool fp8 = c2_format == RQ_C2_FP8_E4M3FNUZ;
     if (c2s_dtype == RQ_DTYPE_F32)
       done = fp8 ? run(DqScaleDouble<RQ_DTYPE_F32, RQ_C2_FP8_E4M3FNUZ>{c2, c2_scales, b2})
