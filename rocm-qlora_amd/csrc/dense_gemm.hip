@@ -12,6 +12,7 @@
 // activation rows, in the same issue slots and LDS as its MFMAs.
 #include "rq_dense_gemm.h"
 #include "rq_dense.h"
+#include "rq_pad.h"
 #include "rq_launch.h"
 
 #include <algorithm>
@@ -60,19 +61,7 @@ struct BlockOf {
   }
 };
 
-constexpr int kDecThreads = 256;
-
-// Eight values in the operand type at p (16-byte aligned): 16 or 32 bytes.
-template <int XT>
-__device__ __forceinline__ void store8(void* p, const float (&v)[8]) {
-  u32x4* o = static_cast<u32x4*>(p);
-  if constexpr (XT == RQ_DTYPE_F32) {
-    o[0] = u32x4{f2u(v[0]), f2u(v[1]), f2u(v[2]), f2u(v[3])};
-    o[1] = u32x4{f2u(v[4]), f2u(v[5]), f2u(v[6]), f2u(v[7])};
-  } else {
-    o[0] = u32x4{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3]), cvt_pk<XT>(v[4], v[5]), cvt_pk<XT>(v[6], v[7])};
-  }
-}
+constexpr int kDecThreads = kPadThreads;
 
 // one value in the operand type, as its storage word
 template <int XT>
@@ -89,8 +78,10 @@ __device__ __forceinline__ Word<XT> to_word(float v) {
 // MALL writes bound it (measured at 4096 x 14336: see launch_decode).
 template <int XT, class Src, class Scale>
 __global__ __launch_bounds__(kDecThreads) void decode_rows_kernel(Src src, Scale scale, BlockOf blk, uint32_t n_chunks,
-                                                                  uint32_t row_chunks, uint8_t* __restrict__ out) {
+                                                                  uint32_t row_chunks, uint8_t* __restrict__ out,
+                                                                  unsigned blocks, PadCopies pads) {
   __shared__ float lut[16];
+  if (blockIdx.x >= blocks) return pad_copy_block<XT>(pads, blockIdx.x - blocks);
   if (threadIdx.x < 16) lut[threadIdx.x] = u2f(kNF4Bits[threadIdx.x]);
   __syncthreads();
   const uint32_t c0 = blockIdx.x * (4 * kDecThreads) + threadIdx.x;
@@ -125,14 +116,17 @@ __global__ __launch_bounds__(kDecThreads) void decode_rows_kernel(Src src, Scale
 // row), which leaves as 128-byte runs of the output's rows.
 template <int XT, class Src, class Scale>
 __global__ __launch_bounds__(kDecThreads) void decode_cols_kernel(Src src, Scale scale, BlockOf blk, int64_t K,
-                                                                  int64_t ldo, uint8_t* __restrict__ out) {
+                                                                  int64_t ldo, uint8_t* __restrict__ out, unsigned gx,
+                                                                  unsigned blocks, PadCopies pads) {
   constexpr int ES = DnEl<XT>::kSize, kRow = 64 * ES;  // bytes of 64 rows' values of one column
   __shared__ float lut[16];
   __shared__ __attribute__((aligned(16))) uint8_t tile[256 * kRow];
+  if (blockIdx.x >= blocks) return pad_copy_block<XT>(pads, blockIdx.x - blocks);
+  const unsigned bx = blockIdx.x % gx, by = blockIdx.x / gx;
   const int t = threadIdx.x, p = t & 31;
   if (t < 16) lut[t] = u2f(kNF4Bits[t]);
   __syncthreads();
-  const int64_t n0 = int64_t(blockIdx.y) * 64, k0 = int64_t(blockIdx.x) * 256, kc = k0 + 32 * (t >> 5);
+  const int64_t n0 = int64_t(by) * 64, k0 = int64_t(bx) * 256, kc = k0 + 32 * (t >> 5);
   constexpr int kPieces = Src::kBytesPer8 / 4;  // 16-byte loads of 32 codes
   if (kc < K) {  // K is a multiple of 32: the thread's columns are all live
     u32x4 w[2][kPieces];
@@ -176,13 +170,16 @@ __global__ __launch_bounds__(kDecThreads) void decode_cols_kernel(Src src, Scale
 template <int XT, class Src, class Scale, bool TRANS>
 __global__ __launch_bounds__(kDecThreads) void decode_any_kernel(Src src, Scale scale, BlockOf blk, int64_t N,
                                                                  int64_t K, int64_t rows, int64_t ldo,
-                                                                 Word<XT>* __restrict__ out) {
+                                                                 Word<XT>* __restrict__ out, unsigned gx,
+                                                                 unsigned blocks, PadCopies pads) {
   __shared__ float lut[16];
   __shared__ Word<XT> tile[64][64 + 4 / sizeof(Word<XT>)];
+  if (blockIdx.x >= blocks) return pad_copy_block<XT>(pads, blockIdx.x - blocks);
+  const unsigned bx = blockIdx.x % gx, by = blockIdx.x / gx;
   const int t = threadIdx.x, c = t & 63;
   if (t < 16) lut[t] = u2f(kNF4Bits[t]);
   __syncthreads();
-  const int64_t k0 = int64_t(blockIdx.x) * 64, n0 = int64_t(blockIdx.y) * 64;
+  const int64_t k0 = int64_t(bx) * 64, n0 = int64_t(by) * 64;
 #pragma unroll 4
   for (int i = 0; i < 16; ++i) {
     const int r = 4 * i + (t >> 6);
@@ -200,54 +197,6 @@ __global__ __launch_bounds__(kDecThreads) void decode_any_kernel(Src src, Scale 
     const int r = 4 * i + (t >> 6);
     const int64_t row = (TRANS ? k0 : n0) + r, col = (TRANS ? n0 : k0) + c;
     if (row < rows && col < ldo) out[row * ldo + col] = TRANS ? tile[c][r] : tile[r][c];
-  }
-}
-
-// The small operands, one launch: `cnt` words zeroed, and up to four copies out[r][c] = RND(in[r * sr + c * sc]) with zeros past the source's
-// rows and columns -- the GEMM's second LoRA operand, and for reduction lengths
-// that are not whole k steps the activations, the LoRA input and the first
-// LoRA factor (fp32: always the first factor).
-struct PadCopy {
-  const void* in;
-  int dt;
-  int64_t sr, sc;
-  int64_t rows, cols;          // live part
-  int64_t out_rows, out_cols;  // out_cols a multiple of 8
-  void* out;
-  int64_t first;               // first workgroup
-};
-struct PadCopies {
-  PadCopy c[4];
-  int n;
-  uint32_t* cnt;
-  int n_cnt;
-};
-
-template <int XT>
-__global__ __launch_bounds__(kDecThreads) void pad_copy_kernel(PadCopies P) {
-  const int64_t g = blockIdx.x;
-  if (g == 0)
-    for (int i = threadIdx.x; i < P.n_cnt; i += kDecThreads) P.cnt[i] = 0u;
-  for (int i = 0; i < P.n; ++i) {
-    const PadCopy& c = P.c[i];
-    const int64_t per = c.out_cols / 8, groups = c.out_rows * per;
-    const int64_t idx = (g - c.first) * kDecThreads + threadIdx.x;
-    if (g < c.first || idx >= groups) continue;
-    // lanes run along the source's contiguous index
-    int64_t r, c8;
-    if (c.sc == 1) {
-      r = idx / per;
-      c8 = (idx - r * per) * 8;
-    } else {
-      const int64_t q = idx / c.out_rows;
-      r = idx - q * c.out_rows;
-      c8 = q * 8;
-    }
-    float v[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      v[e] = r < c.rows && c8 + e < c.cols ? load_as_f32(c.in, r * c.sr + (c8 + e) * c.sc, c.dt) : 0.0f;
-    store8<XT>(static_cast<uint8_t*>(c.out) + (r * c.out_cols + c8) * DnEl<XT>::kSize, v);
   }
 }
 
@@ -435,28 +384,38 @@ struct Product {
 
 template <int XT, class Src, class Scale>
 int launch_decode(Src src, Scale scale, int64_t N, int64_t K, int64_t bs, bool trans, int64_t Rp, void* w,
-                  hipStream_t stream) {
+                  const PadCopies& pads, hipStream_t stream) {
   uint8_t* const out = static_cast<uint8_t*>(w);
   const BlockOf blk{bs, bs > 0 ? pow2_shift(bs) : -1};
   const bool blocks_ok = bs == 0 || (blk.log2 >= 5 && K % bs == 0);
   const int64_t chunks = N * (K / 8);
+  // a linear grid: the decode's workgroups, then the copies'
+  auto grid = [&](int64_t gx, int64_t gy, unsigned* blocks) {
+    const int64_t n = gx * gy, all = n + pads.blocks();
+    if (all > int64_t(INT32_MAX)) return 0u;
+    *blocks = unsigned(n);
+    return unsigned(all);
+  };
+  unsigned blocks = 0, all = 0;
   if (!trans && K % 64 == 0 && blocks_ok && aligned(src.p, 8) && chunks < int64_t(UINT32_MAX) - 4096) {
-    decode_rows_kernel<XT, Src, Scale><<<unsigned(ceil_div(chunks, 4 * kDecThreads)), kDecThreads, 0, stream>>>(
-        src, scale, blk, uint32_t(chunks), uint32_t(K / 8), out);
-  } else if (trans && K % 64 == 0 && N % 64 == 0 && blocks_ok && aligned(src.p, 16) && N / 64 <= 65535) {
+    if (!(all = grid(ceil_div(chunks, 4 * kDecThreads), 1, &blocks))) return RQ_ERR_UNSUPPORTED;
+    decode_rows_kernel<XT, Src, Scale><<<all, kDecThreads, 0, stream>>>(src, scale, blk, uint32_t(chunks),
+                                                                        uint32_t(K / 8), out, blocks, pads);
+  } else if (trans && K % 64 == 0 && N % 64 == 0 && blocks_ok && aligned(src.p, 16)) {
+    const int64_t gx = ceil_div(K, 256);
+    if (!(all = grid(gx, N / 64, &blocks))) return RQ_ERR_UNSUPPORTED;
     decode_cols_kernel<XT, Src, Scale>
-        <<<dim3(unsigned(ceil_div(K, 256)), unsigned(N / 64)), kDecThreads, 0, stream>>>(src, scale, blk, K, Rp, out);
+        <<<all, kDecThreads, 0, stream>>>(src, scale, blk, K, Rp, out, unsigned(gx), blocks, pads);
   } else {
     // tiles over the output: its padded reduction index and its rows
-    const int64_t tk = ceil_div(trans ? K : Rp, 64), tn = ceil_div(trans ? Rp : N, 64);
-    if (tn > 65535) return RQ_ERR_UNSUPPORTED;
-    const dim3 grid{unsigned(tk), unsigned(tn)};
+    const int64_t gx = ceil_div(trans ? K : Rp, 64), gy = ceil_div(trans ? Rp : N, 64);
+    if (!(all = grid(gx, gy, &blocks))) return RQ_ERR_UNSUPPORTED;
     if (trans)
-      decode_any_kernel<XT, Src, Scale, true>
-          <<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, K, Rp, static_cast<Word<XT>*>(w));
+      decode_any_kernel<XT, Src, Scale, true><<<all, kDecThreads, 0, stream>>>(
+          src, scale, blk, N, K, K, Rp, static_cast<Word<XT>*>(w), unsigned(gx), blocks, pads);
     else
-      decode_any_kernel<XT, Src, Scale, false>
-          <<<grid, kDecThreads, 0, stream>>>(src, scale, blk, N, K, N, Rp, static_cast<Word<XT>*>(w));
+      decode_any_kernel<XT, Src, Scale, false><<<all, kDecThreads, 0, stream>>>(
+          src, scale, blk, N, K, N, Rp, static_cast<Word<XT>*>(w), unsigned(gx), blocks, pads);
   }
   return rq_check_launch();
 }
@@ -470,9 +429,6 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
   if (!aligned(scratch, 256)) return RQ_ERR_BAD_ALIGNMENT;
   char* ws = static_cast<char*>(scratch);
   uint32_t* cnt = reinterpret_cast<uint32_t*>(ws + p.cnt);
-  int st = decode(static_cast<void*>(ws + p.w), p.Rp);
-  if (st != RQ_OK) return st;
-
   DenseEpi e = P.e;
   DenseGemmArgs a{};
   a.x = P.x;
@@ -484,12 +440,9 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
   int s_dt = P.lora_dt;
 
   PadCopies pc{};
-  int64_t groups = 0;
   auto copy = [&](const void* in, int dt, int64_t sr, int64_t sc, int64_t rows, int64_t cols, int64_t out_rows,
                   int64_t out_cols, size_t off) -> const void* {
-    pc.c[pc.n++] = PadCopy{in, dt, sr, sc, rows, cols, out_rows, out_cols, ws + off, groups};
-    groups += ceil_div(out_rows * (out_cols / 8), kDecThreads);
-    return ws + off;
+    return pc.add(in, dt, sr, sc, rows, cols, out_rows, out_cols, ws + off);
   };
   if (P.rank > 0) {
     e.rankp = int(p.rankp);
@@ -515,11 +468,9 @@ int run_product(const Product& P, const Decode& decode, void* scratch, size_t by
     pc.cnt = cnt;
     pc.n_cnt = p.tiles_m * p.tiles_n - p.whole;
   }
-  if (pc.n > 0 || pc.n_cnt > 0) {
-    if (groups > int64_t(INT32_MAX)) return RQ_ERR_UNSUPPORTED;
-    pad_copy_kernel<XT><<<unsigned(std::max<int64_t>(groups, 1)), kDecThreads, 0, stream>>>(pc);
-    if ((st = rq_check_launch()) != RQ_OK) return st;
-  }
+  // one launch decodes the weight and makes the copies
+  int st = decode(static_cast<void*>(ws + p.w), p.Rp, pc);
+  if (st != RQ_OK) return st;
   if (P.rank > 0 && !P.u) {
     float* lpart = reinterpret_cast<float*>(ws + p.lpart);
     if constexpr (kF32) {
@@ -586,8 +537,8 @@ int run_weight(const Product& P, const Src& src, const WithScale& with_scale, in
                bool trans, void* scratch, size_t bytes, hipStream_t stream) {
   return run_product<XT>(
       P,
-      [&](void* w, int64_t Rp) {
-        return with_scale([&](auto sc) { return launch_decode<XT>(src, sc, N, K, bs, trans, Rp, w, stream); });
+      [&](void* w, int64_t Rp, const PadCopies& pads) {
+        return with_scale([&](auto sc) { return launch_decode<XT>(src, sc, N, K, bs, trans, Rp, w, pads, stream); });
       },
       scratch, bytes, stream);
 }

@@ -22,6 +22,7 @@
 #include "rq_linear.h"
 #include "rq_linear_dev.h"
 #include "rq_lora.h"
+#include "rq_pad.h"
 
 #include <algorithm>
 
@@ -218,13 +219,21 @@ __global__ __launch_bounds__(256) void lora_grad_finish_kernel(GradOut o0, GradO
 }
 
 // out[m][j] = RND(sum of the K splits' partials in order) (j < R, zeros to
-// R16) when given, and outt[j][m], zeros for M <= m < Mp.  A thread takes 8
-// rows of one rank.
+// R16) when given, and outt[j][m], zeros for M <= m < Mp, for one or two operands
+// in one launch.  A thread takes 8 rows of one rank, four splits in flight.
+struct FinishT {
+  const float* part;
+  int splits;
+  uint16_t* out;
+  uint16_t* outt;
+};
+
 template <int XT>
-__global__ __launch_bounds__(256) void lora_finish_t_kernel(const float* __restrict__ part, int KS, int64_t M, int R,
-                                                            int R16, int64_t Mp, uint16_t* __restrict__ out,
-                                                            uint16_t* __restrict__ outt) {
-  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void lora_finish_t_kernel(FinishT f0, FinishT f1, unsigned first1, int64_t M, int R,
+                                                            int R16, int64_t Mp) {
+  const bool second = blockIdx.x >= first1;
+  const FinishT& f = second ? f1 : f0;
+  const int64_t i = int64_t(blockIdx.x - (second ? first1 : 0u)) * 256 + threadIdx.x;
   const int64_t m8 = i / R16;
   const int j = int(i - m8 * R16);
   if (8 * m8 >= Mp) return;
@@ -232,15 +241,20 @@ __global__ __launch_bounds__(256) void lora_finish_t_kernel(const float* __restr
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = 0.0f;
   if (j < R) {
-    for (int k = 0; k < KS; ++k) {
-      float p[8];
+    for (int k0 = 0; k0 < f.splits; k0 += 4) {
+      float p[4][8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int64_t m = 8 * m8 + e;
-        p[e] = part[(int64_t(k) * M + (m < M ? m : M - 1)) * R + j];
-      }
+      for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = __fadd_rn(v[e], p[e]);
+        for (int e = 0; e < 8; ++e) {
+          const int64_t m = 8 * m8 + e;
+          p[k][e] = f.part[(int64_t(k0 + k < f.splits ? k0 + k : 0) * M + (m < M ? m : M - 1)) * R + j];
+        }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (k0 + k < f.splits) v[e] = __fadd_rn(v[e], p[k][e]);
     }
   }
   uint32_t w[4];
@@ -249,28 +263,17 @@ __global__ __launch_bounds__(256) void lora_finish_t_kernel(const float* __restr
     const float a = 8 * m8 + 2 * e < M ? v[2 * e] : 0.0f, b = 8 * m8 + 2 * e + 1 < M ? v[2 * e + 1] : 0.0f;
     w[e] = cvt_pk<XT>(a, b);
   }
-  *reinterpret_cast<u32x4*>(outt + int64_t(j) * Mp + 8 * m8) = u32x4{w[0], w[1], w[2], w[3]};
-  if (out) {
+  *reinterpret_cast<u32x4*>(f.outt + int64_t(j) * Mp + 8 * m8) = u32x4{w[0], w[1], w[2], w[3]};
+  if (f.out) {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      if (8 * m8 + e < M) out[(8 * m8 + e) * R16 + j] = uint16_t(w[e >> 1] >> (16 * (e & 1)));
+      if (8 * m8 + e < M) f.out[(8 * m8 + e) * R16 + j] = uint16_t(w[e >> 1] >> (16 * (e & 1)));
   }
 }
 
-// out[r][c] = RND(in[r * sr + c * sc]), zeros past rows x cols; 8 columns per
-// thread, lanes along the source's contiguous index.
 template <int XT>
-__global__ __launch_bounds__(256) void pad16_kernel(const void* __restrict__ in, int dt, int64_t sr, int64_t sc,
-                                                    int64_t rows, int64_t cols, int64_t out_rows, int64_t out_cols,
-                                                    uint16_t* __restrict__ out) {
-  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x, per = out_cols / 8;
-  if (i >= out_rows * per) return;
-  const int64_t r = sc == 1 ? i / per : i % out_rows, c = 8 * (sc == 1 ? i % per : i / out_rows);
-  float v[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = r < rows && c + e < cols ? load_as_f32(in, r * sr + (c + e) * sc, dt) : 0.0f;
-  *reinterpret_cast<u32x4*>(out + r * out_cols + c) =
-      u32x4{cvt_pk<XT>(v[0], v[1]), cvt_pk<XT>(v[2], v[3]), cvt_pk<XT>(v[4], v[5]), cvt_pk<XT>(v[6], v[7])};
+__global__ __launch_bounds__(kPadThreads) void pad_copy_kernel(PadCopies P) {
+  pad_copy_block<XT>(P, blockIdx.x);
 }
 
 size_t up(size_t b) { return (b + 255) & ~size_t(255); }
@@ -282,7 +285,7 @@ struct GradPlan {
   LoraRowsPlan lu, lg;
   int splits;
   int64_t rows_per_split;
-  size_t lpart, s, ut, gt, x, y, pa, pb, a, bytes;
+  size_t lu_part, lg_part, s, ut, gt, x, y, pa, pb, a, bytes;
 };
 
 GradPlan plan_grads(int64_t M, int64_t K, int64_t N, int64_t rank, int cus) {
@@ -310,7 +313,8 @@ GradPlan plan_grads(int64_t M, int64_t K, int64_t N, int64_t rank, int cus) {
     off += up(b);
     return o;
   };
-  p.lpart = take(std::max(p.lu.part_bytes, p.lg.part_bytes));
+  p.lu_part = take(p.lu.part_bytes);
+  p.lg_part = take(p.lg.part_bytes);
   p.s = take(size_t(rank) * p.Np * 2);   // RND(B)^T rows
   p.a = p.pad_x ? take(size_t(rank) * p.Kp * 2) : 0;
   // operand rows for every rank block, written up to r16
@@ -349,53 +353,51 @@ int run_grads(const GradCall& C, void* scratch, size_t bytes, hipStream_t stream
   auto at16 = [&](size_t o) { return reinterpret_cast<uint16_t*>(ws + o); };
   auto atf = [&](size_t o) { return reinterpret_cast<float*>(ws + o); };
   int st = RQ_OK;
-  auto pad = [&](const void* in, int dt, int64_t sr, int64_t sc, int64_t rows, int64_t cols, int64_t out_cols,
-                 uint16_t* out) {
-    const int64_t groups = ceil_div(rows * (out_cols / 8), 256);
-    pad16_kernel<XT><<<unsigned(groups), 256, 0, stream>>>(in, dt, sr, sc, rows, cols, rows, out_cols, out);
-    return rq_check_launch();
-  };
   const uint16_t* x = static_cast<const uint16_t*>(C.x);
   const uint16_t* dy = static_cast<const uint16_t*>(C.dy);
   int64_t ldx = C.ldx, lddy = C.lddy;
+  const bool need_g = C.da || C.g, need_u = C.db != nullptr;
+  const void* sa = C.a;
+  int sa_dt = C.lora_dt;
+  int64_t sa_j = C.K;
+  PadCopies pc{};
   if (p.pad_x) {
-    if ((st = pad(C.x, XT, C.ldx, 1, C.M, C.K, p.Kp, at16(p.x))) != RQ_OK) return st;
-    x = at16(p.x);
+    x = static_cast<const uint16_t*>(pc.add(C.x, XT, C.ldx, 1, C.M, C.K, C.M, p.Kp, ws + p.x));
     ldx = p.Kp;
+    if (need_u) {
+      sa = pc.add(C.a, C.lora_dt, C.K, 1, C.rank, C.K, C.rank, p.Kp, ws + p.a);
+      sa_dt = XT;
+      sa_j = p.Kp;
+    }
   }
   if (p.pad_y) {
-    if ((st = pad(C.dy, XT, C.lddy, 1, C.M, C.N, p.Np, at16(p.y))) != RQ_OK) return st;
-    dy = at16(p.y);
+    dy = static_cast<const uint16_t*>(pc.add(C.dy, XT, C.lddy, 1, C.M, C.N, C.M, p.Np, ws + p.y));
     lddy = p.Np;
   }
-  auto finish_t = [&](const LoraRowsPlan& lp, uint16_t* out, uint16_t* outt) {
-    const unsigned blocks = unsigned(ceil_div((p.Mp / 8) * p.r16, 256));
-    lora_finish_t_kernel<XT><<<blocks, 256, 0, stream>>>(atf(p.lpart), lp.splits, C.M, C.rank, int(p.r16), p.Mp, out,
-                                                        outt);
-    return rq_check_launch();
-  };
-  if (C.da || C.g) {
-    // g = RND(dv . RND(B)): S[j][n] = B[n][j] as contiguous 16-bit rows
-    if ((st = pad(C.b, C.lora_dt, 1, C.ldb, C.rank, C.N, p.Np, at16(p.s))) != RQ_OK) return st;
+  // g's factor S[j][n] = B[n][j] as contiguous 16-bit rows
+  if (need_g) pc.add(C.b, C.lora_dt, 1, C.ldb, C.rank, C.N, C.rank, p.Np, ws + p.s);
+  if (pc.blocks() > int64_t(INT32_MAX)) return RQ_ERR_UNSUPPORTED;
+  if (pc.n > 0) {
+    pad_copy_kernel<XT><<<unsigned(pc.blocks()), kPadThreads, 0, stream>>>(pc);
+    if ((st = rq_check_launch()) != RQ_OK) return st;
+  }
+  FinishT f[2] = {};
+  int nf = 0;
+  if (need_g) {
     st = run_lora_rows_parts(XT, dy, lddy, C.M, p.Np, at16(p.s), XT, p.Np, 1, C.rank, true, C.scale, p.lg,
-                             atf(p.lpart), stream);
+                             atf(p.lg_part), stream);
     if (st != RQ_OK) return st;
-    if ((st = finish_t(p.lg, C.g, at16(p.gt))) != RQ_OK) return st;
+    f[nf++] = FinishT{atf(p.lg_part), p.lg.splits, C.g, at16(p.gt)};
   }
-  if (C.db) {
-    const void* s = C.a;
-    int dt = C.lora_dt;
-    int64_t sj = C.K;
-    if (p.pad_x) {
-      if ((st = pad(C.a, C.lora_dt, C.K, 1, C.rank, C.K, p.Kp, at16(p.a))) != RQ_OK) return st;
-      s = at16(p.a);
-      dt = XT;
-      sj = p.Kp;
-    }
-    st = run_lora_rows_parts(XT, x, ldx, C.M, p.Kp, s, dt, sj, 1, C.rank, false, 1.0f, p.lu, atf(p.lpart), stream);
+  if (need_u) {
+    st = run_lora_rows_parts(XT, x, ldx, C.M, p.Kp, sa, sa_dt, sa_j, 1, C.rank, false, 1.0f, p.lu, atf(p.lu_part),
+                             stream);
     if (st != RQ_OK) return st;
-    if ((st = finish_t(p.lu, nullptr, at16(p.ut))) != RQ_OK) return st;
+    f[nf++] = FinishT{atf(p.lu_part), p.lu.splits, nullptr, at16(p.ut)};
   }
+  const unsigned fb = unsigned(ceil_div((p.Mp / 8) * p.r16, 256));
+  lora_finish_t_kernel<XT><<<fb * nf, 256, 0, stream>>>(f[0], f[1], fb, C.M, C.rank, int(p.r16), p.Mp);
+  if ((st = rq_check_launch()) != RQ_OK) return st;
   if (!C.da && !C.db) return RQ_OK;
   GradArgs a{};
   a.M = C.M;
@@ -445,6 +447,7 @@ extern "C" int rq_lora_grads(const void* x, int x_dtype, int64_t M, int64_t K, i
   if (lora_dtype != RQ_DTYPE_F32 && lora_dtype != x_dtype) return RQ_ERR_BAD_DTYPE;
   if (M < 1 || K < 1 || N < 1 || rank < 1 || ldx < K || lddy < N || ld_lora_b < rank) return RQ_ERR_BAD_SHAPE;
   if (rank > 64) return RQ_ERR_UNSUPPORTED;
+  if (!da && !db && !g) return RQ_OK;
   if (!x || !dy || !lora_a || !lora_b) return RQ_ERR_NULL_POINTER;
   if (!rq::aligned(x, 2) || !rq::aligned(dy, 2)) return RQ_ERR_BAD_ALIGNMENT;
   if ((K % 64 == 0 && (!rq::aligned(x, 16) || ldx % 8 != 0)) ||
