@@ -53,6 +53,12 @@ struct SkArgs {
   int groups, splits, nseg;
   float* part;
   uint32_t* cnt;
+  // the LoRA operand inside the launch (la set): this split's part of x . RND(A)^T,
+  // summed over the workgroup's waves and stored to upart [groups][splits][rank
+  // blocks of 16][16][16 MB rows]; A [rank][K], rows 16-byte aligned
+  const void* la;
+  int la_dt;
+  float* upart;
 };
 
 struct SkEpi {
@@ -142,6 +148,25 @@ void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
   // the activation loads are older than the U * kLoads weight loads
   step_barrier<U * Unit::kLoads>();
 
+  // LoRA operand: the split's 32-k steps t = wave, wave + 16, ...; the first rank
+  // block's values of A are requested here, under the units
+  constexpr int kUSteps = U / 2;
+  const int rank = e.rank, nsteps = 8 * nu;
+  u32x4 a_lo[kUSteps], a_hi[kUSteps];
+  auto a_load = [&](int jb) {
+#pragma unroll
+    for (int t = 0; t < kUSteps; ++t) {
+      const int j = 16 * jb + i16;
+      int64_t k = kbeg + 32 * (wave + kSkWaves * t) + 8 * q;
+      k = k < a.K ? k : a.K - 8;
+      const int64_t off = int64_t(j < rank ? j : rank - 1) * a.K + k;
+      const uint8_t* p = static_cast<const uint8_t*>(a.la) + off * (a.la_dt == RQ_DTYPE_F32 ? 4 : 2);
+      a_lo[t] = *reinterpret_cast<const u32x4*>(p);
+      a_hi[t] = *reinterpret_cast<const u32x4*>(p + (a.la_dt == RQ_DTYPE_F32 ? 16 : 0));
+    }
+  };
+  if (a.la) a_load(0);
+
   f32x4 acc[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -174,6 +199,86 @@ void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
     }
   }
 
+  // ---- this split's part of u: every workgroup of a column group needs all of u
+  // at its end, so each computes it for its own K split beside its tiles, and the
+  // split exchange below carries it (a launch of its own before this one took 4.5
+  // us and a gap, and its partials 2 us of the epilogue)
+  float* const up = a.upart + (int64_t(group) * a.splits + split) * (((rank + 15) / 16) * 16 * kXRows);
+  if (a.la) {
+    f32x4* red = reinterpret_cast<f32x4*>(lds);  // [16 waves][MB][64 lanes], over the table
+    static_assert(kSkWaves * 4 * 64 * 16 <= kLutBytes, "u reduction");
+    for (int jb = 0; 16 * jb < rank; ++jb) {
+      if (jb > 0) a_load(jb);
+      f32x4 ua[MB];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) ua[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < kUSteps; ++t) {
+        const int st = wave + kSkWaves * t;
+        if (st < nsteps) {
+          const bool live = kbeg + 32 * st + 8 * q < a.K;
+          u32x4 av = raw8_to_x<XT>(a_lo[t], a_hi[t], a.la_dt);
+          const uint8_t* xp = xs + (st >> 1) * kPiece + i16 * 128 + (((4 * (st & 1) + q) ^ ((i16 >> 1) & 7)) << 4);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) av[c] = live ? av[c] : 0u;
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) {
+            u32x4 xv = *reinterpret_cast<const u32x4*>(xp + mb * 2048);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) xv[c] = live ? xv[c] : 0u;
+            ua[mb] = mfma16x16x32<XT>(av, xv, ua[mb]);
+          }
+        }
+      }
+      __syncthreads();  // the table (or the last block's sums) is no longer read
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) red[(wave * MB + mb) * 64 + lane] = ua[mb];
+      __syncthreads();
+      // value (rank 4 q + r, row 16 mb + i) of lane (i, q): summed in wave order
+      for (int idx = tid; idx < 256 * MB; idx += kSkThreads) {
+        const float* r = reinterpret_cast<const float*>(red) + idx;
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kSkWaves; ++w) v = __fadd_rn(v, r[w * 256 * MB]);
+        const int mb = idx >> 8, l = (idx >> 2) & 63, j = 16 * jb + 4 * (l >> 4) + (idx & 3);
+        __hip_atomic_store(&up[j * kXRows + 16 * mb + (l & 15)], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  }
+
+  // The epilogue's first operands, requested before the splits' tiles so that the
+  // round trips overlap: up to 16 parts of the thread's first u value and the
+  // first 8 ranks of its column's B row, raw.  In-launch u: the splits' parts, rows
+  // contiguous; else the row kernel's partials, ranks contiguous.
+  const int r16 = (rank + 15) / 16 * 16, live = r16 * kXRows;
+  const int64_t ustep = a.la ? int64_t(live) : a.M * rank;
+  const int ns = a.la ? a.splits : e.u_splits;
+  auto u_index = [&](int idx, int& j, int& m) {
+    const bool rows = a.la || idx >= live;
+    j = rows ? idx / kXRows : idx % r16;
+    m = rows ? idx % kXRows : idx / r16;
+    return j < rank && m < a.M;
+  };
+  auto u_load = [&](float (&t)[16], int idx, int j, int m, int s0) {
+    const float* p = a.la ? a.upart + int64_t(group) * ns * live + idx : e.u + m * rank + j;
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      if (s0 + s < ns) t[s] = __hip_atomic_load(p + int64_t(s0 + s) * ustep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  float ut[16];
+  u32x4 b_lo = {0u, 0u, 0u, 0u}, b_hi = {0u, 0u, 0u, 0u};
+  const bool b_pre = e.b_vec && 8 * q + 8 <= rank && (e.b_dt == RQ_DTYPE_F32 || e.ldb % 8 == 0);
+  auto pre_load = [&]() {
+    if (rank <= 0) return;
+    int j, m;
+    if (tid < kXRows * 64 && u_index(tid, j, m)) u_load(ut, tid, j, m, 0);
+    if (b_pre) {
+      const uint8_t* p = static_cast<const uint8_t*>(e.b) + (n * e.ldb + 8 * q) * (e.b_dt == RQ_DTYPE_F32 ? 4 : 2);
+      b_lo = *reinterpret_cast<const u32x4*>(p);
+      b_hi = *reinterpret_cast<const u32x4*>(p + (e.b_dt == RQ_DTYPE_F32 ? 16 : 0));
+    }
+  };
+
   if (a.splits > 1) {
     // tile (16 rows of this wave) x split: MB x 64 lanes x 16 bytes
     uint8_t* base = reinterpret_cast<uint8_t*>(a.part) + (int64_t(group) * kSkWaves + wave) * a.splits * (MB * 1024);
@@ -197,16 +302,18 @@ void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
     if (!last) return;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < a.splits; s0 += 4) {  // four splits' tiles in flight
-      u32x4 v[4][MB];
+    pre_load();
+    constexpr int kFly = MB == 4 ? 4 : (MB == 3 ? 5 : 8);  // splits' tiles in flight
+    for (int s0 = 0; s0 < a.splits; s0 += kFly) {
+      u32x4 v[kFly][MB];
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int s = 0; s < kFly; ++s)
+        if (s0 + s < a.splits)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-          v[s][mb] = buf_load16_coherent(part, uint32_t(lane) * 16u,
-                                         uint32_t(((s0 + s < a.splits ? s0 + s : 0) * MB + mb) * 1024));
+          for (int mb = 0; mb < MB; ++mb)
+            v[s][mb] = buf_load16_coherent(part, uint32_t(lane) * 16u, uint32_t(((s0 + s) * MB + mb) * 1024));
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int s = 0; s < kFly; ++s)
         if (s0 + s < a.splits)
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb)
@@ -214,29 +321,27 @@ void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
             for (int r = 0; r < 4; ++r) acc[mb][r] = __fadd_rn(acc[mb][r], u2f(v[s][mb][r]));
     }
   } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // u's stores, read below by other waves
     __syncthreads();  // the activations' and table's LDS is free
+    pre_load();
   }
 
   // ---- epilogue: acc[mb][r] of lane (i, q) is row 16 mb + i, column n0 +
   // 4 q + r
-  const int rank = e.rank;
   f32x4 lo[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) lo[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (rank > 0) {
     uint16_t* us = reinterpret_cast<uint16_t*>(lds);  // RND(u) [16 MB][kSkUPitch], zero padded to 64 ranks
     for (int idx = tid; idx < kXRows * 64; idx += kSkThreads) {
-      const int m = idx >> 6, j = idx & 63;
+      int j, m;
       float v = 0.0f;
-      if (j < rank && m < a.M) {
-        const float* p = e.u + (m) * rank + j;
-        for (int s0 = 0; s0 < e.u_splits; s0 += 8) {
-          float t[8];
+      if (u_index(idx, j, m)) {
+        for (int s0 = 0; s0 < ns; s0 += 16) {
+          if (idx != tid || s0 > 0) u_load(ut, idx, j, m, s0);
 #pragma unroll
-          for (int s = 0; s < 8; ++s) t[s] = p[int64_t(s0 + s < e.u_splits ? s0 + s : 0) * a.M * rank];
-#pragma unroll
-          for (int s = 0; s < 8; ++s)
-            if (s0 + s < e.u_splits) v = __fadd_rn(v, t[s]);
+          for (int s = 0; s < 16; ++s)
+            if (s0 + s < ns) v = __fadd_rn(v, ut[s]);
         }
       }
       us[m * kSkUPitch + j] = uint16_t(to_x16<XT>(v));
@@ -244,8 +349,9 @@ void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
     __syncthreads();
     for (int j0 = 0; j0 < rank; j0 += 32) {
       const int left = rank - j0 - 8 * q;
-      const u32x4 bv = left > 0 ? load_a8_masked<XT>(e.b, e.b_dt, n * e.ldb + j0 + 8 * q, left, e.b_vec)
-                                : u32x4{0u, 0u, 0u, 0u};
+      u32x4 bv = {0u, 0u, 0u, 0u};
+      if (j0 == 0 && b_pre) bv = raw8_to_x<XT>(b_lo, b_hi, e.b_dt);
+      else if (left > 0) bv = load_a8_masked<XT>(e.b, e.b_dt, n * e.ldb + j0 + 8 * q, left, e.b_vec);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
         lo[mb] = mfma16x16x32<XT>(
@@ -284,7 +390,7 @@ void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
 struct SkPlan {
   int mb, units, groups, nseg, splits;
   LoraRowsPlan lr;
-  size_t part_off, bytes;
+  size_t part_off, u_off, bytes;
 };
 
 SkPlan plan_skinny(int64_t M, int64_t N, int64_t K, int64_t rank, int cus) {
@@ -303,8 +409,10 @@ SkPlan plan_skinny(int64_t M, int64_t N, int64_t K, int64_t rank, int cus) {
     p.lr = plan_lora_rows(M, K, rank, cus);
     p.part_off = p.lr.part_bytes;
   }
-  p.bytes = p.part_off;
-  if (p.splits > 1) p.bytes += size_t(p.groups) * kSkWaves * p.splits * p.mb * 1024;
+  p.u_off = p.part_off;
+  if (p.splits > 1) p.u_off += size_t(p.groups) * kSkWaves * p.splits * p.mb * 1024;
+  p.bytes = p.u_off;
+  if (rank > 0) p.bytes += size_t(p.groups) * p.splits * (ceil_div(rank, 16) * 16) * (16 * p.mb) * 4;
   return p;
 }
 
@@ -381,13 +489,16 @@ int run_skinny_nf4(const LinearArgs& L, void* workspace, size_t bytes, uint32_t*
   const SkPlan p = plan_skinny(L.M, L.N, L.K, L.rank, device_cus());
   if (p.bytes > 0 && (!workspace || bytes < p.bytes || !aligned(workspace, 256))) return RQ_ERR_WORKSPACE;
   SkEpi e{};
+  bool u_in = false;
   e.bias = L.bias;
   e.bias_dt = L.bias_dtype;
   e.y = static_cast<uint16_t*>(L.y);
   e.ldy = L.ldy;
   if (L.rank > 0) {
     float* u = static_cast<float*>(workspace);
-    const int st = run_lora_rows_parts(L.x_dtype, static_cast<const uint16_t*>(L.lora_x), L.ld_lora_x, L.M, L.K,
+    // the operand inside the launch when the adapter reads x itself
+    u_in = L.lora_x == L.x && L.ld_lora_x == L.ldx && aligned(L.lora_a, 16);
+    const int st = u_in ? RQ_OK : run_lora_rows_parts(L.x_dtype, static_cast<const uint16_t*>(L.lora_x), L.ld_lora_x, L.M, L.K,
                                        L.lora_a, L.lora_dtype, L.K, 1, int(L.rank), false, 1.0f, p.lr, u, stream);
     if (st != RQ_OK) return st;
     e.rank = int(L.rank);
@@ -399,7 +510,12 @@ int run_skinny_nf4(const LinearArgs& L, void* workspace, size_t bytes, uint32_t*
     e.b_vec = aligned(L.lora_b, 16) && (L.lora_dtype != RQ_DTYPE_F32 || L.ld_lora_b % 4 == 0);
     e.scaling = L.scaling;
   }
-  const SkArgs a = sk_args(p, L.x, L.ldx, L.w_packed, L.M, L.N, L.K, L.K / 2, L.block_size, workspace, cnt);
+  SkArgs a = sk_args(p, L.x, L.ldx, L.w_packed, L.M, L.N, L.K, L.K / 2, L.block_size, workspace, cnt);
+  if (u_in) {
+    a.la = L.lora_a;
+    a.la_dt = L.lora_dtype;
+    a.upart = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.u_off);
+  }
   return L.x_dtype == RQ_DTYPE_BF16
              ? launch_scale<RQ_DTYPE_BF16, UnitNF4>(a, L.absmax, L.absmax_dtype, L.c2, L.c2_format, L.block2, e, p,
                                                     stream)
