@@ -101,8 +101,10 @@ class FP8LinearWrapper(nn.Module):
             bias = ql.bias.to(x.dtype) if ql.bias is not None else None
             qw = ql.nf4_weight() if ql.bits == 4 else ql.int8_weight()
             lora = self.base
-            if dm.native_adapter(x, lora.lora_A) and type(lora.lora_dropout) in (nn.Dropout, nn.Identity):
-                p = lora.lora_dropout.p if lora._dropout_active() else 0.0
+            drop = lora.lora_dropout
+            if dm.native_adapter(x, lora.lora_A) and type(drop) in (nn.Dropout, nn.Identity) and \
+                    not (drop._forward_hooks or drop._forward_pre_hooks or drop._backward_hooks):
+                p = drop.p if drop.training and isinstance(drop, nn.Dropout) else 0.0
 
                 def base_dx(dy, A, B, s, g, mask, mask_scale):
                     if g is None:

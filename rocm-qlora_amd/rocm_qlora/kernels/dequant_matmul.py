@@ -110,8 +110,10 @@ def _lora_backward(dy, x, A, B, s, need_a, need_b, need_g):
     dv = dY * s, dB = dv^T (x A^T), dA = (dv B)^T x; and dv B (None where the
     torch path runs), which dX's LoRA term starts from.  The HIP kernels run in
     eager first-order backward passes; tracing, create_graph (whose result is
-    differentiated again), fp32 and ranks past 64 run on torch."""
+    differentiated again), forward-mode AD and batched gradients
+    (is_grads_batched: dy without storage), fp32 and ranks past 64 run on torch."""
     if not torch_ops.compiling() and not torch.is_grad_enabled() and dy.dtype == x.dtype and \
+            not _functorch_active() and forward_ad._current_level < 0 and torch._C._has_storage(dy) and \
             ops.lora_grads_supported(x, A):
         return ops.lora_grads(x, dy, A, B, s, need_a, need_b, need_g)
     da = db = None
@@ -189,9 +191,11 @@ class _FusedInt8LinearFunc(torch.autograd.Function):
 
 def native_adapter(x, lora_a) -> bool:
     """Whether the adapter of an INT8 or FP8 layer runs on the LoRA kernels, both
-    ways (eager, 16-bit activations, K a multiple of 64, rank <= 64)."""
+    ways (eager, 16-bit activations, K a multiple of 64, rank <= 64, no autocast
+    to another dtype, which torch's products would follow)."""
     return not torch_ops.compiling() and not _functorch_active() and forward_ad._current_level < 0 and \
-        ops.lora_add_supported(x, lora_a) and ops.lora_grads_supported(x, lora_a)
+        ops.lora_grads_supported(x, lora_a) and ops.lora_add_supported(x, lora_a) and \
+        (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype)
 
 
 class _BaseLoRALinearFunc(torch.autograd.Function):
@@ -208,14 +212,18 @@ class _BaseLoRALinearFunc(torch.autograd.Function):
             xl, mask = torch.ops.aten.native_dropout(x, float(dropout_p), True)
         ctx.base_dx = base_dx
         ctx.scaling = float(scaling)
-        ctx.mask_scale = 1.0 / (1.0 - dropout_p) if mask is not None else 1.0
-        ctx.save_for_backward(xl, lora_a, lora_b, mask)
+        ctx.mask_scale = (1.0 / (1.0 - dropout_p) if dropout_p < 1.0 else 0.0) if mask is not None else 1.0
+        ctx.save_for_backward(x, xl if mask is not None else None, lora_a, lora_b, mask)
         return ops.lora_add_(base(x), xl, lora_a, lora_b, scaling)
 
     @staticmethod
     def backward(ctx, dy):
-        xl, A, B, mask = ctx.saved_tensors
+        x, xl, A, B, mask = ctx.saved_tensors
         need_x, need_a, need_b = ctx.needs_input_grad[:3]
+        if mask is None:
+            xl = x
+        elif torch.is_grad_enabled():  # create_graph: drop(x) as a function of x
+            xl = x * (mask.to(x.dtype) * ctx.mask_scale)
         da, db, g = _lora_backward(dy, xl, A, B, ctx.scaling, need_a, need_b, need_x)
         dx = ctx.base_dx(dy, A, B, ctx.scaling, g, mask, ctx.mask_scale) if need_x else None
         return dx, da, db, None, None, None, None

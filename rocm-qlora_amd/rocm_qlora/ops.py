@@ -173,6 +173,15 @@ def _scratch(size_fn: str, dev, *args) -> Optional[torch.Tensor]:
     return torch.empty(n, dtype=torch.uint8, device=dev) if n else None
 
 
+def _spare(size_fn: str, dev, *args) -> Optional[torch.Tensor]:
+    """_scratch for a call that also runs without it: None on a GPU whose memory
+    is too full for the decoded weight."""
+    try:
+        return _scratch(size_fn, dev, *args)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optional[torch.Tensor],
                out_features: int, block_size: int = 64, bias: Optional[torch.Tensor] = None, *,
                c2: Optional[torch.Tensor] = None, c2_scales: Optional[torch.Tensor] = None,
@@ -243,7 +252,7 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
         b = bias.contiguous() if bias is not None else None
         scratch = None
         if (M > GEMV_MAX_M or not fast_shape) and max(ldx, ldxl) * M * x.element_size() < 1 << 32:
-            scratch = _scratch("rq_nf4_linear_scratch_size", dev, xcode, M, K, N, block_size, rank)
+            scratch = _spare("rq_nf4_linear_scratch_size", dev, xcode, M, K, N, block_size, rank)
         # a call with scratch memory needs no workspace of its own
         ws = _workspace(x.dtype, M, K, N, rank, dev) if scratch is None else None
         codes = c2.reshape(-1).view(torch.uint8).contiguous() if dq else None
@@ -316,7 +325,7 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
         code = nat.dtype_code(dy.dtype)
         scratch = ws = None
         if lddy * M * dy.element_size() < 1 << 32:
-            scratch = _scratch("rq_nf4_linear_dx_scratch_size", dev, code, M, N, K, block_size, rank)
+            scratch = _spare("rq_nf4_linear_dx_scratch_size", dev, code, M, N, K, block_size, rank)
         if scratch is None:
             ws = _scratch("rq_nf4_linear_dx_workspace_size", dev, code, M, N, K, rank)
         codes = c2.reshape(-1).view(torch.uint8).contiguous() if dq else None
@@ -405,7 +414,7 @@ def int8_linear(x: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, out_feat
         if M == 0:
             return y.reshape(*lead, N)
         b = bias.contiguous() if bias is not None else None
-        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(x.dtype), M, K, N, block_size, 0, 0)
+        scratch = _spare("rq_int8_linear_scratch_size", dev, nat.dtype_code(x.dtype), M, K, N, block_size, 0, 0)
         nat.call("rq_int8_linear_scratch", x2.data_ptr(), nat.dtype_code(x.dtype), M, K, ldx,
                  qf.data_ptr(), N, block_size, sc.data_ptr(), nat.dtype_code(sc.dtype),
                  nat.ptr(b), nat.dtype_code(b.dtype) if b is not None else 0,
@@ -451,7 +460,7 @@ def int8_linear_dx(dy: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, in_f
             lcode = nat.dtype_code(la.dtype)
             if lora_mask is not None:
                 mk, ldm = _rows(lora_mask.reshape(-1, K).view(torch.uint8), K)
-        scratch = _scratch("rq_int8_linear_scratch_size", dev, nat.dtype_code(dy.dtype), M, K, N, block_size, 1, rank)
+        scratch = _spare("rq_int8_linear_scratch_size", dev, nat.dtype_code(dy.dtype), M, K, N, block_size, 1, rank)
         if rank and (scratch is None or lddy * M * dy.element_size() >= 1 << 32):
             # past the dense kernel's 32-bit offsets: the adapter's term by torch
             t = lora_g[:, :rank] @ lora_a.to(dy.dtype)

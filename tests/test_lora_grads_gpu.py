@@ -120,3 +120,65 @@ def test_byte_layers_with_adapter(dev, kind, p, M):
         assert a.dtype == b.dtype and a.shape == b.shape
         d, f = (a.float() - b.float()).abs(), b.float()
         assert bool((d <= 2.0 ** -7 * (f.abs() + f.square().mean().sqrt())).all()), (name, float(d.max()))
+
+
+def _int8_layer(dev, K, N, r, dropout):
+    from rocm_qlora import LoRALinear, QuantLinear
+    g = torch.Generator().manual_seed(9)
+    lin = torch.nn.Linear(K, N, bias=False)
+    with torch.no_grad():
+        lin.weight.copy_(torch.randn(N, K, generator=g) * 0.02)
+    layer = LoRALinear(QuantLinear.from_linear(lin.to(dev), bits=8), r=r, lora_alpha=2 * r, lora_dropout=dropout).to(dev)
+    with torch.no_grad():
+        layer.lora_B.copy_(torch.randn(N, r, generator=g) * 0.1)
+    return layer.train()
+
+
+@pytest.mark.parametrize("p", [0.0, 0.5, 1.0])
+def test_int8_second_derivative_through_dropout(dev, p):
+    """dA = s (dY B)^T drop(x) differentiated again: d<dA, V>/dx = s (dY B) V times
+    the dropout mask.  Bound: four bf16 roundings."""
+    K, N, r, M = 128, 192, 8, 40
+    layer = _int8_layer(dev, K, N, r, p)
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn(M, K, generator=g).bfloat16().to(dev).requires_grad_()
+    dy = torch.randn(M, N, generator=g).bfloat16().to(dev)
+    v = torch.randn(r, K, generator=g).to(dev)
+    torch.manual_seed(5)
+    y = layer(x)
+    torch.manual_seed(5)
+    keep = torch.nn.functional.dropout(torch.ones_like(x), p, True) if p else torch.ones_like(x)
+    (da,) = torch.autograd.grad(y, layer.lora_A, dy, create_graph=True)
+    (gx,) = torch.autograd.grad((da * v).sum(), x)
+    ref = (layer.scaling * (dy.float() @ layer.lora_B.float()) @ v) * keep.float()
+    assert (gx.float() - ref).norm() <= 4 * 2.0 ** -9 * ref.norm()
+
+
+def test_linears_without_room_for_the_decoded_weight(dev, monkeypatch):
+    """A GPU too full for the decoded weight: the other route's results, which
+    differ from the dense route's by the order of fp32 sums (one bf16 rounding of
+    each value, and one of the adapter's intermediates)."""
+    layer = _int8_layer(dev, 256, 320, 16, 0.0)
+    from rocm_qlora.quantization import quantize_int4
+    g = torch.Generator().manual_seed(2)
+    w = (torch.randn(1000, 333, generator=g) * 0.02).to(dev)
+    packed, absmax = quantize_int4(w, 64)
+    x, x4 = torch.randn(70, 256, generator=g).bfloat16().to(dev).requires_grad_(), torch.randn(70, 333, generator=g).bfloat16().to(dev)
+    dy, dy4 = torch.randn(70, 320, generator=g).bfloat16().to(dev), torch.randn(70, 1000, generator=g).bfloat16().to(dev)
+
+    def call():
+        y = layer(x)
+        return (y.detach(), torch.autograd.grad(y, x, dy)[0], ops.nf4_linear(x4, packed, absmax, 1000, 64),
+                ops.nf4_linear_dx(dy4, packed, absmax, 333, 64))
+
+    ref = call()
+    real = ops._scratch
+
+    def full(size_fn, d, *args):
+        if size_fn.endswith("linear_scratch_size") or size_fn.endswith("linear_dx_scratch_size"):
+            raise torch.OutOfMemoryError("full")
+        return real(size_fn, d, *args)
+
+    monkeypatch.setattr(ops, "_scratch", full)
+    for a, b in zip(call(), ref):
+        assert (a.float() - b.float()).norm() <= 3 * 2.0 ** -9 * b.float().norm()
