@@ -184,6 +184,155 @@ __global__ __launch_bounds__(64 * kByteGvWaves) void byte_gemv_kernel(ByteGemvAr
 }
 
 // ---------------------------------------------------------------------------
+// byte_gemv_kernel's work for more tiles than compute units: one workgroup per
+// compute unit takes tiles blockIdx.x, + gridDim.x, ..., the activations in LDS
+// once (rows padded so that the 16 rows' reads fall on distinct banks), and a
+// wave's chunks over all its tiles form one sequence whose weights are three
+// chunks ahead in registers, so the stream does not stop between tiles or at
+// their reductions (one workgroup of 16 waves fits a compute unit either way:
+// a launch of one tile per workgroup drained and refilled it seven times at
+// 8192 -> 28672: 3.5 TB/s from HBM, 4.5 streamed; still bound by the weight stream
+// and its decode, about 2.5 VALU operations a byte).  The sums and their order are byte_gemv_kernel's, hence the
+// bits.  Rows i >= M read row 0: their products go to output rows that are never
+// stored.  ROW: one scale per weight row, loaded once a chunk.
+// ---------------------------------------------------------------------------
+constexpr int kByteStRed = 2 * kByteGvWaves * 64 * 16;  // two tiles' wave sums
+constexpr int kByteStLds = 160 * 1024;
+constexpr int kByteStOut = 8 * 1024;                    // the workgroup's outputs, fp32 [tile][row][16]
+constexpr int kByteStX = kByteStLds - kByteStRed - kByteStOut;  // activations
+// bytes of an activation row in LDS: whole 1 KiB loads with at least 64 zeros past
+// K (what pieces past K multiply), and 16 bytes of pad
+__host__ __device__ inline int64_t byte_st_pitch(int64_t K) { return (K + 64 + 511) / 512 * 1024 + 16; }
+
+template <class Scale, bool ROW>
+struct ByteUnit {
+  u32x4 w[kByteGvPieces];
+  typename Scale::Raw s[ROW ? 1 : kByteGvPieces];
+};
+
+template <int XT, class Scale, bool ROW>
+__global__ __launch_bounds__(64 * kByteGvWaves) void byte_gemv_stream_kernel(ByteGemvArgs a, Scale scale, int tiles,
+                                                                             int per_wave) {
+  using Unit = ByteUnit<Scale, ROW>;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kByteStLds];
+  f32x4* red = reinterpret_cast<f32x4*>(lds);
+  float* outs = reinterpret_cast<float*>(lds + kByteStRed);
+  constexpr int kXs = kByteStRed + kByteStOut;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i16 = lane & 15, g4 = lane >> 4;
+  const int M = int(a.M);
+  const uint32_t K = uint32_t(a.K);
+  const uint32_t pitch = uint32_t(byte_st_pitch(a.K));
+  // activations: 512 k of a row per load, lanes past K a live address
+  {
+    const int per_row = int((a.K + 511) / 512);
+    for (int t = wave; t < int(a.M) * per_row; t += kByteGvWaves) {
+      const int r = t / per_row, p = t - r * per_row;
+      uint32_t k = uint32_t(p) * 512u + uint32_t(lane) * 8u;
+      k = k < K ? k : K - 8u;
+      dma16(a.x, (uint32_t(r) * uint32_t(a.ldx) + k) * 2u,
+            __builtin_amdgcn_readfirstlane(uint32_t(kXs) + uint32_t(r) * pitch + uint32_t(p) * 1024u));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(a.w, uint32_t(a.N * a.K));
+  const int nt = (tiles - int(blockIdx.x) + int(gridDim.x) - 1) / int(gridDim.x);  // this workgroup's tiles
+  const int units = nt * per_wave;
+  int it = 0, ij = 0;  // the next unit to request: tile, chunk
+  auto issue = [&](Unit& u) {
+    int64_t n = (int64_t(blockIdx.x) + int64_t(it) * gridDim.x) * 16 + i16;
+    n = n < a.N ? n : a.N - 1;  // rows past N re-read a live row; never stored
+    const uint32_t kb = uint32_t(wave + kByteGvWaves * ij) * kByteGvChunk;
+    const uint32_t row = uint32_t(n) * K + 16u * uint32_t(g4);
+    const int64_t sb = n * a.blocks_per_row;
+    if constexpr (ROW) u.s[0] = scale.load(n);
+#pragma unroll
+    for (int t = 0; t < kByteGvPieces; ++t) {
+      const uint32_t k = kb + 64u * t;
+      // pieces past K and units past the last: a load that returns zeros
+      u.w[t] = buf_load16(wrs, it < nt && k < K ? row + k : kOobOffset);
+      if constexpr (!ROW) u.s[t] = scale.load(sb + ((k < K ? k : 0u) >> a.bs_log2));
+    }
+    if (++ij == per_wave) {
+      ij = 0;
+      ++it;
+    }
+    asm volatile("" ::: "memory");  // no load shared between units: the wait below counts them
+  };
+  Unit u0, u1, u2;
+  issue(u0);
+  issue(u1);
+  issue(u2);
+  __builtin_amdgcn_sched_barrier(0);
+  step_barrier<3 * kByteGvPieces>();  // the activations are older than the weights
+  {
+    const uint32_t tail = (pitch - 16u) / 16u - K / 8u;  // 16-byte pieces past K of a row
+    for (uint32_t i = tid; i < uint32_t(M) * tail; i += 64 * kByteGvWaves)
+      *reinterpret_cast<u32x4*>(lds + kXs + (i / tail) * pitch + 2u * K + 16u * (i % tail)) = u32x4{0u, 0u, 0u, 0u};
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  const uint8_t* xr = lds + kXs + (i16 < M ? uint32_t(i16) * pitch : 0u) + 32 * g4;
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  int ct = 0, cj = 0;  // the unit to compute
+  auto step = [&](Unit& u) {
+    const uint32_t kb = uint32_t(wave + kByteGvWaves * cj) * kByteGvChunk;
+#pragma unroll
+    for (int t = 0; t < kByteGvPieces; ++t) {
+      // no branch, also past K: the compiler's waits then leave the later units in flight
+      const uint32_t k = kb + 64u * t, kx = k < K ? k : K;
+      const float s = k < K ? scale.value(u.s[ROW ? 0 : t]) : 0.0f;
+      const u32x4 x0 = *reinterpret_cast<const u32x4*>(xr + 2u * kx);
+      const u32x4 x1 = *reinterpret_cast<const u32x4*>(xr + 2u * kx + 16);
+      const uint2 p0 = decode4_pk<XT>(u.w[t].x, s), p1 = decode4_pk<XT>(u.w[t].y, s);
+      const uint2 p2 = decode4_pk<XT>(u.w[t].z, s), p3 = decode4_pk<XT>(u.w[t].w, s);
+      acc = mfma16x16x32<XT>(x0, u32x4{p0.x, p0.y, p1.x, p1.y}, acc);
+      acc = mfma16x16x32<XT>(x1, u32x4{p2.x, p2.y, p3.x, p3.y}, acc);
+    }
+    issue(u);
+    if (++cj < per_wave) return;
+    // the tile's sums: one of two LDS areas, so that one barrier a tile is
+    // enough; wave ct % 16 adds them in wave order
+    f32x4* rd = red + (ct & 1) * kByteGvWaves * 64;
+    rd[wave * 64 + lane] = acc;
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (wave == (ct & (kByteGvWaves - 1))) {
+      f32x4 sum = rd[lane];
+#pragma unroll 3
+      for (int w = 1; w < kByteGvWaves; ++w) {  // few at a time: the units hold most registers
+        const f32x4 v = rd[w * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] = __fadd_rn(sum[r], v[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * g4 + r < M) outs[(ct * M + 4 * g4 + r) * 16 + i16] = sum[r];
+    }
+    cj = 0;
+    ++ct;
+  };
+  int u = 0;  // the same count in every wave; no exit inside the loop, as above
+  for (; u + 3 <= units; u += 3) {
+    step(u0);
+    step(u1);
+    step(u2);
+  }
+  if (u < units) step(u0);
+  if (u + 1 < units) step(u1);
+  __syncthreads();
+  for (int i = tid; i < nt * M * 16; i += 64 * kByteGvWaves) {
+    const int t = i / (16 * M), m = (i >> 4) - t * M;
+    const int64_t n = (int64_t(blockIdx.x) + int64_t(t) * gridDim.x) * 16 + (i & 15);
+    if (n >= a.N) continue;
+    float v = outs[i];
+    if (a.bias) v = __fadd_rn(v, round_x<XT>(load_as_f32(a.bias, n, a.bias_dt)));
+    a.y[m * a.ldy + n] = uint16_t(to_x16<XT>(round_x<XT>(v)));
+  }
+}
+
+// ---------------------------------------------------------------------------
 // FP8 per-tensor quantization (fp8_linear.py:37-42): absmax over the whole
 // tensor (two deterministic max passes), s = fp32(double(absmax) / 240),
 // code = fnuz(RND_dt(float(t) / s)) with the division in fp32 and RND_dt the
@@ -310,6 +459,28 @@ static int launch_byte(const ByteLinearArgs& A, Scale scale, hipStream_t stream)
     g.blocks_per_row = bpr; g.bs_log2 = bsl;
     g.bias = A.bias; g.bias_dt = A.bias_dtype;
     g.y = static_cast<uint16_t*>(A.y); g.ldy = A.ldy;
+    // Tiles streamed through persistent workgroups: more than three 256-k chunks a
+    // wave, K long enough for most waves to have one, activations that fit the LDS.
+    // One tile a workgroup against streamed, us, weights past the MALL (row scales
+    // unless said): 8192 -> 28672 M = 1 67.7 / 52.2 and M = 6 72.2 / 51.1, 4096 ->
+    // 28672 35.5 / 29.4, 2048 -> 28672 M = 12 27.7 / 20.3, 4096 -> 14336 blocks of 64
+    // 24.5 / 22.2 (M = 8 29.6 / 24.1); on the line 4096 -> 12288 16.7 / 17.2; beyond it
+    // 4096 -> 4608 12.8 / 14.0, 2048 -> 14336 blocks of 64 15.4 / 19.5, 1024 -> 28672
+    // blocks of 64 17.4 / 25.6.
+    const int64_t tiles = (A.N + 15) / 16;
+    const int cus = device_cus();
+    if (double(tiles) * double(A.K) > 3.0 * cus * kByteGvChunk * kByteGvWaves && A.K >= (A.block_size ? 3072 : 2048) &&
+        tiles > cus && A.M * byte_st_pitch(A.K) <= kByteStX &&
+        ceil_div(tiles, int64_t(cus)) * A.M * 64 <= kByteStOut && double(A.N) * double(A.K) <= double(kOobOffset)) {
+      const int per_wave = int(ceil_div(A.K, int64_t(kByteGvChunk) * kByteGvWaves));
+      if (A.block_size == 0)
+        byte_gemv_stream_kernel<XT, Scale, true>
+            <<<unsigned(cus), 64 * kByteGvWaves, 0, stream>>>(g, scale, int(tiles), per_wave);
+      else
+        byte_gemv_stream_kernel<XT, Scale, false>
+            <<<unsigned(cus), 64 * kByteGvWaves, 0, stream>>>(g, scale, int(tiles), per_wave);
+      return rq_check_launch();
+    }
     byte_gemv_kernel<XT, Scale><<<unsigned((A.N + 15) / 16), 64 * kByteGvWaves, 0, stream>>>(g, scale);
     return rq_check_launch();
   }

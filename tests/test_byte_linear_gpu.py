@@ -210,3 +210,30 @@ def test_fp8_short_and_ragged_k(dev, M, K):
     wc, ws = ops.fp8_quantize(w.to(dev))
     y = ops.fp8_linear(x.to(dev), wc, ws, bias.to(dev))
     _check(y, R.fp8_linear(x, w, bias))
+
+
+@pytest.mark.parametrize("M,K,N,block", [
+    (1, 8192, 6161, 0), (3, 4160, 12200, 64), (16, 3072, 16500, 64), (7, 2048, 25000, 0), (2, 2112, 24100, 0),
+    (5, 8256, 6300, 0), (13, 4096, 12400, 128), (16, 4096, 12400, 0), (1, 2048, 50001, 0), (1, 4096, 12288, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_int8_gemv_streamed_tiles(dev, M, K, N, block, dtype):
+    """Weights of more than three chunks a wave (50 M codes on 256 compute units, and
+    one just under): a last tile of one row, uneven tile counts, K that ends inside
+    a wave's chunk, one to three chunks a wave, activations that fit the LDS and
+    that do not.  The sums are the one-tile kernel's in the same order, so pieces
+    of the weight, which run there, give the same bits."""
+    print(f"int8 gemv stream {M} {K} {N} {block} {dtype}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    q = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device="cuda")
+    sc = torch.rand((N, K // block if block else 1), generator=g, device="cuda") * 0.01
+    bias = torch.randn(N, generator=g, device="cuda").to(dtype)
+    got = ops.int8_linear(x, q, sc, N, block, bias)
+    parts = [ops.int8_linear(x, q[i:i + 4096], sc[i:i + 4096], q[i:i + 4096].shape[0], block, bias[i:i + 4096])
+             for i in range(0, N, 4096)]
+    assert torch.equal(got, torch.cat(parts, 1))
+    w = (q.float().view(N, -1, block or K) * sc.view(N, -1, 1)).view(N, K).to(dtype).double()
+    ref = x.double() @ w.T + bias.double()
+    tol = 2.0 ** (-9 if dtype == torch.bfloat16 else -12) + 1e-5  # one rounding, and fp32 sums
+    assert (got.double() - ref).norm() <= tol * ref.norm()
