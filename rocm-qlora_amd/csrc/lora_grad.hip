@@ -16,7 +16,8 @@
 // whole 256-byte row pieces per instruction.  A wave covers 128 columns x 32
 // rows per step with 8 x (r / 16) MFMAs.  Bound by reading dY and x: at M =
 // 4096, K = 4096, N = 14336, r = 64 the library GEMMs, the dY * s pass and the
-// casts it replaces took 182 us.
+// casts it replaces took 182 us; now g 46 us, u 16 us, their finish 14 us and this
+// kernel 69 us (2.2 TB/s with 64 ranks; 8 ranks at M = 1500, K = 11008: 12 us).
 #include "rq_mfma.h"
 #include "rq_launch.h"
 #include "rq_linear.h"

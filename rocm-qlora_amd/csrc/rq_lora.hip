@@ -190,7 +190,8 @@ __global__ __launch_bounds__(256) void lora_finish_kernel(const float* __restric
 // FP8).  A workgroup takes 32 rows x 256 columns, a wave 64 of the columns as
 // 16x16x32 MFMAs with B's rows as the A operand (a lane's four results along a
 // row); the terms go through LDS so that y moves in whole 512-byte row pieces.
-// Bound by reading and writing y (512 x 28672: see rq_lora_add).
+// Bound by reading and writing y (512 x 28672: 16.6 us, 3.5 TB/s; the products,
+// multiply, add and casts of the torch expression took 64 us with its GEMMs).
 constexpr int kAddRows = 32, kAddCols = 256, kAddPitch = kAddCols + 8;
 
 template <int XT>
