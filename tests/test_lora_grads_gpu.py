@@ -42,6 +42,34 @@ def test_lora_grads(dev, M, K, N, rank, dtype, lora32):
     assert not gg[:, rank:].any()
 
 
+@pytest.mark.parametrize("M,K,N,rank,dtype", [(4096, 4096, 14336, 64, "bf16"), (2048, 1024, 4096, 64, "fp16"),
+                                              (333, 1000, 1501, 12, "bf16"), (1024, 4096, 4096, 16, "bf16")])
+def test_lora_grads_exact_sums(dev, M, K, N, rank, dtype):
+    """Small whole numbers, whose sums are exact in fp32 in any order: every bit
+    equals the torch expressions of the adapter's gradients in float64 with one
+    rounding to the activation dtype after each of them, so rounding points and
+    widths are theirs and other inputs can differ by the order of the sums alone.
+    (|u|, |g| stay near 2^8 to 2^10, past bf16's 8 bits, and the last sums below
+    2^24.)"""
+    print(f"lora grads, exact sums {M} {K} {N} {rank} {dtype}", flush=True)
+    dt = DT[dtype]
+    g = torch.Generator(device=dev).manual_seed(M + rank)
+
+    def ints(lo, hi, *shape):
+        return torch.randint(lo, hi + 1, shape, generator=g, device=dev).float()
+
+    big = 4 if dtype == "bf16" else 2  # fp16: the sums stay below its largest value
+    x, dy = ints(-1, 1, M, K).to(dt), ints(-1, 1, M, N).to(dt)
+    a, b, s = ints(-big, big, rank, K), ints(-big, big, N, rank), 0.5
+    da, db, gg = ops.lora_grads(x, dy, a, b, s, True, True, True)
+    dv = (dy.double() * s).to(dt).double()
+    u, gv = (x.double() @ a.double().T).to(dt).double(), (dv @ b.double()).to(dt).double()
+    sa, sb = gv.T @ x.double(), dv.T @ u
+    assert max(float(t.abs().max()) for t in (sa, sb)) < 2.0 ** 24 and float(u.abs().max()) > 2 ** 7
+    assert torch.equal(gg[:, :rank].double(), gv) and not gg[:, rank:].any()
+    assert torch.equal(da, sa.to(dt).float()) and torch.equal(db, sb.to(dt).float())
+
+
 def test_lora_grads_strided_and_partial(dev):
     """Strided rows (16-byte aligned and not) give the same bits as packed
     ones, and each gradient alone the same as all together."""
