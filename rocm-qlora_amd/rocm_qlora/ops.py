@@ -267,6 +267,25 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
     return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
 
 
+def _check_lora_g(lora_g: torch.Tensor, M: int, rank: int, dtype: torch.dtype) -> None:
+    """Raise unless lora_g is what lora_grads returns for M rows of dtype and this
+    rank: the dX kernels read [M, rank rounded up to 16] values behind its pointer."""
+    if rank == 0:
+        raise RuntimeError("lora_g without the adapter's factors")
+    if dtype == torch.float32 or lora_g.dtype != dtype or lora_g.shape != (M, -(-rank // 16) * 16) or \
+            not lora_g.is_contiguous():
+        raise RuntimeError(f"lora_g {tuple(lora_g.shape)} {lora_g.dtype} (contiguous: {lora_g.is_contiguous()}) is not "
+                           f"lora_grads' operand of {M} rows, rank {rank}, {dtype} (16-bit only)")
+
+
+def _mask_rows(lora_mask: torch.Tensor, M: int, K: int, dev: torch.device) -> Tuple[torch.Tensor, int]:
+    """The dropout mask's M rows of K bytes, and their stride."""
+    mk, ldm = _rows(lora_mask.reshape(-1, K).view(torch.uint8), K)
+    if mk.shape[0] != M or mk.device != dev:
+        raise RuntimeError(f"lora_mask has {mk.shape[0]} rows on {mk.device}, dY {M} on {dev}")
+    return mk, ldm
+
+
 def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optional[torch.Tensor],
                   in_features: int, block_size: int = 64, *,
                   c2: Optional[torch.Tensor] = None, c2_scales: Optional[torch.Tensor] = None,
@@ -279,14 +298,14 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
     differentiated).  With lora_mask (the dropout mask of the adapter's input,
     [..., K] bool), the LoRA term goes through dropout's backward: times
     mask * mask_scale.  lora_g: the adapter's (dY * s) . B as lora_grads returns
-    it, when the caller has it.  dy: [..., N] fp32/bf16/fp16 on the GPU; output
+    it (16-bit dY), when the caller has it.  dy: [..., N] fp32/bf16/fp16 on the GPU; output
     [..., K] in dy's dtype.  Shapes outside the MFMA dX kernel's (N or K not
     multiples of 64, other block sizes, fp32 dy) run on the generic kernels."""
     N = dy.shape[-1]
     K = int(in_features)
     dq = c2 is not None
     scales = c2_scales if dq else weight_scales
-    dev = nat.require_gpu(dy, weight_quant, scales, lora_a, lora_b, c2)
+    dev = nat.require_gpu(dy, weight_quant, scales, lora_a, lora_b, c2, lora_g)
     if weight_quant.dtype != torch.uint8:
         raise TypeError(f"NF4 weight_quant must be uint8, got {weight_quant.dtype}")
     if weight_quant.numel() * 2 < N * K:
@@ -319,9 +338,9 @@ def nf4_linear_dx(dy: torch.Tensor, weight_quant: torch.Tensor, weight_scales: O
             lcode = nat.dtype_code(la.dtype)
         mk, ldm = None, 0
         if rank > 0 and lora_mask is not None:
-            mk, ldm = _rows(lora_mask.reshape(-1, K).view(torch.uint8), K)
-            if mk.shape[0] != M:
-                raise RuntimeError(f"lora_mask has {mk.shape[0]} rows, dY {M}")
+            mk, ldm = _mask_rows(lora_mask, M, K, dev)
+        if lora_g is not None:
+            _check_lora_g(lora_g, M, rank, dy.dtype)
         code = nat.dtype_code(dy.dtype)
         scratch = ws = None
         if lddy * M * dy.element_size() < 1 << 32:
@@ -453,13 +472,14 @@ def int8_linear_dx(dy: torch.Tensor, q: torch.Tensor, scales: torch.Tensor, in_f
             return dx.reshape(*dy.shape[:-1], K)
         rank, la, lcode, mk, ldm = 0, None, 0, None, 0
         if lora_g is not None:
-            rank = lora_a.shape[0]
-            if lora_a.shape[1] != K or lora_g.shape != (M, -(-rank // 16) * 16) or lora_g.dtype != dy.dtype:
-                raise RuntimeError(f"LoRA shapes {tuple(lora_a.shape)} / {tuple(lora_g.shape)} do not fit {M}x{K}")
+            rank = lora_a.shape[0] if lora_a is not None else 0
+            _check_lora_g(lora_g, M, rank, dy.dtype)
+            if lora_a.shape[1] != K:
+                raise RuntimeError(f"lora_a {tuple(lora_a.shape)} does not fit {M}x{K}")
             la = (lora_a if lora_a.dtype in (torch.float32, dy.dtype) else lora_a.float()).contiguous()
             lcode = nat.dtype_code(la.dtype)
             if lora_mask is not None:
-                mk, ldm = _rows(lora_mask.reshape(-1, K).view(torch.uint8), K)
+                mk, ldm = _mask_rows(lora_mask, M, K, dev)
         scratch = _spare("rq_int8_linear_scratch_size", dev, nat.dtype_code(dy.dtype), M, K, N, block_size, 1, rank)
         if rank and (scratch is None or lddy * M * dy.element_size() >= 1 << 32):
             # past the dense kernel's 32-bit offsets: the adapter's term by torch
