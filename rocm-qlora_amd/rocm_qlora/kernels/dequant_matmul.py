@@ -96,6 +96,16 @@ class Int8Weight:
         return w.reshape(-1)[:n].view(self.N, self.K).to(dtype)
 
 
+_functorch_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: True)
+
+
+def _plain_eager() -> bool:
+    """Whether the call runs as it stands: no tracing (torch.compile,
+    torch.jit.trace), functorch transform or forward-mode AD active."""
+    return not torch_ops.compiling() and not torch._C._is_tracing() and not _functorch_active() and \
+        forward_ad._current_level < 0
+
+
 def _lora_present(lora_a, lora_b) -> bool:
     return lora_a is not None and lora_b is not None and lora_a.shape[0] > 0
 
@@ -112,8 +122,7 @@ def _lora_backward(dy, x, A, B, s, need_a, need_b, need_g):
     eager first-order backward passes; tracing, create_graph (whose result is
     differentiated again), forward-mode AD and batched gradients
     (is_grads_batched: dy without storage), fp32 and ranks past 64 run on torch."""
-    if not torch_ops.compiling() and not torch.is_grad_enabled() and dy.dtype == x.dtype and \
-            not _functorch_active() and forward_ad._current_level < 0 and torch._C._has_storage(dy) and \
+    if _plain_eager() and not torch.is_grad_enabled() and dy.dtype == x.dtype and torch._C._has_storage(dy) and \
             ops.lora_grads_supported(x, A):
         return ops.lora_grads(x, dy, A, B, s, need_a, need_b, need_g)
     da = db = None
@@ -193,8 +202,7 @@ def native_adapter(x, lora_a) -> bool:
     """Whether the adapter of an INT8 or FP8 layer runs on the LoRA kernels, both
     ways (eager, 16-bit activations, K a multiple of 64, rank <= 64, no autocast
     to another dtype, which torch's products would follow)."""
-    return not torch_ops.compiling() and not _functorch_active() and forward_ad._current_level < 0 and \
-        ops.lora_grads_supported(x, lora_a) and ops.lora_add_supported(x, lora_a) and \
+    return _plain_eager() and ops.lora_grads_supported(x, lora_a) and ops.lora_add_supported(x, lora_a) and \
         (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype)
 
 
@@ -272,9 +280,6 @@ def composed_dx(dx, dy, A, B, s, mask, mask_scale):
     return dx + (t * (mask.to(dt) * mask_scale) if mask is not None else t)
 
 
-_functorch_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: True)
-
-
 def _nothing_recorded(*inputs) -> bool:
     """Whether autograd records nothing for an op on these inputs, so that the
     forward can run without its autograd function: no gradient asked for, and
@@ -282,7 +287,7 @@ def _nothing_recorded(*inputs) -> bool:
     through the function, which accepts or refuses them)."""
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs):
         return False
-    return not torch_ops.compiling() and not _functorch_active() and forward_ad._current_level < 0
+    return _plain_eager()
 
 
 def nf4_linear(x: torch.Tensor, w: NF4Weight, bias: Optional[torch.Tensor] = None,

@@ -427,6 +427,24 @@ def test_custom_operators_opcheck(dev):
                           (dy, p, s, K, 64, None, None, 256, True, a, b, 2.0, None, 1.0))
 
 
+@pytest.mark.parametrize("kind", ["nf4", "nf4_lora", "int8", "int8_lora", "fp8_lora"])
+def test_jit_trace_is_refused(dev, kind):
+    """torch.jit.trace cannot run the layers' autograd functions without their
+    Python weights: it raises, also where no gradient is recorded, rather than
+    return a module whose output nothing fills."""
+    from rocm_qlora.fp8 import FP8LinearWrapper
+    layer = QuantLinear.from_linear(nn.Linear(128, 64).to(dev), bits=8 if kind.startswith("int8") else 4)
+    if kind.endswith("lora"):
+        layer = LoRALinear(layer, r=8, lora_alpha=16).to(dev)
+    if kind.startswith("fp8"):
+        layer = FP8LinearWrapper(layer)
+    x = torch.randn(5, 128, device=dev, dtype=torch.bfloat16)
+    with torch.no_grad():
+        layer(x)
+        with pytest.raises(RuntimeError):
+            torch.jit.trace(layer, x, check_trace=False)
+
+
 def test_torch_compile_without_graph_breaks(dev):
     """LoRALinear(QuantLinear) under torch.compile (fullgraph: no graph break
     at the HIP calls; AOT autograd traces the backward through the dX

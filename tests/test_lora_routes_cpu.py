@@ -1,6 +1,8 @@
 """The adapters' gradients where the HIP kernels cannot run: batched output
 gradients (torch.autograd.grad(is_grads_batched=True), tensors without storage)
-and forward-mode AD take the torch expressions, on any device."""
+and forward-mode AD take the torch expressions, on any device; and calls inside
+torch.jit.trace keep their autograd functions, without which the trace would hold
+an output allocation and nothing that fills it."""
 import pytest
 import torch
 from torch.autograd import forward_ad
@@ -49,3 +51,17 @@ def test_forward_mode_gradients(kernels_refused):
     x, a, b, dys = _inputs()
     with forward_ad.dual_level(), torch.no_grad():
         dm._lora_backward(dys[0], x, a, b, 2.0, True, True, False)
+
+
+def test_calls_inside_jit_trace_keep_their_autograd_function():
+    x, a = torch.zeros(5, 64).bfloat16(), torch.zeros(8, 64)
+    seen = []
+
+    def f(t):
+        seen.append((dm._nothing_recorded(t), dm.native_adapter(t, a)))
+        return t + 1
+
+    with torch.no_grad():
+        f(x)
+        torch.jit.trace(f, (x,), check_trace=False)
+    assert seen == [(True, True), (False, False)]
