@@ -249,6 +249,8 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
             lcode = nat.dtype_code(la.dtype)
             if lora_x is not None:
                 xl, ldxl = (_aligned_rows if wide else _rows)(lora_x.to(x.dtype), K)
+                if xl.shape[0] != M or xl.device != dev:
+                    raise RuntimeError(f"lora_x has {xl.shape[0]} rows on {xl.device}, x {M} on {dev}")
         b = bias.contiguous() if bias is not None else None
         scratch = None
         if (M > GEMV_MAX_M or not fast_shape) and max(ldx, ldxl) * M * x.element_size() < 1 << 32:

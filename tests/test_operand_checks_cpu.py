@@ -1,5 +1,5 @@
-"""Operands that the dX kernels read by pointer (the adapter's (dY s) . B and the
-dropout mask): a wrong shape, dtype, layout or device raises on the host, before
+"""Operands that the kernels read by pointer (dX: the adapter's (dY s) . B and the
+dropout mask; the forward: the adapter's own input): a wrong shape, dtype, layout or device raises on the host, before
 any library call.  The library is replaced, so no GPU is needed."""
 import contextlib
 
@@ -31,6 +31,7 @@ def no_library(monkeypatch):
     monkeypatch.setattr(nat, "call", call)
     monkeypatch.setattr(nat, "stream_handle", lambda dev: 0)
     monkeypatch.setattr(ops, "on", lambda dev: contextlib.nullcontext())
+    monkeypatch.setattr(ops, "_workspace", lambda *args: None)
     monkeypatch.setattr(ops, "_bytes", lambda fn, dev, *args: 64)
 
 
@@ -82,3 +83,13 @@ def test_lora_g_without_adapters_raises(no_library, fn):
 def test_wrong_lora_mask_raises(no_library, fn, bad):
     with pytest.raises(RuntimeError):
         fn(**_adapter(lora_g=_g(), lora_mask=bad))
+
+
+@pytest.mark.parametrize("bad", [torch.zeros(M - 1, K), torch.zeros(2 * M, K), torch.zeros(M, K, device="meta")],
+                         ids=["short", "long", "device"])
+def test_wrong_lora_x_raises(no_library, bad):
+    x, packed, s = torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(N * K // 2, dtype=torch.uint8), torch.ones(N * K // 64)
+    with pytest.raises(_Launched):
+        ops.nf4_linear(x, packed, s, N, 64, **_adapter(lora_x=torch.ones_like(x)))
+    with pytest.raises(RuntimeError):
+        ops.nf4_linear(x, packed, s, N, 64, **_adapter(lora_x=bad))
