@@ -579,7 +579,7 @@ extern "C" int rq_int8_linear_scratch_size(int x_dtype, int64_t M, int64_t K, in
                     (block_size == 0 ||
                      (block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0));
   const int64_t C = dx ? K : N, R = dx ? N : K;
-  *bytes = fast && !rq::dense_beats_fused(M, C, R, false) ? 0 : int64_t(rq::dense_scratch_bytes(x_dtype, M, C, R, dx ? rank : 0));
+  *bytes = fast && !rq::dense_beats_fused(M, C, R, rq::kFusedInt8) ? 0 : int64_t(rq::dense_scratch_bytes(x_dtype, M, C, R, dx ? rank : 0));
   return RQ_OK;
 }
 

@@ -575,24 +575,52 @@ size_t dense_scratch_bytes(int x_dtype, int64_t M, int64_t C, int64_t R, int64_t
   return plan_dense(x_dtype, M, C, R, rank > 0 ? rank : 0, device_cus()).bytes;
 }
 
-// Estimates in microseconds from measurements on the Llama-3-8B shapes (M = 64
-// .. 2048): the fused GEMM takes 1.15 us per 64-k step of a full wave of
-// 256 x 128 tiles (0.9 us while fewer than half the compute units have one),
-// 6 us per wave of tiles and 12 us for its K splits; decoding takes 0.5 us per million weights and its
-// launches 8 us.  Both sides near the line, fused against dense: q forward M =
-// 2048 93 / 105 us, gate forward M = 512 86 / 111 us and M = 1024 165 / 142 us,
-// q dX M = 1024 90 / 62 us, down dX M = 512 98 / 116 us, M = 1024 183 / 145 us.
-bool dense_beats_fused(int64_t M, int64_t C, int64_t R, bool splits) {
+namespace {
+// Microseconds of a tiled product, fitted to measurements (957 calls: 17 to 4096
+// rows, 1024 to 14336 columns and reduction lengths, both routes timed in turn).
+// A round of tiles costs `round` and, per 64-k step, `alone` while at most half
+// of the compute units have a workgroup, growing to alone + shared when all do;
+// splitting K costs `split`, the call `call`.
+struct ProductCost {
+  double alone, shared, round, split, call;
+};
+constexpr ProductCost kFusedCost[3] = {
+    {0.73, 0.28, 6.6, 7.2, 1.5},  // kFusedNF4
+    {0.92, 0.16, 4.8, 0.0, 5.7},  // kFusedNF4Dx
+    {0.78, 0.26, 6.0, 0.0, 0.9},  // kFusedInt8
+};
+// by tile: 128 x 128, 256 x 256 (the call: its decode launch)
+constexpr ProductCost kDenseCost[2] = {{0.20, 0.23, 5.3, 2.6, 9.0}, {0.84, 0.57, 9.2, 13.6, 9.0}};
+constexpr double kDecodeUs = 0.48e-6;  // a weight's, written and read back
+
+double product_us(const ProductCost& c, int64_t rounds, int64_t tail, int splits, int64_t nk, int cus) {
+  auto step = [&](int64_t busy) { return c.alone + c.shared * std::max(0.0, 2.0 * std::min<int64_t>(busy, cus) / cus - 1.0); };
+  return c.call + double(rounds) * (double(nk) * step(cus) + c.round) +
+         (tail > 0 ? double(ceil_div(nk, splits)) * step(tail * splits) + c.round : 0.0) + (splits > 1 ? c.split : 0.0);
+}
+}  // namespace
+
+// Both sides measured, us, fused against dense: NF4 forward 4096 -> 4096 M = 256
+// 27.6 / 37.3, M = 1536 62.5 / 72.1, M = 3072 120 / 96.4; 14336 -> 4096 M = 256 58.3
+// / 76.9, M = 1024 130 / 139, M = 2048 242 / 213; 4096 -> 14336 M = 640 106 / 111, M =
+// 1024 135 / 120; dX from 4096 to 11008 columns M = 256 71.5 / 56.0; INT8 1024 ->
+// 8192 M = 512 20.2 / 28.1.  The rule sends here three
+// of the 957 calls, and four of 328 further ones of drawn sizes, that are more than
+// 3 % faster fused (8 % at most); the 3 % that it asks for keeps calls that gain
+// nothing from taking scratch memory.
+bool dense_beats_fused(int64_t M, int64_t C, int64_t R, FusedKernel kernel) {
   if (M <= kGemvMaxM) return false;
   const int cus = device_cus();
-  const GemmPlan f = plan_gemm(M, C, R, 0, cus, splits);
+  const GemmPlan f = plan_gemm(M, C, R, 0, cus, kernel == kFusedNF4);
   const int64_t T = int64_t(f.tiles_m) * f.tiles_n;
-  const double nk = double(R) / 64.0, step = T * f.splits >= cus / 2 ? 1.15 : 0.9;
-  const double waves = f.splits > 1 ? double(f.lf * 8 / cus) + 1.0 / f.splits : double(ceil_div(T, cus));
-  const double fused = nk * step * waves + 6.0 * double(ceil_div(T, cus)) + (f.splits > 1 ? 12.0 : 0.0);
+  const int64_t rounds = f.splits > 1 ? f.lf * 8 / cus : T / cus;
+  const double fused = product_us(kFusedCost[kernel], rounds, T - rounds * cus, f.splits, ceil_div(R, 64), cus);
   DensePlan p{};
-  const double dense = pick_tiles(p, RQ_DTYPE_BF16, M, C, int((R + 63) / 64), cus);
-  return dense + 8.0 + 0.5e-6 * double(C) * double(R) < fused;
+  const int64_t nk = ceil_div(R, 64);
+  pick_tiles(p, RQ_DTYPE_BF16, M, C, int(nk), cus);
+  const int64_t D = int64_t(p.tiles_m) * p.tiles_n;
+  const double dense = product_us(kDenseCost[p.halves - 1], D / cus, D % cus, p.splits, nk, cus);
+  return dense + kDecodeUs * double(C) * double(R) < 0.97 * fused;
 }
 
 // fp32 forward against the GEMV kernels over blocks of 16 rows, about 1.2 us per

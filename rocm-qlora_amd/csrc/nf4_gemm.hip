@@ -550,7 +550,7 @@ extern "C" int rq_nf4_linear_dx_scratch_size(int dy_dtype, int64_t M, int64_t N,
   if (M < 0 || N <= 0 || K <= 0 || block_size < 1 || rank < 0 || rank > 256) return RQ_ERR_BAD_SHAPE;
   const bool fast = dy_dtype != RQ_DTYPE_F32 && N % 64 == 0 && K % 64 == 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0 &&
                     K % block_size == 0;
-  *bytes = fast && !rq::dense_beats_fused(M, K, N, false) ? 0
+  *bytes = fast && !rq::dense_beats_fused(M, K, N, rq::kFusedNF4Dx) ? 0
                                                           : int64_t(rq::dense_scratch_bytes(dy_dtype, M, K, N, rank));
   return RQ_OK;
 }

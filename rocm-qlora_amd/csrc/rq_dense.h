@@ -18,9 +18,11 @@ namespace rq {
 // (fp32 activations, operands past 32-bit offsets).
 size_t dense_scratch_bytes(int x_dtype, int64_t M, int64_t C, int64_t R, int64_t rank);
 
-// Whether the dense path is the faster one for a call the fused GEMM takes
-// (splits: that call's GEMM splits K for the last wave's tiles).
-bool dense_beats_fused(int64_t M, int64_t C, int64_t R, bool splits);
+// The GEMM over the stored codes that a call runs on otherwise (the NF4 forward's
+// splits K for its last round of tiles).
+enum FusedKernel { kFusedNF4, kFusedNF4Dx, kFusedInt8 };
+// Whether the dense path is the faster one for a call that kernel takes.
+bool dense_beats_fused(int64_t M, int64_t C, int64_t R, FusedKernel kernel);
 
 // The same for fp32 activations and the row-block GEMV kernels (forward).
 bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R);
