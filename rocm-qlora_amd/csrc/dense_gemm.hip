@@ -623,15 +623,24 @@ bool dense_beats_fused(int64_t M, int64_t C, int64_t R, FusedKernel kernel) {
   return dense + kDecodeUs * double(C) * double(R) < 0.97 * fused;
 }
 
-// fp32 forward against the GEMV kernels over blocks of 16 rows, about 1.2 us per
-// million weights and block (4096 x 4096: 20 us a block with the LoRA operand):
-// decoding takes 1 us per million weights and its launches 10 us.
-bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R) {
+// fp32 forward against the GEMV kernels over blocks of 16 rows.  A block costs 3.9 +
+// 0.0021 K us per round of 16-column tiles (one per compute unit), its LoRA operand
+// 2.6 us plus, per rank, 0.14 us a round and 13 ps per k; the dense side the
+// product's estimate, 0.8 us per million weights decoded, 8 us of launches and for
+// LoRA 7 us + 0.16 us per rank.  Of 240 calls timed on both routes (512 to 14336
+// columns and reduction lengths, 32 to 256 rows, ranks 0, 16, 64) one taken here is
+// slower, by 4 %.  Blocks against dense, us: 4096 -> 4096 M = 64 49 / 64, M = 96 74 /
+// 64, rank 16 M = 64 75 / 74; 1024 -> 1024 rank 16 M = 48 35 / 33, M = 256 186 / 34;
+// 14336 -> 4096 M = 64 149 / 177.
+bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R, int64_t rank) {
   if (M <= kGemvMaxM) return false;
+  const int cus = device_cus();
+  const double rounds = double(ceil_div(ceil_div(C, 16), cus)), K = double(R), r = double(rank);
+  const double block = rounds * (3.9 + 0.0021 * K) + (rank > 0 ? 2.6 + r * (0.14 * rounds + 1.3e-5 * K) : 0.0);
   DensePlan p{};
-  const double mw = 1e-6 * double(C) * double(R);
-  return pick_tiles(p, RQ_DTYPE_F32, M, C, int(ceil_div(R, 32)), device_cus()) + 10.0 + 1.0 * mw <
-         1.2 * mw * double(ceil_div(M, 16));
+  const double dense = pick_tiles(p, RQ_DTYPE_F32, M, C, int(ceil_div(R, 32)), cus) + 8.0 +
+                       0.8e-6 * double(C) * K + (rank > 0 ? 7.0 + 0.16 * r : 0.0);
+  return dense < block * double(ceil_div(M, 16));
 }
 
 bool dense_nf4_linear_ok(const LinearArgs& L) {

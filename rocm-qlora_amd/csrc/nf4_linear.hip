@@ -1652,7 +1652,7 @@ extern "C" int rq_nf4_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int
   const bool f32 = x_dtype == RQ_DTYPE_F32;
   const bool fast = K % 64 == 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0 &&
                     (!f32 || rank <= 64);
-  const bool faster = !fast || (f32 ? dense_beats_f32_blocks(M, N, K)
+  const bool faster = !fast || (f32 ? dense_beats_f32_blocks(M, N, K, rank)
                                  : !skinny_takes(M, N, K, rank) && dense_beats_fused(M, N, K, kFusedNF4));
   *bytes = faster ? int64_t(dense_scratch_bytes(x_dtype, M, N, K, rank)) : 0;
   return RQ_OK;

@@ -25,7 +25,7 @@ enum FusedKernel { kFusedNF4, kFusedNF4Dx, kFusedInt8 };
 bool dense_beats_fused(int64_t M, int64_t C, int64_t R, FusedKernel kernel);
 
 // The same for fp32 activations and the row-block GEMV kernels (forward).
-bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R);
+bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R, int64_t rank);
 
 // Whether the operands' alignment suits the dense path (any, once the
 // reduction is padded; else activation rows of 16-byte chunks).

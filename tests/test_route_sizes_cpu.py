@@ -46,6 +46,17 @@ INT8 = [
     (2048, 3072, 3072, False),   # 48.8 / 61.1
     (256, 4096, 4096, True),     # 56.8 / 38.4
 ]
+# (M, K, N, rank, dense), times row blocks / dense
+FORWARD_F32 = [
+    (64, 4096, 4096, 0, False),    # 49 / 64
+    (96, 4096, 4096, 0, True),     # 74 / 64
+    (48, 14336, 4096, 16, False),  # 137 / 190
+    (64, 14336, 4096, 0, False),   # 149 / 177
+    (128, 14336, 4096, 0, True),   # 298 / 178
+    (64, 4096, 14336, 16, True),   # 241 / 198
+    (128, 1024, 1024, 0, True),    # 51 / 25
+    (256, 512, 512, 64, True),     # 256 / 36
+]
 
 
 @pytest.mark.parametrize("M,K,N,dense", FORWARD)
@@ -62,3 +73,8 @@ def test_nf4_dx_route(M, K, N, dense):
 @pytest.mark.parametrize("M,K,N,dense", INT8)
 def test_int8_forward_route(M, K, N, dense):
     assert (_size("rq_int8_linear_scratch_size", BF16, M, K, N, 64, 0, 0) > 0) == dense
+
+
+@pytest.mark.parametrize("M,K,N,rank,dense", FORWARD_F32)
+def test_nf4_forward_fp32_route(M, K, N, rank, dense):
+    assert (_size("rq_nf4_linear_scratch_size", F32, M, K, N, 64, rank) > 0) == dense
