@@ -184,10 +184,14 @@ int rq_nf4_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
 /* rq_nf4_linear with optional scratch memory (256-byte aligned device memory,
  * contents ignored, free again once the call's kernels are done).  A call
  * given the bytes it needs decodes the weight into it once and multiplies
- * by the dense MFMA GEMM (same operand roundings, another order of fp32 sums);
- * any other call is rq_nf4_linear.  rq_nf4_linear_scratch_size reports those
- * bytes where that is the faster route (many rows, and most calls that
- * otherwise run on the generic kernels), 0 elsewhere. */
+ * by the dense MFMA GEMM -- or, with 17 to 64 rows of 16-bit activations in a
+ * specialized kernel's shape, runs the skinny kernel, whose K splits meet there
+ * (at most 128 MiB; up to 1.5 MiB in the workspace instead) and are counted in
+ * the workspace's synchronization area --
+ * with the same operand roundings and another order of fp32 sums; any other
+ * call is rq_nf4_linear.  rq_nf4_linear_scratch_size reports those bytes where
+ * that is the faster route (also every call that otherwise runs on the generic
+ * kernels), 0 elsewhere. */
 int rq_nf4_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int64_t N, int64_t block_size, int64_t rank,
                                int64_t* bytes);
 int rq_nf4_linear_scratch(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,

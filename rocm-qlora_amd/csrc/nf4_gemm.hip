@@ -300,8 +300,10 @@ static size_t dx_at_bytes(int64_t K, int64_t rank16) { return (size_t(K) * size_
 
 int gemm_workspace(const LinearArgs& L, size_t* bytes) {
   *bytes = plan_gemm(L.M, L.N, L.K, L.rank, device_cus(), true).ws_bytes;
-  if (skinny_takes(L.M, L.N, L.K, L.rank))
-    *bytes = std::max(*bytes, skinny_workspace(L.M, L.N, L.K, L.rank));
+  if (skinny_takes(L.M, L.N, L.K, L.rank)) {
+    const size_t need = skinny_scratch(L.M, L.N, L.K, L.rank);
+    if (need <= kSkinnyHeldBytes) *bytes = std::max(*bytes, need);
+  }
   return RQ_OK;
 }
 
@@ -310,16 +312,20 @@ size_t gemm_min_workspace(const LinearArgs& L) {
 }
 
 int run_nf4_gemm(const LinearArgs& L, void* workspace, size_t ws_bytes, uint32_t* tile_cnt, size_t n_cnt,
-                 hipStream_t stream) {
+                 void* scratch, size_t scratch_bytes, hipStream_t stream) {
   // the activation operands are loaded 16 bytes at a time
   if (!aligned(L.x, 16) || L.ldx % 8 != 0) return RQ_ERR_BAD_ALIGNMENT;
   if (!offsets_fit(L.M, L.ldx, L.N, L.K)) return RQ_ERR_UNSUPPORTED;
-  // few rows: the skinny kernel, given room for its splits
+  // few rows: the skinny kernel, given room for its splits in the scratch memory
+  // or the workspace
   if (skinny_takes(L.M, L.N, L.K, L.rank)) {
-    const size_t need = skinny_workspace(L.M, L.N, L.K, L.rank), counters = skinny_counters(L.M, L.N, L.K);
-    if ((need == 0 || (workspace && ws_bytes >= need && aligned(workspace, 256))) &&
+    const size_t need = skinny_scratch(L.M, L.N, L.K, L.rank), counters = skinny_counters(L.M, L.N, L.K);
+    const bool given = scratch && scratch_bytes >= need && aligned(scratch, 256);
+    void* const room = given ? scratch : workspace;
+    const size_t room_bytes = given ? scratch_bytes : ws_bytes;
+    if ((need == 0 || (room && room_bytes >= need && aligned(room, 256))) &&
         (counters == 0 || (tile_cnt && counters <= n_cnt)) && aligned(L.w_packed, 16))
-      return run_skinny_nf4(L, workspace, ws_bytes, tile_cnt, stream);
+      return run_skinny_nf4(L, room, room_bytes, tile_cnt, stream);
   }
   // K splits need the zeroed tile counts and room for their partial tiles;
   // without them the GEMM runs unsplit

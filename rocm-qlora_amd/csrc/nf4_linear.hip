@@ -1600,19 +1600,23 @@ extern "C" int rq_nf4_linear_workspace_size(int x_dtype, int64_t M, int64_t K, i
     f32_linear_workspace(L, &f);
   } else {
     st = M <= kGemvMaxM ? gemv_workspace(L, &f) : gemm_workspace(L, &f);
-    if (M > kGemvMaxM && f > 0) f += kLinearSyncBytes;
+    // the skinny kernel's splits are counted in the synchronization area
+    const bool counted = M > kGemvMaxM && skinny_takes(M, N, K, rank) && skinny_counters(M, N, K) > 0;
+    if (M > kGemvMaxM && (f > 0 || counted)) f += kLinearSyncBytes;
   }
   *bytes = int64_t(std::max(b, f));
   return st;
 }
 
-// rq_nf4_linear's routes; scratch: optional memory for the decoded weight
+// rq_nf4_linear's routes; scratch: optional memory for the decoded weight, or for
+// the skinny kernel's splits where that kernel takes the call
 static int run_linear(const LinearArgs& L, void* workspace, int64_t workspace_bytes, void* scratch,
                       int64_t scratch_bytes, hipStream_t stream) {
   int st = validate_linear(L);
   if (st != RQ_OK || L.M == 0) return st;
   if (workspace_bytes < 0 || scratch_bytes < 0) return RQ_ERR_BAD_SHAPE;
-  if (scratch && scratch_bytes > 0) {
+  const bool skinny = L.x_dtype != RQ_DTYPE_F32 && linear_fast_ok(L) && skinny_takes(L.M, L.N, L.K, L.rank);
+  if (scratch && scratch_bytes > 0 && !skinny) {
     const size_t need = dense_scratch_bytes(L.x_dtype, L.M, L.N, L.K, L.rank);
     if (need > 0 && size_t(scratch_bytes) >= need && dense_nf4_linear_ok(L))
       return run_dense_nf4_linear(L, scratch, size_t(scratch_bytes), stream);
@@ -1628,7 +1632,7 @@ static int run_linear(const LinearArgs& L, void* workspace, int64_t workspace_by
                       area ? reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kLinearSyncBytes -
                                                          kGemmCountBytes)
                            : nullptr,
-                      kGemmCountBytes / 4, stream);
+                      kGemmCountBytes / 4, scratch, size_t(scratch_bytes), stream);
 }
 
 extern "C" int rq_nf4_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
@@ -1652,8 +1656,12 @@ extern "C" int rq_nf4_linear_scratch_size(int x_dtype, int64_t M, int64_t K, int
   const bool f32 = x_dtype == RQ_DTYPE_F32;
   const bool fast = K % 64 == 0 && block_size >= 64 && (block_size & (block_size - 1)) == 0 && K % block_size == 0 &&
                     (!f32 || rank <= 64);
-  const bool faster = !fast || (f32 ? dense_beats_f32_blocks(M, N, K, rank)
-                                 : !skinny_takes(M, N, K, rank) && dense_beats_fused(M, N, K, kFusedNF4));
+  if (fast && !f32 && skinny_takes(M, N, K, rank)) {
+    const size_t need = skinny_scratch(M, N, K, rank);
+    *bytes = need > kSkinnyHeldBytes ? int64_t(need) : 0;
+    return RQ_OK;
+  }
+  const bool faster = !fast || (f32 ? dense_beats_f32_blocks(M, N, K, rank) : dense_beats_fused(M, N, K, kFusedNF4));
   *bytes = faster ? int64_t(dense_scratch_bytes(x_dtype, M, N, K, rank)) : 0;
   return RQ_OK;
 }

@@ -102,8 +102,9 @@ int f32_linear_workspace(const LinearArgs& L, size_t* bytes);
 int run_nf4_linear_f32(const LinearArgs& L, void* workspace, size_t ws_bytes, hipStream_t stream);
 // tile_cnt: n_cnt zeroed counters the GEMM's K splits use (and leave zero);
 // without them the GEMM runs unsplit.
+// scratch: optional, for the skinny kernel's splits (rq_skinny.h)
 int run_nf4_gemm(const LinearArgs& L, void* workspace, size_t ws_bytes, uint32_t* tile_cnt, size_t n_cnt,
-                 hipStream_t stream);
+                 void* scratch, size_t scratch_bytes, hipStream_t stream);
 
 // Unpacked arguments of rq_nf4_linear_dx (see include/rocm_qlora_amd.h).
 struct DxArgs {

@@ -13,11 +13,16 @@ namespace rq {
 // being those the fused GEMMs take, LoRA rank at most 64).
 bool skinny_takes(int64_t M, int64_t N, int64_t K, int64_t rank);
 
-// Its workspace: the K splits' partial tiles and the LoRA operand's partials.
-size_t skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t rank);
+// Its scratch memory: the K splits' partial tiles and the LoRA operand's partials
+// (contents ignored; 0: none needed).
+// Up to kSkinnyHeldBytes of it are part of the workspace, which callers keep: a
+// call that small is bound by its host time, and memory of its own for each call
+// costs 1.6 of 15 us.  More is asked for per call and given back.
+constexpr size_t kSkinnyHeldBytes = size_t(1536) << 10;
+size_t skinny_scratch(int64_t M, int64_t N, int64_t K, int64_t rank);
 // Tile counters it uses (zero before and after the call; 0: none).
 size_t skinny_counters(int64_t M, int64_t N, int64_t K);
 
-int run_skinny_nf4(const LinearArgs& L, void* workspace, size_t bytes, uint32_t* cnt, hipStream_t stream);
+int run_skinny_nf4(const LinearArgs& L, void* scratch, size_t bytes, uint32_t* cnt, hipStream_t stream);
 
 }  // namespace rq

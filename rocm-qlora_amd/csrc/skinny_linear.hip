@@ -471,12 +471,20 @@ SkArgs sk_args(const SkPlan& p, const void* x, int64_t ldx, const void* w, int64
 
 }  // namespace
 
+// Bounded by the bytes the splits exchange: they are written and read once beside
+// the weight, 0.19 N K of them at up to 48 rows and 0.5 N K at 64 (the packed weight
+// is 0.5 N K).  Against the fused GEMM, us: 4096 -> 128256 48 rows 159 / 268 (100 MB),
+// 64 rows 235 / 267 and with LoRA 281 / 287 (266 MB); 14336 -> 14336 64 rows 95 / 107
+// and 113 / 117 (104 MB); 4096 -> 14336 31 / 41.
+constexpr size_t kSkMaxScratch = size_t(128) << 20;
+
 bool skinny_takes(int64_t M, int64_t N, int64_t K, int64_t rank) {
   // 32-bit offsets into weights and activations are the callers' fast-path checks
-  return M > kGemvMaxM && M <= kSkRows && rank <= 64 && K % 64 == 0 && double(N) * double(K) < 8.58e9;
+  return M > kGemvMaxM && M <= kSkRows && rank <= 64 && K % 64 == 0 && double(N) * double(K) < 8.58e9 &&
+         plan_skinny(M, N, K, rank, device_cus()).bytes <= kSkMaxScratch;
 }
 
-size_t skinny_workspace(int64_t M, int64_t N, int64_t K, int64_t rank) {
+size_t skinny_scratch(int64_t M, int64_t N, int64_t K, int64_t rank) {
   return plan_skinny(M, N, K, rank, device_cus()).bytes;
 }
 
@@ -485,9 +493,9 @@ size_t skinny_counters(int64_t M, int64_t N, int64_t K) {
   return p.splits > 1 ? size_t(p.groups) : 0;
 }
 
-int run_skinny_nf4(const LinearArgs& L, void* workspace, size_t bytes, uint32_t* cnt, hipStream_t stream) {
+int run_skinny_nf4(const LinearArgs& L, void* scratch, size_t bytes, uint32_t* cnt, hipStream_t stream) {
   const SkPlan p = plan_skinny(L.M, L.N, L.K, L.rank, device_cus());
-  if (p.bytes > 0 && (!workspace || bytes < p.bytes || !aligned(workspace, 256))) return RQ_ERR_WORKSPACE;
+  if (p.bytes > 0 && (!scratch || bytes < p.bytes || !aligned(scratch, 256))) return RQ_ERR_WORKSPACE;
   SkEpi e{};
   bool u_in = false;
   e.bias = L.bias;
@@ -495,7 +503,7 @@ int run_skinny_nf4(const LinearArgs& L, void* workspace, size_t bytes, uint32_t*
   e.y = static_cast<uint16_t*>(L.y);
   e.ldy = L.ldy;
   if (L.rank > 0) {
-    float* u = static_cast<float*>(workspace);
+    float* u = static_cast<float*>(scratch);
     // the operand inside the launch when the adapter reads x itself
     u_in = L.lora_x == L.x && L.ld_lora_x == L.ldx && aligned(L.lora_a, 16);
     const int st = u_in ? RQ_OK : run_lora_rows_parts(L.x_dtype, static_cast<const uint16_t*>(L.lora_x), L.ld_lora_x, L.M, L.K,
@@ -510,11 +518,11 @@ int run_skinny_nf4(const LinearArgs& L, void* workspace, size_t bytes, uint32_t*
     e.b_vec = aligned(L.lora_b, 16) && (L.lora_dtype != RQ_DTYPE_F32 || L.ld_lora_b % 4 == 0);
     e.scaling = L.scaling;
   }
-  SkArgs a = sk_args(p, L.x, L.ldx, L.w_packed, L.M, L.N, L.K, L.K / 2, L.block_size, workspace, cnt);
+  SkArgs a = sk_args(p, L.x, L.ldx, L.w_packed, L.M, L.N, L.K, L.K / 2, L.block_size, scratch, cnt);
   if (u_in) {
     a.la = L.lora_a;
     a.la_dt = L.lora_dtype;
-    a.upart = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.u_off);
+    a.upart = reinterpret_cast<float*>(static_cast<char*>(scratch) + p.u_off);
   }
   return L.x_dtype == RQ_DTYPE_BF16
              ? launch_scale<RQ_DTYPE_BF16, UnitNF4>(a, L.absmax, L.absmax_dtype, L.c2, L.c2_format, L.block2, e, p,

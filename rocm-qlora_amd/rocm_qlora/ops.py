@@ -19,6 +19,9 @@ from rocm_qlora._device import on
 # activation rows up to which the NF4 linear runs as a weight-streaming GEMV
 # (kGemvMaxM in csrc/rq_linear.h); above it, the MFMA GEMM
 GEMV_MAX_M = 16
+# rows up to which a 16-bit call may run on the skinny kernel (kSkRows in
+# csrc/skinny_linear.hip)
+SKINNY_MAX_M = 64
 # largest N * (row stride of LoRA B) the decode GEMV addresses (2^29 elements)
 GEMV_MAX_B_ELEMS = 1 << 29
 
@@ -255,8 +258,9 @@ def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optio
         scratch = None
         if (M > GEMV_MAX_M or not fast_shape) and max(ldx, ldxl) * M * x.element_size() < 1 << 32:
             scratch = _spare("rq_nf4_linear_scratch_size", dev, xcode, M, K, N, block_size, rank)
-        # a call with scratch memory needs no workspace of its own
-        ws = _workspace(x.dtype, M, K, N, rank, dev) if scratch is None else None
+        # a dense call needs no workspace beside its scratch memory; the skinny
+        # kernel counts its splits in the workspace's synchronization area
+        ws = _workspace(x.dtype, M, K, N, rank, dev) if scratch is None or (fast_shape and M <= SKINNY_MAX_M) else None
         codes = c2.reshape(-1).view(torch.uint8).contiguous() if dq else None
         nat.call("rq_nf4_linear_scratch",
                  x2.data_ptr(), xcode, M, K, ldx,

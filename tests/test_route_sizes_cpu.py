@@ -78,3 +78,18 @@ def test_int8_forward_route(M, K, N, dense):
 @pytest.mark.parametrize("M,K,N,rank,dense", FORWARD_F32)
 def test_nf4_forward_fp32_route(M, K, N, rank, dense):
     assert (_size("rq_nf4_linear_scratch_size", F32, M, K, N, 64, rank) > 0) == dense
+
+
+@pytest.mark.parametrize("M,K,N,rank", [(17, 4096, 1024, 0), (48, 4096, 14336, 16), (48, 4096, 128256, 16), (64, 4096, 128256, 0),
+                                        (64, 4096, 128256, 64), (64, 16384, 16384, 64), (33, 1024, 512, 0)])
+def test_skinny_memory(M, K, N, rank):
+    """The skinny kernel's splits, past 1.5 MiB, live in scratch memory of at most 128
+    MiB, freed after the call; the workspace, which callers keep, holds what the fused GEMM
+    needs (its K splits' tiles, at most one per compute unit) and the area the
+    splits are counted in."""
+    ws, scratch = _size("rq_nf4_linear_workspace_size", BF16, M, K, N, rank), _size("rq_nf4_linear_scratch_size", BF16, M, K, N, 64, rank)
+    assert (131328 if (M, N) != (64, 128256) else 0) <= ws <= 131328 + 256 * 256 * 128 * 4 + (2 << 20)
+    assert scratch <= 128 << 20
+    # splits x rows x columns of fp32, or none: too much, or little enough for the workspace
+    assert scratch == 0 or scratch >= 4 * M * N
+    assert (scratch == 0) == ((M, K, N) in ((64, 4096, 128256), (64, 16384, 16384), (17, 4096, 1024), (33, 1024, 512)))

@@ -2,7 +2,7 @@
 16, the last segment partly past K, one to many K splits, both segment counts
 per split, partial column groups, LoRA ranks up to 64, against the oracle at the
 tolerance of the other 16-bit linears (rtol = atol = 1e-2); and the same bits
-from three calls, whichever split counts itself last."""
+from three calls, whichever split counts itself last, and from replays of a graph."""
 import pytest
 import torch
 
@@ -46,3 +46,30 @@ def test_skinny_linear(dev, M, K, N, block, rank, dtype, dq):
     err = (outs[0].cpu().float() - ref.float()).abs()
     bad = err > 1e-2 + 1e-2 * ref.float().abs()
     assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside tol; max err {float(err.max()):.4g}"
+
+
+def test_skinny_linear_replayed(dev):
+    """Two captured calls that share the capture's scratch memory and counters,
+    replayed among eager calls on the same operands: the eager bits every time."""
+    g = torch.Generator().manual_seed(4)
+    calls = []
+    for M, K, N in ((40, 4096, 512), (64, 2048, 1088)):
+        packed, s = quantize_int4((torch.randn(N, K, generator=g) * 0.02).to(dev), 64)
+        x = torch.randn(M, K, generator=g).bfloat16().to(dev)
+        a, b = (torch.randn(16, K, generator=g) * 0.02).to(dev), (torch.randn(N, 16, generator=g) * 0.05).to(dev)
+        calls.append(lambda x=x, packed=packed, s=s, N=N, a=a, b=b: ops.nf4_linear(x, packed, s, N, 64, lora_a=a, lora_b=b, scaling=0.5))
+    ref = [c() for c in calls]
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        [c() for c in calls]
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            out = [c() for c in calls]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        [o.fill_(float("nan")) for o in out]
+        graph.replay()
+        eager = [c() for c in calls]
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, r) and torch.equal(e, r) for o, e, r in zip(out, eager, ref))
