@@ -176,13 +176,33 @@ def _scratch(size_fn: str, dev, *args) -> Optional[torch.Tensor]:
     return torch.empty(n, dtype=torch.uint8, device=dev) if n else None
 
 
+# Devices that had no room for a call's scratch memory: the smallest size that
+# failed, the calls to go without it after the last failure, and those left.  A
+# failed allocation makes torch give back its cached blocks to the driver, so on a
+# GPU that stays full the tries are 1, 2, 4 .. _FULL_MOST_CALLS calls apart.
+_FULL: dict = {}
+_FULL_MOST_CALLS = 256
+
+
 def _spare(size_fn: str, dev, *args) -> Optional[torch.Tensor]:
     """_scratch for a call that also runs without it: None on a GPU whose memory
     is too full for the decoded weight."""
-    try:
-        return _scratch(size_fn, dev, *args)
-    except torch.OutOfMemoryError:
+    full = _FULL.get(dev.index)
+    counts = full is not None and _bytes(size_fn, dev.index, *args) >= full[0]
+    if counts and full[2] > 0:
+        _FULL[dev.index] = (full[0], full[1], full[2] - 1)
         return None
+    try:
+        t = _scratch(size_fn, dev, *args)
+    except torch.OutOfMemoryError:
+        n, wait = _bytes(size_fn, dev.index, *args), 1
+        if full is not None:
+            n, wait = min(n, full[0]), min(2 * full[1], _FULL_MOST_CALLS)
+        _FULL[dev.index] = (n, wait, wait)
+        return None
+    if counts:
+        _FULL.pop(dev.index, None)
+    return t
 
 
 def nf4_linear(x: torch.Tensor, weight_quant: torch.Tensor, weight_scales: Optional[torch.Tensor],
