@@ -45,6 +45,15 @@ def _stored_dx(dy: torch.Tensor, qw) -> torch.Tensor:
     return dm.int8_dx(dy, qw)
 
 
+def _is_probability(drop: nn.Module) -> bool:
+    """Whether calling the adapter's dropout module is torch's dropout of its
+    probability and nothing else: no hooks (its own or global ones), no other
+    forward, not in place."""
+    return type(drop) in (nn.Dropout, nn.Identity) and "forward" not in drop.__dict__ and \
+        not (drop._forward_hooks or drop._forward_pre_hooks or drop._backward_hooks or drop._backward_pre_hooks) and \
+        not getattr(drop, "inplace", False) and not nn.modules.module._has_any_global_hook()
+
+
 class _FP8LinearFunc(torch.autograd.Function):
     """FP8 forward, dX = dY . W backward (fp8_linear.py:19-67).  w_q: the
     weight's FP8 codes and scale (or None: w_fp16 is quantized here); qw: the
@@ -102,8 +111,7 @@ class FP8LinearWrapper(nn.Module):
             qw = ql.nf4_weight() if ql.bits == 4 else ql.int8_weight()
             lora = self.base
             drop = lora.lora_dropout
-            if dm.native_adapter(x, lora.lora_A) and type(drop) in (nn.Dropout, nn.Identity) and \
-                    not (drop._forward_hooks or drop._forward_pre_hooks or drop._backward_hooks):
+            if dm.native_adapter(x, lora.lora_A) and _is_probability(drop):
                 p = drop.p if drop.training and isinstance(drop, nn.Dropout) else 0.0
 
                 def base_dx(dy, A, B, s, g, mask, mask_scale):

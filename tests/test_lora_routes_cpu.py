@@ -3,11 +3,15 @@ gradients (torch.autograd.grad(is_grads_batched=True), tensors without storage)
 and forward-mode AD take the torch expressions, on any device; and calls inside
 torch.jit.trace keep their autograd functions, without which the trace would hold
 an output allocation and nothing that fills it."""
+import types
+
 import pytest
 import torch
+import torch.nn as nn
 from torch.autograd import forward_ad
 
-from rocm_qlora import ops
+from rocm_qlora import LoRALinear, QuantLinear, ops
+from rocm_qlora.fp8 import fp8_linear
 from rocm_qlora.kernels import dequant_matmul as dm
 
 
@@ -65,3 +69,53 @@ def test_calls_inside_jit_trace_keep_their_autograd_function():
         f(x)
         torch.jit.trace(f, (x,), check_trace=False)
     assert seen == [(True, True), (False, False)]
+
+
+def _patch_forward(drop):
+    forward = drop.forward
+    drop.forward = lambda x: forward(x)
+
+
+class _MyDropout(nn.Dropout):
+    pass
+
+
+# what makes a call of the adapter's dropout module more than its probability
+DROPOUTS = {
+    "subclass": lambda: _MyDropout(0.1),
+    "in_place": lambda: nn.Dropout(0.1, inplace=True),
+    "forward_hook": lambda: _with(nn.Dropout(0.1), lambda d: d.register_forward_hook(lambda m, i, o: None)),
+    "forward_pre_hook": lambda: _with(nn.Identity(), lambda d: d.register_forward_pre_hook(lambda m, i: None)),
+    "backward_hook": lambda: _with(nn.Dropout(0.1), lambda d: d.register_full_backward_hook(lambda m, i, o: None)),
+    "backward_pre_hook": lambda: _with(nn.Dropout(0.1), lambda d: d.register_full_backward_pre_hook(lambda m, o: None)),
+    "replaced_forward": lambda: _with(nn.Dropout(0.1), _patch_forward),
+    "global_hook": lambda: nn.Dropout(0.1),
+    "plain": lambda: nn.Dropout(0.1),
+    "none": lambda: nn.Identity(),
+}
+
+
+def _with(drop, change):
+    change(drop)
+    return drop
+
+
+@pytest.mark.parametrize("kind", DROPOUTS)
+def test_fp8_layer_calls_a_dropout_module_that_is_more_than_its_probability(monkeypatch, kind):
+    layer = LoRALinear(QuantLinear(64, 32, bits=4, bias=False), r=8, lora_alpha=16)
+    layer.lora_dropout = DROPOUTS[kind]()
+    wrapper = fp8_linear.FP8LinearWrapper(layer)
+    wrapper.backend = "native"
+    wrapper._weight = lambda dtype: None
+    routes = []
+    monkeypatch.setattr(dm, "native_adapter", lambda x, a: True)
+    monkeypatch.setattr(dm, "base_lora_linear", lambda *a: routes.append("kernels"))
+    monkeypatch.setattr(fp8_linear, "_FP8LinearFunc",
+                        types.SimpleNamespace(apply=lambda x, *a: (routes.append("module"), torch.zeros(x.shape[0], 32))[1]))
+    hook = nn.modules.module.register_module_forward_hook(lambda m, i, o: None) if kind == "global_hook" else None
+    try:
+        wrapper(torch.randn(5, 64))
+    finally:
+        if hook is not None:
+            hook.remove()
+    assert routes == (["kernels"] if kind in ("plain", "none") else ["module"])
