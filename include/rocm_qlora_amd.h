@@ -245,6 +245,11 @@ uint32_t rq_set_gemv_wait_us(uint32_t us);
  * tiles. */
 int rq_gemm_tile_config(int32_t* out);
 
+/* Tiles of the dense MFMA GEMM behind the *_scratch entry points, for M rows, C
+ * output columns and a reduction of R: out[0..3] = rows and columns of a tile
+ * (256 or 128), tiles run whole, tiles whose reduction is split, splits. */
+int rq_dense_tile_plan(int x_dtype, int64_t M, int64_t C, int64_t R, int32_t* out);
+
 /* Bytes of device workspace rq_nf4_linear_dx needs (0 when none; dy_dtype
  * fp32, bf16 or fp16). */
 int rq_nf4_linear_dx_workspace_size(int dy_dtype, int64_t M, int64_t N, int64_t K, int64_t rank,

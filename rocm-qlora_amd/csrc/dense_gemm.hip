@@ -704,3 +704,15 @@ int run_dense_int8(const GenericInt8& A, bool dx, void* scratch, size_t bytes, h
 }
 
 }  // namespace rq
+
+extern "C" int rq_dense_tile_plan(int x_dtype, int64_t M, int64_t C, int64_t R, int32_t* out) {
+  if (!out) return RQ_ERR_NULL_POINTER;
+  if (!rq::valid_float_dtype(x_dtype)) return RQ_ERR_BAD_DTYPE;
+  if (M < 1 || C < 1 || R < 1 || rq::dense_scratch_bytes(x_dtype, M, C, R, 0) == 0) return RQ_ERR_BAD_SHAPE;
+  const rq::DensePlan p = rq::plan_dense(x_dtype, M, C, R, 0, rq::device_cus());
+  out[0] = 128 * p.halves;
+  out[1] = p.whole;
+  out[2] = p.tiles_m * p.tiles_n - p.whole;
+  out[3] = p.splits;
+  return RQ_OK;
+}

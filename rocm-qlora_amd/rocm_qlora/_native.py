@@ -58,6 +58,7 @@ SIGNATURES = {
                               _P, _I64, _P],                 # y, ldy, stream
     "rq_set_gemv_wait_us": [ctypes.c_uint32],
     "rq_gemm_tile_config": [_P],
+    "rq_dense_tile_plan": [_I32, _I64, _I64, _I64, _P],      # dtype, M, columns, reduction, out
     "rq_stream_capture_id": [_P, _P],
     "rq_nf4_linear_dx_workspace_size": [_I32, _I64, _I64, _I64, _I64, _P],
     "rq_nf4_linear_dx_scratch_size": [_I32, _I64, _I64, _I64, _I64, _I64, _P],

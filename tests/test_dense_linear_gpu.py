@@ -1,9 +1,10 @@
 """Linears that decode the weight once into scratch memory and multiply by the
-dense MFMA GEMM (csrc/dense_gemm.hip): tile edges of both tile sizes, K
-splits, reduction lengths that are padded, every decode kernel, the LoRA and
-dropout epilogues, against the oracle at the tolerance of the other linears
-(16-bit results: rtol = atol = 1e-2, fp32 1e-3, gradients relative to the
-largest).
+dense MFMA GEMM (csrc/dense_gemm.hip): tile edges, K splits, reduction lengths
+that are padded, every decode kernel, the LoRA and dropout epilogues, against the
+oracle at the tolerance of the other linears (16-bit results: rtol = atol = 1e-2,
+fp32 1e-3, gradients relative to the largest).  FORWARD and the INT8 shapes run on
+128 x 128 tiles; LARGE reaches the 256 x 256 ones, with operands whose sums are
+exact in fp32, so that every bit is compared.
 
 The entry points are called with scratch memory of the size the library
 reports for the dense path, whatever the row count, through the C ABI."""
@@ -35,8 +36,7 @@ def _check(got, ref, relative=False):
     assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside tol; max err {float(err.max()):.4g}"
 
 
-# (M, K, N, block, rank, dtype, storage): rows and columns around the 128- and
-# 256-wide tiles, one to many 64-k steps (prefetches past the end; odd step
+# (M, K, N, block, rank, dtype, storage): rows and columns around multiples of 128, one to many 64-k steps (prefetches past the end; odd step
 # counts), splits (few tiles, long K), lengths padded to 64, blocks of 32 and
 # blocks that straddle rows, ranks of one and two epilogue steps and past 64
 FORWARD = [
@@ -180,3 +180,83 @@ def test_dense_rule_matches_general_path(dev):
             # one bf16 rounding may fall the other way: 2^-8 of the value
             d = (got.float() - ref.float()).abs()
             assert bool((d <= 2.0 ** -7 * ref.float().abs() + 1e-5 * float(ref.abs().max())).all()), f"call {i}"
+
+
+# (M, R, C, rank, dtype, bias) and what the plan makes of them: tile edge, whole
+# tiles, split tiles, splits.  256 x 256 tiles with ragged rows and columns; 11
+# (the fewest the plan gives them) and 12 steps; a padded reduction; one split
+# count each of whole tiles mixed with split ones; split tiles alone, with an odd
+# number of steps a split.  And the 128 x 128 tiles' mix.
+LARGE = [
+    (4000, 700, 4001, 0, "bf16", True, (256, 256, 0, 1)),
+    (3841, 768, 3841, 12, "fp16", True, (256, 256, 0, 1)),
+    (4097, 3100, 4097, 16, "bf16", False, (256, 256, 33, 4)),
+    (5000, 2560, 3600, 64, "bf16", True, (256, 256, 44, 4)),
+    (4097, 4096, 4609, 16, "fp16", False, (256, 256, 67, 2)),
+    (700, 11001, 4000, 8, "bf16", False, (256, 0, 48, 4)),
+    (1290, 4096, 4096, 16, "bf16", True, (128, 256, 96, 2)),
+]
+
+
+def _tile_plan(dtype, M, C, R):
+    out = (ctypes.c_int32 * 4)()
+    nat.call("rq_dense_tile_plan", nat.dtype_code(DTYPES[dtype]), M, C, R, out)
+    return tuple(out)
+
+
+def _ints(g, dev, lo, hi, *shape):
+    return torch.randint(lo, hi + 1, shape, generator=g, device=dev).double()
+
+
+def _whole_weight(g, dev, N, K):
+    """An NF4 weight of the values -2, -1, 0, 1, 2: codes of -1, 0 and 1 and absmax 1
+    or 2."""
+    code = torch.tensor([0, 7, 15], dtype=torch.uint8, device=dev)[torch.randint(0, 3, (N * K + N * K % 2,), generator=g, device=dev)]
+    absmax = torch.randint(1, 3, (-(-N * K // 64),), generator=g, device=dev).float()
+    value = torch.tensor([-1.0, 0.0, 1.0], dtype=torch.float64, device=dev)[(code.long() + 7) // 8]
+    w = (value[:N * K] * absmax.double().repeat_interleave(64)[:N * K]).reshape(N, K)
+    return code[0::2] | (code[1::2] << 4), absmax, w
+
+
+@pytest.mark.parametrize("M,R,C,rank,dtype,bias,plan", LARGE)
+def test_dense_tiles_forward_exact(dev, always_dense, M, R, C, rank, dtype, bias, plan):
+    print(f"dense exact forward {M} {R} {C} {rank} {dtype} {plan}", flush=True)
+    assert _tile_plan(dtype, M, C, R) == plan
+    dt, g = DTYPES[dtype], torch.Generator(device=dev).manual_seed(M + R + C)
+
+    def rnd(t):
+        return t.to(dt).double()
+
+    packed, absmax, w = _whole_weight(g, dev, C, R)
+    x, b = _ints(g, dev, -3, 3, M, R), _ints(g, dev, -500, 500, C)
+    la, lb = _ints(g, dev, -2, 2, rank, R), _ints(g, dev, -1, 1, C, rank)
+    y = ops.nf4_linear(x.to(dt), packed, absmax, C, 64, b.to(dt) if bias else None, lora_a=la.float() if rank else None,
+                       lora_b=lb.float() if rank else None, scaling=0.5)
+    ref = rnd(x @ w.T + (rnd(b) if bias else 0.0))
+    if rank:
+        ref = rnd(ref + rnd(rnd(rnd(x @ la.T) @ lb.T) * 0.5))
+    assert float((x @ w.T).abs().max()) > 256  # past bf16's 8 bits
+    assert torch.equal(y.double(), ref)
+
+
+@pytest.mark.parametrize("M,R,C,rank,dtype,masked,plan", [(*c[:5], m, c[6]) for c in LARGE for m in (False, True) if c[3] or not m])
+def test_dense_tiles_dx_exact(dev, always_dense, M, R, C, rank, dtype, masked, plan):
+    print(f"dense exact dx {M} {R} {C} {rank} {dtype} {masked} {plan}", flush=True)
+    assert _tile_plan(dtype, M, C, R) == plan
+    dt, g = DTYPES[dtype], torch.Generator(device=dev).manual_seed(M + R + C + 1)
+
+    def rnd(t):
+        return t.to(dt).double()
+
+    packed, absmax, w = _whole_weight(g, dev, R, C)  # [N, K] = [R, C]
+    dy = _ints(g, dev, -3, 3, M, R)
+    la, lb = _ints(g, dev, -1, 1, rank, C), _ints(g, dev, -2, 2, R, rank)
+    mask = torch.rand(M, C, generator=g, device=dev) < 0.8
+    dx = ops.nf4_linear_dx(dy.to(dt), packed, absmax, C, 64, lora_a=la.float() if rank else None,
+                           lora_b=lb.float() if rank else None, scaling=0.5, lora_mask=mask if masked else None,
+                           mask_scale=1.25 if masked else 1.0)
+    ref = rnd(dy @ w)
+    if rank:
+        term = rnd(rnd(rnd(dy * 0.5) @ lb) @ la)
+        ref = rnd(ref + (rnd(term * mask * 1.25) if masked else term))
+    assert torch.equal(dx.double(), ref)
