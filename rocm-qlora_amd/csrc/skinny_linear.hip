@@ -76,13 +76,12 @@ struct SkEpi {
   int64_t ldy;
 };
 
-// Weight formats.  A unit is 16 rows x 256 k of a wave; lane (i, q) = (lane %
-// 16, lane / 16) owns row i.  Its steps are MFMAs of 32 k, 8 consecutive k per
+// A unit is 16 rows x 256 k of a wave; lane (i, q) = (lane % 16, lane / 16) owns row
+// i.  Its steps are MFMAs of 32 k, 8 consecutive k per
 // lane; piece(s), chunk(s, q): where step s's k lie in the activations' 64-k
 // pieces of 8 chunks.
 template <int XT, class Scale>
 struct UnitNF4 {
-  static constexpr bool kTable = true;
   static constexpr int kLoads = 2 + 2 * Scale::kLoads;
   u32x4 w[2];                    // k = 32 q + 128 h + [0, 32)
   typename Scale::Raw s[2];
@@ -104,10 +103,10 @@ struct UnitNF4 {
   __device__ static __forceinline__ int chunk(int st, int q) { return 4 * (q & 1) + (st & 3); }
 };
 
-template <int XT, template <int, class> class UnitT, class Scale, int MB, int U>
+template <int XT, class Scale, int MB, int U>
 __global__ __launch_bounds__(kSkThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
-  using Unit = UnitT<XT, Scale>;
+  using Unit = UnitNF4<XT, Scale>;
   constexpr int kXRows = 16 * MB, kPiece = kXRows * 128;
   __shared__ __attribute__((aligned(16))) uint8_t lds[kSkLds];
   u32x2* lut = reinterpret_cast<u32x2*>(lds);
@@ -144,7 +143,7 @@ void skinny_kernel(SkArgs a, Scale scale, SkEpi e) {
 #pragma unroll
   for (int u = 0; u < U; ++u) un[u].load(a, scale, wr, n, q, kbeg + int64_t(u < nu ? u : nu - 1) * kSkSeg);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (Unit::kTable) fill_f32pair_lut<kSkThreads>(lut, tid);
+  fill_f32pair_lut<kSkThreads>(lut, tid);
   // the activation loads are older than the U * kLoads weight loads
   step_barrier<U * Unit::kLoads>();
 
@@ -416,57 +415,37 @@ SkPlan plan_skinny(int64_t M, int64_t N, int64_t K, int64_t rank, int cus) {
   return p;
 }
 
-template <int XT, template <int, class> class UnitT, class Scale>
+template <int XT, class Scale>
 int launch_skinny(const SkArgs& a, Scale scale, const SkEpi& e, const SkPlan& p, hipStream_t stream) {
   const unsigned grid = unsigned(p.groups * p.splits);
-  if (p.mb == 4) skinny_kernel<XT, UnitT, Scale, 4, 2><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
+  if (p.mb == 4) skinny_kernel<XT, Scale, 4, 2><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
   else if (p.mb == 3 && p.units == 4)
-    skinny_kernel<XT, UnitT, Scale, 3, 4><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
-  else if (p.mb == 3) skinny_kernel<XT, UnitT, Scale, 3, 2><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
-  else if (p.units == 4) skinny_kernel<XT, UnitT, Scale, 2, 4><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
-  else skinny_kernel<XT, UnitT, Scale, 2, 2><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
+    skinny_kernel<XT, Scale, 3, 4><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
+  else if (p.mb == 3) skinny_kernel<XT, Scale, 3, 2><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
+  else if (p.units == 4) skinny_kernel<XT, Scale, 2, 4><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
+  else skinny_kernel<XT, Scale, 2, 2><<<grid, kSkThreads, 0, stream>>>(a, scale, e);
   return rq_check_launch();
 }
 
-template <int XT, template <int, class> class UnitT>
+template <int XT>
 int launch_scale(const SkArgs& a, const void* s, int sdt, const uint8_t* c2, int c2_format, int64_t block2,
                  const SkEpi& e, const SkPlan& p, hipStream_t stream) {
   if (c2) {
     const int sh = pow2_shift(block2);
     switch (sdt) {
       case RQ_DTYPE_F32:
-        return launch_skinny<XT, UnitT>(a, ScaleDQ<RQ_DTYPE_F32>{c2, s, c2_format, sh, block2}, e, p, stream);
+        return launch_skinny<XT>(a, ScaleDQ<RQ_DTYPE_F32>{c2, s, c2_format, sh, block2}, e, p, stream);
       case RQ_DTYPE_BF16:
-        return launch_skinny<XT, UnitT>(a, ScaleDQ<RQ_DTYPE_BF16>{c2, s, c2_format, sh, block2}, e, p, stream);
+        return launch_skinny<XT>(a, ScaleDQ<RQ_DTYPE_BF16>{c2, s, c2_format, sh, block2}, e, p, stream);
       default:
-        return launch_skinny<XT, UnitT>(a, ScaleDQ<RQ_DTYPE_F16>{c2, s, c2_format, sh, block2}, e, p, stream);
+        return launch_skinny<XT>(a, ScaleDQ<RQ_DTYPE_F16>{c2, s, c2_format, sh, block2}, e, p, stream);
     }
   }
   switch (sdt) {
-    case RQ_DTYPE_F32: return launch_skinny<XT, UnitT>(a, ScaleAbsmax<RQ_DTYPE_F32>{s}, e, p, stream);
-    case RQ_DTYPE_BF16: return launch_skinny<XT, UnitT>(a, ScaleAbsmax<RQ_DTYPE_BF16>{s}, e, p, stream);
-    default: return launch_skinny<XT, UnitT>(a, ScaleAbsmax<RQ_DTYPE_F16>{s}, e, p, stream);
+    case RQ_DTYPE_F32: return launch_skinny<XT>(a, ScaleAbsmax<RQ_DTYPE_F32>{s}, e, p, stream);
+    case RQ_DTYPE_BF16: return launch_skinny<XT>(a, ScaleAbsmax<RQ_DTYPE_BF16>{s}, e, p, stream);
+    default: return launch_skinny<XT>(a, ScaleAbsmax<RQ_DTYPE_F16>{s}, e, p, stream);
   }
-}
-
-SkArgs sk_args(const SkPlan& p, const void* x, int64_t ldx, const void* w, int64_t M, int64_t N, int64_t K,
-               int64_t row_bytes, int64_t block_size, void* workspace, uint32_t* cnt) {
-  SkArgs a{};
-  a.x = static_cast<const uint16_t*>(x);
-  a.ldx = ldx;
-  a.w = static_cast<const uint8_t*>(w);
-  a.M = M;
-  a.N = N;
-  a.K = K;
-  a.row_bytes = row_bytes;
-  a.blocks_per_row = block_size ? K / block_size : 1;
-  a.bs_log2 = block_size ? pow2_shift(block_size) : 62;  // per row: k >> 62 == 0
-  a.groups = p.groups;
-  a.splits = p.splits;
-  a.nseg = p.nseg;
-  a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.part_off);
-  a.cnt = cnt;
-  return a;
 }
 
 }  // namespace
@@ -506,8 +485,9 @@ int run_skinny_nf4(const LinearArgs& L, void* scratch, size_t bytes, uint32_t* c
     float* u = static_cast<float*>(scratch);
     // the operand inside the launch when the adapter reads x itself
     u_in = L.lora_x == L.x && L.ld_lora_x == L.ldx && aligned(L.lora_a, 16);
-    const int st = u_in ? RQ_OK : run_lora_rows_parts(L.x_dtype, static_cast<const uint16_t*>(L.lora_x), L.ld_lora_x, L.M, L.K,
-                                       L.lora_a, L.lora_dtype, L.K, 1, int(L.rank), false, 1.0f, p.lr, u, stream);
+    const int st = u_in ? RQ_OK
+                        : run_lora_rows_parts(L.x_dtype, static_cast<const uint16_t*>(L.lora_x), L.ld_lora_x, L.M, L.K,
+                                              L.lora_a, L.lora_dtype, L.K, 1, int(L.rank), false, 1.0f, p.lr, u, stream);
     if (st != RQ_OK) return st;
     e.rank = int(L.rank);
     e.u = u;
@@ -518,17 +498,28 @@ int run_skinny_nf4(const LinearArgs& L, void* scratch, size_t bytes, uint32_t* c
     e.b_vec = aligned(L.lora_b, 16) && (L.lora_dtype != RQ_DTYPE_F32 || L.ld_lora_b % 4 == 0);
     e.scaling = L.scaling;
   }
-  SkArgs a = sk_args(p, L.x, L.ldx, L.w_packed, L.M, L.N, L.K, L.K / 2, L.block_size, scratch, cnt);
+  SkArgs a{};
+  a.x = static_cast<const uint16_t*>(L.x);
+  a.ldx = L.ldx;
+  a.w = L.w_packed;
+  a.M = L.M;
+  a.N = L.N;
+  a.K = L.K;
+  a.row_bytes = L.K / 2;
+  a.blocks_per_row = L.K / L.block_size;
+  a.bs_log2 = pow2_shift(L.block_size);
+  a.groups = p.groups;
+  a.splits = p.splits;
+  a.nseg = p.nseg;
+  a.part = reinterpret_cast<float*>(static_cast<char*>(scratch) + p.part_off);
+  a.cnt = cnt;
   if (u_in) {
     a.la = L.lora_a;
     a.la_dt = L.lora_dtype;
     a.upart = reinterpret_cast<float*>(static_cast<char*>(scratch) + p.u_off);
   }
-  return L.x_dtype == RQ_DTYPE_BF16
-             ? launch_scale<RQ_DTYPE_BF16, UnitNF4>(a, L.absmax, L.absmax_dtype, L.c2, L.c2_format, L.block2, e, p,
-                                                    stream)
-             : launch_scale<RQ_DTYPE_F16, UnitNF4>(a, L.absmax, L.absmax_dtype, L.c2, L.c2_format, L.block2, e, p,
-                                                   stream);
+  auto launch = L.x_dtype == RQ_DTYPE_BF16 ? launch_scale<RQ_DTYPE_BF16> : launch_scale<RQ_DTYPE_F16>;
+  return launch(a, L.absmax, L.absmax_dtype, L.c2, L.c2_format, L.block2, e, p, stream);
 }
 
 }  // namespace rq
