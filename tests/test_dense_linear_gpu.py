@@ -260,3 +260,49 @@ def test_dense_tiles_dx_exact(dev, always_dense, M, R, C, rank, dtype, masked, p
         term = rnd(rnd(rnd(dy * 0.5) @ lb) @ la)
         ref = rnd(ref + (rnd(term * mask * 1.25) if masked else term))
     assert torch.equal(dx.double(), ref)
+
+
+def test_replayed_training_operands(dev):
+    """One graph with the calls of training steps (dense products with and without
+    split tiles, the adapters' gradients, INT8 dX with the adapter's term, the
+    adapter added in place), replayed among eager calls and changed inputs: the
+    eager bits each time."""
+    g = torch.Generator(device=dev).manual_seed(8)
+
+    def randn(*shape, scale=1.0):
+        return torch.randn(*shape, generator=g, device=dev) * scale
+
+    M, K, N, r = 1290, 4096, 4096, 16
+    packed, s = quantize_int4(randn(N, K, scale=0.02), 64)
+    q, qs = quantize_int8(randn(N, K, scale=0.02), 64)
+    x, dy = randn(M, K).bfloat16(), randn(M, N, scale=0.05).bfloat16()
+    a, b = randn(r, K, scale=0.02), randn(N, r, scale=0.05)
+
+    def calls():
+        da, db, gg = ops.lora_grads(x, dy, a, b, 2.0, True, True, True)
+        y8 = ops.lora_add_(ops.int8_linear(x, q, qs, N, 64), x, a, b, 2.0)
+        xf = x[:48].float()
+        return (ops.nf4_linear(x[:300], packed, s, N, 64, lora_a=a, lora_b=b, scaling=2.0),
+                ops.nf4_linear_dx(dy, packed, s, K, 64, lora_a=a, lora_b=b, scaling=2.0, lora_g=gg),
+                ops.int8_linear_dx(dy, q, qs, K, 64, lora_a=a, lora_g=gg), da, db, y8,
+                ops.nf4_linear(xf.repeat(4, 1), packed, s, N, 64, lora_a=a, lora_b=b, scaling=2.0),
+                ops.nf4_linear(x, packed, s, N, 64, lora_a=a, lora_b=b, scaling=2.0))
+
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        calls()
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            out = calls()
+    torch.cuda.synchronize()
+    for _ in range(4):
+        x.copy_(randn(M, K))
+        dy.copy_(randn(M, N, scale=0.05))
+        eager = calls()
+        [o.fill_(float("nan")) for o in out]
+        graph.replay()
+        again = calls()
+        torch.cuda.synchronize()
+        for i, (o, e, f) in enumerate(zip(out, eager, again)):
+            assert torch.equal(o, e) and torch.equal(e, f), i
