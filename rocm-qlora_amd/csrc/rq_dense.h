@@ -15,7 +15,7 @@ namespace rq {
 
 // Scratch bytes of a product of M activation rows with C output columns over
 // a reduction of R, LoRA rank included; 0 when the product never runs here
-// (fp32 activations, operands past 32-bit offsets).
+// (operands past 32-bit offsets, more than 256 ranks).
 size_t dense_scratch_bytes(int x_dtype, int64_t M, int64_t C, int64_t R, int64_t rank);
 
 // The GEMM over the stored codes that a call runs on otherwise (the NF4 forward's

@@ -4,10 +4,12 @@
 y = base(x) + ((drop(x) @ A^T) @ B^T * s).to(base dtype), s = alpha / r,
 A [r, in] Kaiming-uniform(a=sqrt 5), B [out, r] zeros.  With an NF4 base on
 the GPU, the adapter term runs inside the quantized linear's kernel sequence
-(the LoRA epilogue of the GEMV / GEMM) -- with active dropout, on drop(x),
-whose mask the dX kernel applies in the backward pass -- and the backward
-pass runs the fused NF4 dX kernel plus two small library GEMMs for dA and
-dB.  Otherwise the base layer and the adapter are composed as in the
+(the LoRA epilogue of the GEMV / GEMM); with an INT8 base and 16-bit
+activations it is added in place by the LoRA kernels.  Active dropout: on
+drop(x), whose mask the dX kernels apply in the backward pass.  The backward
+pass runs the adapters' gradient kernels (16-bit activations, rank <= 64; torch
+products otherwise) and the dX kernel, which takes the adapter's input gradient
+from them.  Otherwise the base layer and the adapter are composed as in the
 reference.
 """
 from __future__ import annotations
