@@ -627,12 +627,12 @@ bool dense_beats_fused(int64_t M, int64_t C, int64_t R, FusedKernel kernel) {
 // fp32 forward against the GEMV kernels over blocks of 16 rows.  A block costs 3.9 +
 // 0.0021 K us per round of 16-column tiles (one per compute unit), its LoRA operand
 // 2.6 us plus, per rank, 0.14 us a round and 13 ps per k; the dense side the
-// product's estimate, 0.8 us per million weights decoded, 8 us of launches and for
+// product's estimate, 0.9 us per million weights decoded, 8 us of launches and for
 // LoRA 7 us + 0.16 us per rank.  Of 240 calls timed on both routes (512 to 14336
-// columns and reduction lengths, 32 to 256 rows, ranks 0, 16, 64) one taken here is
-// slower, by 4 %.  Blocks against dense, us: 4096 -> 4096 M = 64 49 / 64, M = 96 74 /
-// 64, rank 16 M = 64 75 / 74; 1024 -> 1024 rank 16 M = 48 35 / 33, M = 256 186 / 34;
-// 14336 -> 4096 M = 64 149 / 177.
+// columns and reduction lengths, 32 to 256 rows, ranks 0, 16, 64) two taken here are
+// slower, by 4 %.  Blocks against dense, us: 4096 -> 4096 M = 64 49 / 65, M = 96 74 /
+// 65, rank 16 M = 64 75 / 75; 1024 -> 1024 rank 16 M = 48 35 / 33, M = 256 186 / 34;
+// 14336 -> 4096 M = 64 149 / 181.
 bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R, int64_t rank) {
   if (M <= kGemvMaxM) return false;
   const int cus = device_cus();
@@ -640,7 +640,7 @@ bool dense_beats_f32_blocks(int64_t M, int64_t C, int64_t R, int64_t rank) {
   const double block = rounds * (3.9 + 0.0021 * K) + (rank > 0 ? 2.6 + r * (0.14 * rounds + 1.3e-5 * K) : 0.0);
   DensePlan p{};
   const double dense = pick_tiles(p, RQ_DTYPE_F32, M, C, int(ceil_div(R, 32)), cus) + 8.0 +
-                       0.8e-6 * double(C) * K + (rank > 0 ? 7.0 + 0.16 * r : 0.0);
+                       0.9e-6 * double(C) * K + (rank > 0 ? 7.0 + 0.16 * r : 0.0);
   return dense < block * double(ceil_div(M, 16));
 }
 
