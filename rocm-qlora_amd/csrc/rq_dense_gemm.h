@@ -18,10 +18,10 @@
 // soon as every wave has read it, 1.5 to 2 steps ahead of its next use, and
 // the waits leave the younger half tiles in flight (vmcnt 12 of 16).
 //
-// What bounds it: power.  With zero operands (no toggling) the loop runs at
-// 2.05 PFLOP/s (4096 x 4096 x 14336: 235 us, 0.82 of the dense peak), with
-// N(0, 1) operands at 1.25-1.43 PFLOP/s on the boxes measured (340-384 us) as
-// the clock drops.  The fused eight-wave kernel it replaces for many rows
+// What bounds it: power first, then the loop.  4096 x 4096 x 14336, launches in a
+// row: with N(0, 1) operands 367 to 517 us as the clock drops (1.31 to 0.93
+// PFLOP/s), with zero operands (no toggling) 283 to 308 us throughout (1.70 to 1.56,
+// two thirds of the dense peak).  The fused eight-wave kernel it replaces for many rows
 // (nf4_gemm8_kernel), which dequantizes each weight tile again for every 256
 // activation rows, reached 0.89 PFLOP/s.
 #pragma once
