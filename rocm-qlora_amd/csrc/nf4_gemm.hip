@@ -425,10 +425,12 @@ int dx_workspace(const DxArgs& D, size_t* bytes) {
   // the larger of the MFMA kernel's and the generic kernels' (the operands'
   // alignment and the block size, unknown here, decide which runs)
   const size_t g = generic_lora_bytes(D.dy_dtype, D.M, D.rank);
-  const bool fast = D.dy_dtype != RQ_DTYPE_F32 && D.N % 64 == 0 && D.K % 64 == 0;
+  *bytes = g;
+  if (D.dy_dtype == RQ_DTYPE_F32 || D.N % 64 != 0 || D.K % 64 != 0) return RQ_OK;
+  // plans only reductions of whole 64-k steps
   const size_t core = (plan_gemm(D.M, D.K, D.N, D.rank > 0 ? D.rank : 0, device_cus()).ws_bytes + 255) & ~size_t(255);
   const int64_t r16 = D.rank > 0 ? (D.rank + 15) & ~int64_t(15) : 0;
-  *bytes = std::max(g, fast ? core + dx_scale_t_bytes(D.N, D.K, 64) + (r16 ? dx_at_bytes(D.K, r16) : 0) : size_t(0));
+  *bytes = std::max(g, core + dx_scale_t_bytes(D.N, D.K, 64) + (r16 ? dx_at_bytes(D.K, r16) : 0));
   return RQ_OK;
 }
 

@@ -83,3 +83,12 @@ def test_cpu_tensor_without_gpu_raises():
         pytest.skip("GPU present")
     with pytest.raises(RuntimeError, match="GPU"):
         quantize_int4(torch.randn(128))
+
+
+def test_dx_workspace_of_short_reductions():
+    """Fewer than 64 columns of dY with an adapter: the generic kernels' LoRA
+    operand (the GEMM's plan divides by the reduction's 64-k steps, none here)."""
+    nb = ctypes.c_int64(0)
+    for dtype, M, N, K, rank in ((nat.DTYPE_F32, 574, 3, 256, 16), (nat.DTYPE_BF16, 5, 63, 64, 8), (nat.DTYPE_F16, 1, 1, 1, 1)):
+        nat.call("rq_nf4_linear_dx_workspace_size", dtype, M, N, K, rank, ctypes.byref(nb))
+        assert nb.value >= M * rank * (4 if dtype == nat.DTYPE_F32 else 2)
